@@ -193,6 +193,14 @@ struct gr_ctx {
     std::vector<int> z_batch_off;
     std::vector<long long> z_rec_off;
     int *z_net_ids = nullptr, *z_records = nullptr, *z_raw_cap = nullptr, *z_raw = nullptr;
+    // per batch its nets with the DP in LDS, then the others: descriptors,
+    // subnets and records of the former, batch positions of the latter
+    int4* z_desc = nullptr;
+    int *z_fast_ids = nullptr, *z_recs = nullptr, *z_list = nullptr;
+    struct ZBatch {
+        int fast_off, fast, fast_nmax, slow_off, slow;
+    };
+    std::vector<ZBatch> z_split;
     // FLT stage: phase-two route words, resident DAG records, batch tables
     int route2_per_pin = 100;
     int* pin_off2 = nullptr;
@@ -966,6 +974,97 @@ void require_stage(gr_ctx* c, int begin, int count) {
     if (!c->net_ids) throw GrError(GR_E_STATE, "no L-shape stage topology uploaded");
     if (!c->routes) throw GrError(GR_E_STATE, "no route storage");
     if (begin < 0 || count < 0 || begin + count > c->stage_count) throw GrError(GR_E_ARG, "slot range outside the stage");
+}
+
+// The Z-shape nets of a plan that zshape_net_kernel can route, in its record
+// layout (ZnetArgs), and the batch positions of the others (a tree too large
+// for LDS, two nodes at one place, a node without exactly one parent, a gap
+// in the child slots: the shared map of the general kernels gives those
+// cases their meaning).  n: side of the map the records' positions index.
+struct ZnetPlan {
+    std::vector<int4> desc;
+    std::vector<int> ids, recs, list;
+    std::vector<gr_ctx::ZBatch> split;
+};
+
+ZnetPlan plan_znets(const DeviceGrid& g, int n, int nbatch, const int* batch_off, const int* net_ids,
+                    const long long* rec_off, const int* records, const int* raw_cap) {
+    ZnetPlan zp;
+    zp.split.resize(nbatch);
+    std::vector<int> parent, height, at, level, pos, order;
+    for (int b = 0; b < nbatch; ++b) {
+        gr_ctx::ZBatch& zb = zp.split[b];
+        zb = {int(zp.desc.size()), 0, 1, int(zp.list.size()), 0};
+        const int begin = batch_off[b], count = batch_off[b + 1] - begin;
+        for (int k = 0; k < count; ++k) {
+            const int* rec = records + rec_off[b] + records[rec_off[b] + k];
+            const int m = rec[1];
+            rec += 2;
+            bool fast = m <= kZnetMaxNodes && znet_lds_bytes(g.L, m) <= kZnetLds && zp.recs.size() < size_t(INT32_MAX / 2);
+            int H = 0;
+            if (fast) {
+                parent.assign(m, -1);
+                height.assign(m, 0);
+                pos.resize(m);
+                for (int i = 0; i < m; ++i) pos[i] = rec[6 * i];
+                std::sort(pos.begin(), pos.end());
+                fast = std::adjacent_find(pos.begin(), pos.end()) == pos.end();
+                for (int i = m - 1; i >= 0 && fast; --i)
+                    for (int j = 0; j < 3; ++j) {
+                        const int ch = rec[6 * i + 3 + j];
+                        if (ch == -1) continue;
+                        if ((j && rec[6 * i + 2 + j] == -1) || parent[ch / 6] >= 0) fast = false;
+                        parent[ch / 6] = i | j << 16;
+                        height[i] = std::max(height[i], height[ch / 6] + 1);
+                    }
+                for (int i = 1; i < m && fast; ++i) fast = parent[i] >= 0;
+            }
+            if (!fast) {
+                zp.list.push_back(k);
+                ++zb.slow;
+                continue;
+            }
+            H = height[0];
+            level.assign(H + 2, 0);
+            for (int i = 0; i < m; ++i) ++level[height[i] + 1];
+            for (int h = 0; h <= H; ++h) level[h + 1] += level[h];
+            at.resize(m);
+            order.resize(m);
+            {
+                std::vector<int>& next = pos;  // level starts, consumed
+                next.assign(level.begin(), level.end());
+                for (int i = 0; i < m; ++i) at[i] = next[height[i]]++, order[at[i]] = i;
+            }
+            const size_t base = zp.recs.size();
+            zp.recs.resize(base + 4 * size_t(m) + (m + 1) + (H + 2) + m);
+            int* out = zp.recs.data() + base;
+            int items = 0;
+            for (int q = 0; q < m; ++q) {
+                const int i = order[q];
+                const int* r = rec + 6 * i;
+                const int x = r[0] / n, y = r[0] % n;
+                int nchild = 0, children = 0;
+                for (int j = 0; j < 3 && r[3 + j] != -1; ++j, ++nchild) children |= (at[r[3 + j] / 6] + 1) << (10 * j);
+                out[4 * q] = x | y << 16;
+                out[4 * q + 1] = (r[1] + 1) | (r[2] + 1) << 8 | nchild << 16;
+                out[4 * q + 2] = i ? at[parent[i] & 0xFFFF] | (parent[i] >> 16) << 16 : 0;
+                out[4 * q + 3] = children;
+                out[4 * m + q] = items;
+                if (i) {
+                    const int pp = rec[6 * (parent[i] & 0xFFFF)], px = pp / n, py = pp % n;
+                    items += px == x || py == y ? 1 : std::abs(px - x) + std::abs(py - y);
+                }
+            }
+            out[5 * m] = items;
+            std::copy(level.begin(), level.end(), out + 5 * m + 1);
+            for (int i = 0; i < m; ++i) out[5 * m + 1 + H + 2 + i] = at[i];
+            zp.desc.push_back(make_int4(int(base), m, H, raw_cap[begin + k]));
+            zp.ids.push_back(net_ids[begin + k]);
+            ++zb.fast;
+            zb.fast_nmax = std::max(zb.fast_nmax, m);
+        }
+    }
+    return zp;
 }
 
 // Soft DP forward over slots [begin, begin + count): the smooth cost model
@@ -1847,12 +1946,24 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
                 }
             }
         }
+        ZnetPlan zp = plan_znets(g, n, nbatch, batch_off, net_ids, rec_off, records, raw_cap);
         c->z_ws.carve([&](auto& cv) {
             c->z_net_ids = cv.template take<int>(nets);
             c->z_records = cv.template take<int>(words);
             c->z_raw_cap = cv.template take<int>(nets);
             c->z_raw = cv.template take<int>(max_raw);
+            c->z_desc = cv.template take<int4>(zp.desc.size());
+            c->z_fast_ids = cv.template take<int>(zp.ids.size());
+            c->z_recs = cv.template take<int>(zp.recs.size());
+            c->z_list = cv.template take<int>(zp.list.size());
         });
+        if (!zp.desc.empty()) {
+            upload(c->z_desc, zp.desc.data(), sizeof(int4) * zp.desc.size(), c->stream);
+            upload(c->z_fast_ids, zp.ids.data(), sizeof(int) * zp.ids.size(), c->stream);
+            upload(c->z_recs, zp.recs.data(), sizeof(int) * zp.recs.size(), c->stream);
+        }
+        if (!zp.list.empty()) upload(c->z_list, zp.list.data(), sizeof(int) * zp.list.size(), c->stream);
+        c->z_split = std::move(zp.split);
         if (nets) {
             upload(c->z_net_ids, net_ids, sizeof(int) * nets, c->stream);
             upload(c->z_raw_cap, raw_cap, sizeof(int) * nets, c->stream);
@@ -1898,13 +2009,21 @@ int gr_zshape_run(gr_ctx* c, int first_stamp, double* elapsed_ms) {
             const int begin = c->z_batch_off[b], count = c->z_batch_off[b + 1] - begin;
             launch_refresh(c, 0);
             if (!count) continue;
+            const gr_ctx::ZBatch& zb = c->z_split[b];
             a.points = c->z_records + c->z_rec_off[b];
-            a.count = count;
+            a.list = c->z_list + zb.slow_off;
+            a.count = zb.slow;
             a.raw_cap = c->z_raw_cap + begin;
             timed(c, GR_K_ZSHAPE, 0.0, [&] {
-                hipLaunchKernelGGL(zshape_reset_kernel, dim3(count), dim3(256), 0, c->stream, a);
-                hipLaunchKernelGGL(zshape_solve_kernel, dim3(count), dim3(kWave), 0, c->stream, a);
-                hipLaunchKernelGGL(zshape_convert_kernel, dim3((count + 255) / 256), dim3(256), 0, c->stream, a,
+                if (zb.fast) {
+                    const ZnetArgs f{g, c->presum, c->vcost, c->z_desc + zb.fast_off, c->z_fast_ids + zb.fast_off,
+                                     c->z_recs, rs, c->error};
+                    launch_zshape_nets(f, zb.fast, zb.fast_nmax, c->stream);
+                }
+                if (!zb.slow) return;
+                hipLaunchKernelGGL(zshape_reset_kernel, dim3(zb.slow), dim3(256), 0, c->stream, a);
+                hipLaunchKernelGGL(zshape_solve_kernel, dim3(zb.slow), dim3(kWave), 0, c->stream, a);
+                hipLaunchKernelGGL(zshape_convert_kernel, dim3((zb.slow + 255) / 256), dim3(256), 0, c->stream, a,
                                    (const int*)(c->z_net_ids + begin), rs);
             });
             launch_commit(c, begin, count, first_stamp + b, 1, c->z_net_ids);

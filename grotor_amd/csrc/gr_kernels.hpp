@@ -171,7 +171,8 @@ struct ZshapeArgs {
     int* map;    // 6 planes of layers * n * n
     int* prev;   // 16 planes
     const int* points;   // batch records: per-net record offsets, then records
-    int count;
+    const int* list;     // positions in the batch of the nets to route
+    int count;           // entries of the list
     int* raw;            // raw route words of the batch
     const int* raw_cap;  // raw words per net
     int n, layers, dirv;
@@ -180,6 +181,30 @@ struct ZshapeArgs {
 __global__ void zshape_reset_kernel(ZshapeArgs a);
 __global__ void zshape_solve_kernel(ZshapeArgs a);
 __global__ void zshape_convert_kernel(ZshapeArgs a, const int* net_ids, RouteStore rs);
+
+// Nets routed with their DP in LDS (zshape_net_kernel): trees of at most
+// kZnetMaxNodes nodes whose tables take at most kZnetLds bytes, every node at
+// a place of its own, child slots filled from the first.
+constexpr int kZnetThreads = 256;
+constexpr int kZnetMaxNodes = 512;
+constexpr size_t kZnetLds = 48 * 1024;
+struct ZnetArgs {
+    DeviceGrid g;
+    const double* presum;
+    const float* vcost;
+    const int4* desc;    // per net: record's first word, nodes, root height, raw words
+    const int* net_ids;  // per net: its subnet
+    // per record, nodes by (height, preorder), n of them, H the root's height:
+    // 4 words per node (x | y << 16, min layer + 1 | max layer + 1 << 8 |
+    // children << 16, parent | slot << 16, children + 1 in 10 bits each), n + 1
+    // prefix sums of the edges' bends, H + 2 level starts, the nodes in preorder
+    const int* recs;
+    RouteStore rs;
+    int* error;
+};
+size_t znet_lds_bytes(int L, int n);
+// nmax: the most nodes of a net in the list
+void launch_zshape_nets(const ZnetArgs& a, int count, int nmax, hipStream_t stream);
 
 // FLT routing DAGs
 constexpr int kFltStride = 10;  // layer index 1..L of the FLT tables (L <= 9), 0 unused
