@@ -176,7 +176,11 @@ struct gr_ctx {
     long long geom_points = 0, geom_hsegs = 0, geom_vsegs = 0;
     std::vector<int> geom_pt_off;  // host copy of the point offsets
     // soft DP: cost arrays, per-cell gradients, checkpointed tables
-    Workspace soft_ws, soft_tables;
+    Workspace soft_ws, soft_tables, soft_level_ws;
+    // the nodes of the last call's slot range by height, kept while the range
+    // and the uploaded stage stay the same
+    SoftLevels soft_levels;
+    std::vector<int> soft_levels_key;  // stage generation, begin, count
     SoftCostArgs soft_cost{};
     SoftArgs soft{};
     int soft_precision = 0;
@@ -1067,6 +1071,27 @@ ZnetPlan plan_znets(const DeviceGrid& g, int n, int nbatch, const int* batch_off
     return zp;
 }
 
+// The level order of slots [begin, begin + count) for the soft passes.
+void ensure_soft_levels(gr_ctx* c, int begin, int count, int nodes) {
+    const std::vector<int> key{c->stage_gen, begin, count};
+    if (key == c->soft_levels_key) return;
+    c->soft_levels_key.clear();
+    int levels = 1;
+    for (int s = begin; s < begin + count; ++s) levels = std::max(levels, c->height_h[s] + 1);
+    SoftLevelArgs a{c->node_off, c->parents, c->lvl, begin, count, levels, nullptr, nullptr, nullptr};
+    c->soft_level_ws.carve([&](auto& cv) {
+        a.cursor = cv.template take<int>(levels);
+        a.start = cv.template take<int>(levels + 1);
+        a.order = cv.template take<int4>(nodes);
+    });
+    launch_soft_levels(a, nodes, c->cus, c->stream);
+    hip_check(hipGetLastError(), "soft level kernels");
+    c->soft_levels.start.resize(levels + 1);
+    c->soft_levels.order = a.order;
+    download(c->soft_levels.start.data(), a.start, sizeof(int) * (levels + 1), c->stream);
+    c->soft_levels_key = key;
+}
+
 // Soft DP forward over slots [begin, begin + count): the smooth cost model
 // at (slope, zero_slope, via_weight), or, with wcost and vcost (IDX order,
 // host), those costs.
@@ -1121,17 +1146,21 @@ void soft_forward(gr_ctx* c, int begin, int count, double slope, double zero_slo
     a.node_off = c->node_off;
     a.nodes = c->nodes;
     a.parents = c->parents;
+    a.link = c->link;
     a.begin = begin;
     a.count = count;
+    a.node0 = c->node_off_h[begin];
+    a.table_nodes = int(nodes);
     a.tau = tau;
     a.scratch = tables;
+    if (count) ensure_soft_levels(c, begin, count, int(nodes));
     hipEvent_t e0 = take_event(c), e1 = take_event(c);
     hip_check(hipEventRecord(e0, c->stream), "hipEventRecord");
     if (given)
         hipLaunchKernelGGL(soft_prefix_kernel, dim3(c->tracks), dim3(256), 0, c->stream, c->g, sc.wcost, sc.presum);
     else
         hipLaunchKernelGGL(soft_costs_kernel, dim3(c->tracks), dim3(256), 0, c->stream, sc);
-    if (count) launch_soft_forward(a, precision, c->soft_kind, c->cus, c->stream);
+    if (count) launch_soft_forward(a, c->soft_levels, precision, c->soft_kind, c->cus, c->stream);
     hip_check(hipEventRecord(e1, c->stream), "hipEventRecord");
     hip_check(hipGetLastError(), "soft forward kernels");
     std::vector<double> v(std::max(count, 1));

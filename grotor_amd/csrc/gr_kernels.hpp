@@ -1,6 +1,8 @@
 // Kernel declarations and launch-argument structures of the gfx950 hot path.
 #pragma once
 
+#include <vector>
+
 #include "gr_device.hpp"
 
 namespace grotor {
@@ -287,9 +289,11 @@ struct SoftArgs {
     const int* node_off;  // stage topology (uploaded slots)
     const int* nodes;
     const int* parents;
+    const int* link;      // per node: (first child + 1) | (next smaller sibling + 1) << 16
     int begin, count;
+    int node0, table_nodes;  // first stage node of the nets [begin, begin + count), and how many
     double tau;
-    void* scratch;   // checkpointed tables of the nets [begin, begin + count)
+    void* scratch;   // checkpointed tables of those nodes
     double* value;   // soft value per net
     double* gw;      // dF/dwcost per cell
     double* gv;      // dF/dvcost per cell
@@ -299,8 +303,24 @@ __global__ void soft_params_kernel(SoftCostArgs c, const double* gw, const doubl
 __global__ void soft_prefix_kernel(DeviceGrid g, const double* wcost, double* presum);
 constexpr int kSoftLayers = 10;  // routing layers the soft DP supports
 size_t soft_scratch_bytes(int L, long long nodes, int precision);
+// The nodes of the slots [begin, begin + count) by height: `levels` heights,
+// order[start[h] .. start[h + 1]) the nodes of height h.
+struct SoftLevelArgs {
+    const int* node_off;
+    const int* parents;
+    const int* lvl;  // per net position: node | height << 16
+    int begin, count, levels;
+    int* cursor;  // [levels]
+    int* start;   // [levels + 1]
+    int4* order;  // {node, first node of its net, slot - begin, parent (-1: root)}
+};
+void launch_soft_levels(const SoftLevelArgs& a, int nodes, int cus, hipStream_t stream);
+struct SoftLevels {
+    std::vector<int> start;  // host copy
+    const int4* order = nullptr;
+};
 // kind 0: L-shape edges, 1: the Z-shape route family
-void launch_soft_forward(const SoftArgs& a, int precision, int kind, int cus, hipStream_t stream);
+void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, int cus, hipStream_t stream);
 void launch_soft_backward(const SoftArgs& a, int precision, int kind, int cus, hipStream_t stream);
 
 // Evaluator-equivalent score (resources/evaluator.cpp:458-675)

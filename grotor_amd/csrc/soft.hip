@@ -32,10 +32,10 @@
 // scatters dF/dwcost (expected wire edge use) and dF/dvcost (expected via
 // landings) into FP64 accumulators.
 //
-// One wavefront per net: lanes over a node's intervals and layers, and for
-// kind 1 over an edge's bend positions (64 at a time), whose per-lane soft
-// minima (running minimum and scaled sum) merge across the wave.  R, the
-// type of the tables and of exp / log, is float or double; costs and
+// The forward pass runs level by level over the nodes of all nets (see "level
+// order" below), L lanes per node, and for kind 1 over the edges of a level,
+// 16 lanes each, lane = bend position; the adjoint one wavefront per net.  R,
+// the type of the tables and of exp / log, is float or double; costs and
 // gradients stay FP64.
 #include "gr_kernels.hpp"
 
@@ -175,24 +175,34 @@ __device__ __forceinline__ void stack_grad(const SoftArgs& a, int x, int y, int 
     for (int k = min(l0, l1); k < max(l0, l1); ++k) atomicAdd(a.gv + cell_of(a.g, k, x, y), gr);
 }
 
+// Checkpointed tables of the nodes [node0, node0 + table_nodes) of the call,
+// node by node.
 template <class R>
-struct NetTables {
-    R *D, *best, *diag, *W1, *W2, *gD;
+struct SoftTables {
+    R *D, *gD, *best, *diag;
 };
 
 template <class R>
-__device__ __forceinline__ NetTables<R> net_tables(const SoftArgs& a, int slot) {
+__device__ __forceinline__ SoftTables<R> soft_tables(const SoftArgs& a) {
     const int L = a.g.L, T = L * (L + 1) / 2;
-    const size_t stride = size_t(2 * T + 4 * L);
-    R* base = reinterpret_cast<R*>(a.scratch) + size_t(a.node_off[slot] - a.node_off[a.begin]) * stride;
-    const int n = a.node_off[slot + 1] - a.node_off[slot];
-    NetTables<R> t;
-    t.D = base;
-    t.gD = t.D + size_t(n) * T;
-    t.best = t.gD + size_t(n) * T;
-    t.diag = t.best + size_t(n) * L;
-    t.W1 = t.diag + size_t(n) * L;
-    t.W2 = t.W1 + size_t(n) * L;
+    const size_t N = size_t(a.table_nodes);
+    SoftTables<R> t;
+    t.D = reinterpret_cast<R*>(a.scratch);
+    t.gD = t.D + N * T;
+    t.best = t.gD + N * T;
+    t.diag = t.best + N * L;
+    return t;
+}
+
+template <class R>
+__device__ __forceinline__ SoftTables<R> net_tables(const SoftArgs& a, int slot) {
+    const int L = a.g.L, T = L * (L + 1) / 2;
+    const size_t n0 = size_t(a.node_off[slot] - a.node0);
+    SoftTables<R> t = soft_tables<R>(a);
+    t.D += n0 * T;
+    t.gD += n0 * T;
+    t.best += n0 * L;
+    t.diag += n0 * L;
     return t;
 }
 
@@ -221,85 +231,6 @@ struct Edge {
 // the route's weight and then scatter(w) adds w to the route's cells.  The
 // Z-shapes are visited through their nested soft minima: per bend, F1 over
 // the leaving layer, M over the middle layer, then the arriving layer.
-
-// Forward: per-lane soft minima per arriving layer, then merged over the wave.
-template <class R>
-__device__ __forceinline__ void zedge_forward(const SoftArgs& a, const Edge& E, const R* best, R tau, R* out) {
-    const DeviceGrid& g = a.g;
-    const int L = g.L, lane = threadIdx.x;
-    const int x = E.x, y = E.y, px = E.px, py = E.py;
-    Lse<R> st[kSoftLayers];
-#pragma unroll
-    for (int e = 0; e < kSoftLayers; ++e) st[e] = lse_empty<R>();
-    if (x == px || y == py) {
-        const int e = lane;
-        const int dv = x == px;  // a column (also when both coordinates agree)
-        if (e < L && layer_dir(g, e) == dv) {
-            const double c = dv ? leg(a, e, 1, x, y, py) : leg(a, e, 0, y, x, px);
-            if (best[e] < R(kSoftBig)) lse_add(st[e], best[e] + R(c), tau);
-        }
-    } else {
-        // L-shapes, lane e = arriving layer
-        const int e = lane;
-        if (e < L) {
-            if (layer_dir(g, e) == 0) {  // vertical, corner (x, py), horizontal on e
-                const double last = leg(a, e, 0, py, x, px);
-                for (int s = 0; s < L; ++s)
-                    if (layer_dir(g, s) == 1 && best[s] < R(kSoftBig))
-                        lse_add(st[e], best[s] + R(leg(a, s, 1, x, y, py) + stack(a, x, py, s, e) + last), tau);
-            } else {  // horizontal, corner (px, y), vertical on e
-                const double last = leg(a, e, 1, px, y, py);
-                for (int s = 0; s < L; ++s)
-                    if (layer_dir(g, s) == 0 && best[s] < R(kSoftBig))
-                        lse_add(st[e], best[s] + R(leg(a, s, 0, y, x, px) + stack(a, px, y, s, e) + last), tau);
-            }
-        }
-        // Z-shapes: rows strictly between y and py (vertical, horizontal, vertical),
-        // then columns strictly between x and px (horizontal, vertical, horizontal)
-        for (int pass = 0; pass < 2; ++pass) {
-            const int lo = pass == 0 ? min(y, py) : min(x, px), hi = pass == 0 ? max(y, py) : max(x, px);
-            const int d1 = pass == 0 ? 1 : 0;  // direction of the first and last legs
-            for (int b0 = lo + 1; b0 < hi; b0 += kWave) {
-                const int b = b0 + lane;
-                if (b >= hi) continue;
-                // bend cells: (x, b) and (px, b) for rows, (b, y) and (b, py) for columns
-                const int ax = pass == 0 ? x : b, ay = pass == 0 ? b : y;
-                const int bx = pass == 0 ? px : b, by = pass == 0 ? b : py;
-                R f1[kSoftLayers];
-                for (int m = 0; m < L; ++m) {
-                    Lse<R> s1 = lse_empty<R>();
-                    if (layer_dir(g, m) != d1)
-                        for (int s = 0; s < L; ++s)
-                            if (layer_dir(g, s) == d1 && best[s] < R(kSoftBig)) {
-                                const double c = (pass == 0 ? leg(a, s, 1, x, y, b) : leg(a, s, 0, y, x, b)) +
-                                                 stack(a, ax, ay, s, m);
-                                lse_add(s1, best[s] + R(c), tau);
-                            }
-                    f1[m] = lse_value(s1, tau);
-                }
-                for (int e = 0; e < L; ++e) {
-                    if (layer_dir(g, e) != d1) continue;
-                    Lse<R> s2 = lse_empty<R>();
-                    for (int m = 0; m < L; ++m)
-                        if (layer_dir(g, m) != d1 && f1[m] < R(kSoftBig)) {
-                            const double c = (pass == 0 ? leg(a, m, 0, b, x, px) : leg(a, m, 1, b, y, py)) +
-                                             stack(a, bx, by, m, e);
-                            lse_add(s2, f1[m] + R(c), tau);
-                        }
-                    const R mv = lse_value(s2, tau);
-                    if (mv < R(kSoftBig)) {
-                        const double c = pass == 0 ? leg(a, e, 1, px, b, py) : leg(a, e, 0, py, b, px);
-                        lse_add(st[e], mv + R(c), tau);
-                    }
-                }
-            }
-        }
-    }
-    for (int e = 0; e < L; ++e) {
-        const Lse<R> m = lse_wave(st[e], tau);
-        if (lane == e) out[e] = lse_value(m, tau);
-    }
-}
 
 // Adjoint of zedge_forward: gdiag[e] = dF/d diag[e]; adds each route's
 // weight to gb[s] (this lane's share of dF/d best[s]) and its cells.
@@ -486,104 +417,443 @@ __global__ __launch_bounds__(256) void soft_costs_kernel(SoftCostArgs a) {
 }
 
 
-// One wavefront per net (grid-stride over the slots [begin, begin + count)).
-template <class R, int K>
-__global__ __launch_bounds__(kWave) void soft_forward_kernel(SoftArgs a) {
-    __shared__ unsigned char s_lo[kSoftMaxT], s_hi[kSoftMaxT];
-    __shared__ R s_best[kSoftLayers], s_diag[kSoftLayers];
-    __shared__ double s_w1[kSoftLayers], s_w2[kSoftLayers];
-    const int lane = threadIdx.x;
-    const DeviceGrid& g = a.g;
-    const int L = g.L, X = g.X, Y = g.Y, XY = g.XY, T = L * (L + 1) / 2;
-    const R tau = R(a.tau);
-    interval_table(L, s_lo, s_hi);
+// ---- level order ----
+//
+// Both passes run over the nodes of all nets of the call level by level: a
+// node's level is its height in its tree, so a level's nodes depend on lower
+// levels only (forward) or on higher ones only (adjoint), and every launch
+// has the whole batch's nodes of a level to fill the chip with.  One
+// wavefront per net, its nodes one after another, kept 8 of 64 lanes busy and
+// every table a dependent round trip away.
+//
+// The order is three small kernels per (stage, slot range): count the nodes
+// per height, scan, place.  Blocks gather their counts in LDS (heights below
+// kLevelBins), one atomic per block and height.
+constexpr int kLevelBins = 256;
+constexpr int kLevelThreads = 256;
+
+__global__ __launch_bounds__(kLevelThreads) void soft_level_count_kernel(SoftLevelArgs a) {
+    __shared__ int s_bin[kLevelBins];
+    for (int h = threadIdx.x; h < kLevelBins; h += kLevelThreads) s_bin[h] = 0;
     __syncthreads();
-    for (int slot = a.begin + blockIdx.x; slot < a.begin + a.count; slot += gridDim.x) {
-        const int n0 = a.node_off[slot], n = a.node_off[slot + 1] - n0;
-        const int* nodes = a.nodes + n0;
-        const int* parents = a.parents + n0;
-        const NetTables<R> t = net_tables<R>(a, slot);
-        for (int q = lane; q < n * T; q += kWave) {
-            const int i = q / T, e = q % T;
-            const int v = nodes[i], fixed = v / XY, x = v / Y % X, y = v % Y;
-            const int lo = s_lo[e], hi = s_hi[e];
-            R val = R(kSoftInf);
-            if (!(fixed < L && (lo > fixed || hi < fixed))) {
-                R s = 0;
-                for (int l = lo; l < hi; ++l) s += R(a.vcost[cell_of(g, l, x, y)]);
-                val = s;
-            }
-            t.D[size_t(i) * T + e] = val;
+    const int q0 = a.node_off[a.begin], q1 = a.node_off[a.begin + a.count];
+    for (int q = q0 + blockIdx.x * kLevelThreads + threadIdx.x; q < q1; q += gridDim.x * kLevelThreads) {
+        const int h = a.lvl[q] >> 16;
+        atomicAdd(h < kLevelBins ? s_bin + h : a.cursor + h, 1);
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < min(kLevelBins, a.levels); h += kLevelThreads)
+        if (s_bin[h]) atomicAdd(a.cursor + h, s_bin[h]);
+}
+
+// cursor[h]: counts in, exclusive prefix out; start[0 .. levels] the same
+// with the total at the end.  One workgroup.
+__global__ __launch_bounds__(kLevelThreads) void soft_level_scan_kernel(SoftLevelArgs a) {
+    __shared__ int s_part[kLevelThreads];
+    const int k = (a.levels + kLevelThreads - 1) / kLevelThreads;
+    const int p0 = min(a.levels, int(threadIdx.x) * k), p1 = min(a.levels, p0 + k);
+    int sum = 0;
+    for (int p = p0; p < p1; ++p) sum += a.cursor[p];
+    s_part[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int run = 0;
+        for (int t = 0; t < kLevelThreads; ++t) {
+            const int v = s_part[t];
+            s_part[t] = run;
+            run += v;
         }
-        __syncthreads();
-        for (int i = n - 1; i >= 1; --i) {
-            const int p = parents[i];
-            const Edge E{nodes[i] / Y % X, nodes[i] % Y, nodes[p] / Y % X, nodes[p] % Y};
-            const R* Di = t.D + size_t(i) * T;
-            if (lane < L) {
-                Lse<R> st = lse_empty<R>();
-                for (int lo = 0; lo <= lane; ++lo)
-                    for (int hi = lane; hi < L; ++hi) lse_add(st, Di[tri_index(L, lo, hi)], tau);
-                const R b = lse_value(st, tau);
-                s_best[lane] = b;
-                t.best[size_t(i) * L + lane] = b;
-            }
-            __syncthreads();
-            if (K == 0) {
-                const int x = E.x, y = E.y, px = E.px, py = E.py;
-                const bool straight = x == px || y == py;
-                if (lane < L) {
-                    const int c = lane, d = layer_dir(g, c);
-                    double w1 = 0.0, w2 = 0.0;
-                    if (!straight || (d ? x == px : y == py)) w1 = d ? leg(a, c, 1, x, y, py) : leg(a, c, 0, y, x, px);
-                    if (!straight) w2 = d ? leg(a, c, 1, px, y, py) : leg(a, c, 0, py, x, px);
-                    s_w1[c] = w1;
-                    s_w2[c] = w2;
-                    t.W1[size_t(i) * L + c] = R(w1);
-                    t.W2[size_t(i) * L + c] = R(w2);
-                }
-                __syncthreads();
-                if (lane < L) {
-                    const int pl = lane, d = layer_dir(g, pl);
-                    Lse<R> st = lse_empty<R>();
-                    if (straight) {
-                        if ((d ? x == px : y == py) && s_best[pl] < R(kSoftBig))
-                            lse_add(st, s_best[pl] + R(s_w1[pl]), tau);
-                    } else {
-                        for (int cl = (pl & 1) ^ 1; cl < L; cl += 2) {
-                            if (!(s_best[cl] < R(kSoftBig))) continue;
-                            const int lo = min(cl, pl), hi = max(cl, pl);
-                            double f = 0.0;
-                            for (int l = lo + 1; l < hi; ++l)
-                                f += layer_dir(g, cl) ? a.vcost[cell_of(g, l, x, py)] : a.vcost[cell_of(g, l, px, y)];
-                            lse_add(st, s_best[cl] + R(s_w1[cl] + f + s_w2[pl]), tau);
-                        }
-                    }
-                    s_diag[pl] = lse_value(st, tau);
-                }
-            } else {
-                zedge_forward<R>(a, E, s_best, tau, s_diag);
-            }
-            __syncthreads();
-            if (lane < L) t.diag[size_t(i) * L + lane] = s_diag[lane];
-            R* Dp = t.D + size_t(p) * T;
-            for (int e = lane; e < T; e += kWave) {
-                Lse<R> st = lse_empty<R>();
-                for (int h = s_lo[e]; h <= s_hi[e]; ++h) lse_add(st, s_diag[h], tau);
-                const R cval = lse_value(st, tau);
-                const R d = Dp[e];
-                Dp[e] = (!(d < R(kSoftBig)) || !(cval < R(kSoftBig))) ? R(kSoftInf) : d + cval;
-            }
-            __syncthreads();
-        }
-        Lse<R> st = lse_empty<R>();
-        for (int e = lane; e < T; e += kWave) lse_add(st, t.D[e], tau);
-        st = lse_wave(st, tau);
-        if (lane == 0) a.value[slot - a.begin] = double(lse_value(st, tau));
-        __syncthreads();
+        a.start[a.levels] = run;
+    }
+    __syncthreads();
+    int run = s_part[threadIdx.x];
+    for (int p = p0; p < p1; ++p) {
+        const int v = a.cursor[p];
+        a.cursor[p] = a.start[p] = run;
+        run += v;
     }
 }
 
+// order[...] = {node, first node of its net, slot - begin, parent (-1: root)};
+// one thread per slot
+__global__ __launch_bounds__(kLevelThreads) void soft_level_place_kernel(SoftLevelArgs a) {
+    __shared__ int s_bin[kLevelBins];
+    const int k = blockIdx.x * kLevelThreads + threadIdx.x;
+    const int n0 = k < a.count ? a.node_off[a.begin + k] : 0;
+    const int n = k < a.count ? a.node_off[a.begin + k + 1] - n0 : 0;
+    for (int h = threadIdx.x; h < kLevelBins; h += kLevelThreads) s_bin[h] = 0;
+    __syncthreads();
+    for (int i = 0; i < n; ++i) {
+        const int h = a.lvl[n0 + i] >> 16;
+        if (h < kLevelBins) atomicAdd(s_bin + h, 1);
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < min(kLevelBins, a.levels); h += kLevelThreads)
+        if (s_bin[h]) s_bin[h] = atomicAdd(a.cursor + h, s_bin[h]);
+    __syncthreads();
+    for (int i = 0; i < n; ++i) {
+        const int q = a.lvl[n0 + i], h = q >> 16, v = q & 0xFFFF;
+        const int at = atomicAdd(h < kLevelBins ? s_bin + h : a.cursor + h, 1);
+        a.order[at] = make_int4(n0 + v, n0, k, a.parents[n0 + v]);
+    }
+}
+
+namespace {
+
+// ---- a node on a group of L lanes ----
+//
+// Lane lo of a group holds row lo of an interval table in registers, entry m
+// = interval [lo, lo + m]; entries past the last layer are absent.  What a
+// layer needs of the rows that contain it comes by shuffles at distance m,
+// so no table goes through LDS.
+template <int L>
+constexpr int kNodesPerWave = kWave / L;
+
+template <class T>
+__device__ __forceinline__ T from_lane(T v, int lane) {
+    return __shfl(v, lane, kWave);
+}
+
+// an added entry, without a branch: one exponential
+template <class R>
+__device__ __forceinline__ void lse_push(Lse<R>& a, R x, R tau) {
+    const R e = r_exp<R>(-(x < a.mn ? a.mn - x : x - a.mn) / tau);
+    const bool fin = x < R(kSoftBig), less = x < a.mn;
+    a.s = fin ? (less ? (a.mn < R(kSoftBig) ? a.s * e : R(0)) + R(1) : a.s + e) : a.s;
+    a.mn = fin && less ? x : a.mn;
+}
+
+// C[lo][lo + m] = smin of diag[lo .. lo + m] for every m of the lane's row,
+// handed to f(m, value) in ascending m; dl: the lane's own diag.
+template <int L, class R, class F>
+__device__ __forceinline__ void closure_row(R dl, int lane, int wl, R tau, F&& f) {
+    Lse<R> st = lse_empty<R>();
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+        const R x = from_lane(dl, lane + m < L ? wl + m : wl);
+        if (lane + m < L) {
+            lse_push(st, x, tau);
+            f(m, lse_value(st, tau));
+        }
+    }
+}
+
+struct SoftNode {
+    int x, y, fixed;
+};
+__device__ __forceinline__ SoftNode soft_node(const DeviceGrid& g, int v) { return SoftNode{v / g.Y % g.X, v % g.Y, v / g.XY}; }
+
+// Kind 0 costs of the edge from (x, y) to (px, py) on lane l: the first leg
+// (the whole of a straight edge) and the second leg of layer l, and the via
+// costs of layer l at the corners (x, py) and (px, y).
+struct EdgeCosts {
+    double w1, w2, va, vb;
+    bool straight, along;
+};
+__device__ __forceinline__ EdgeCosts edge_costs(const SoftArgs& a, int l, int x, int y, int px, int py) {
+    const int d = layer_dir(a.g, l);
+    EdgeCosts c{0.0, 0.0, 0.0, 0.0, x == px || y == py, false};
+    c.along = d ? x == px : y == py;
+    if (!c.straight || c.along) c.w1 = d ? leg(a, l, 1, x, y, py) : leg(a, l, 0, y, x, px);
+    if (!c.straight) {
+        c.w2 = d ? leg(a, l, 1, px, y, py) : leg(a, l, 0, py, x, px);
+        c.va = a.vcost[cell_of(a.g, l, x, py)];
+        c.vb = a.vcost[cell_of(a.g, l, px, y)];
+    }
+    return c;
+}
+
+// Visits the candidates of a bent kind 0 edge on lane pl (arriving layer):
+// f(d, down, valid, cl, sum) for the leaving layers cl = pl - d (down) and pl
+// + d, odd d, with sum = first leg + corner vias strictly between + second
+// leg.  The corner column is (x, py) under a vertical first leg, else (px,
+// y); its sums run upwards from the lower of the two layers.
+template <int L, class F>
+__device__ __forceinline__ void bent_candidates(const DeviceGrid& g, const EdgeCosts& c, int pl, int wl, F&& f) {
+    const bool v = layer_dir(g, pl) != 0;
+    const double own = v ? c.va : c.vb, other = v ? c.vb : c.va;  // columns of a first leg on pl, on pl +- 1
+    double ua = 0.0, ub = 0.0;  // sums over the own / other column of layers pl + 1 .. pl + d - 1
+#pragma unroll
+    for (int d = 1; d < L; ++d) {
+        const bool lo = pl >= d, hi = pl + d < L;
+        const int below = lo ? wl - d : wl, above = hi ? wl + d : wl;
+        if (d % 2) {
+            // lane pl - d's own column is the one of its first leg
+            const double fd = from_lane(ua, below), wd = from_lane(c.w1, below), wu = from_lane(c.w1, above);
+            f(d, true, lo, pl - d, wd + fd + c.w2);
+            f(d, false, hi, pl + d, wu + ub + c.w2);
+        }
+        // layer pl + d has pl's direction for even d: its own / other columns swap with the parity
+        const double ad = from_lane(d % 2 ? other : own, above), bd = from_lane(d % 2 ? own : other, above);
+        ua += hi ? ad : 0.0;
+        ub += hi ? bd : 0.0;
+    }
+}
+
+}  // namespace
+
+// One level of the forward pass: per node its intervals (via stack plus the
+// closures of its children), the soft minima per layer, and for kind 0 the
+// edge to its parent; a root's value.  L lanes per node.  Bound by the
+// instruction issue of the exponentials and logarithms (about 4 L per lane)
+// and, on the upper levels, by the launch itself.  Against one wavefront per
+// net, forward over 465k nodes of 8 layers in binary32: 1.61 -> 0.33 ms.
+template <class R, int L, int K>
+__global__ __launch_bounds__(256) void soft_forward_level_kernel(SoftArgs a, const int4* order, int count) {
+    constexpr int T = L * (L + 1) / 2, G = kNodesPerWave<L>;
+    const DeviceGrid& g = a.g;
+    const R tau = R(a.tau);
+    const int wl = threadIdx.x & (kWave - 1), grp = wl / L, lane = wl % L;
+    const SoftTables<R> t = soft_tables<R>(a);
+    const int waves = gridDim.x * (256 / kWave);
+    for (int w = blockIdx.x * (256 / kWave) + threadIdx.x / kWave; w * G < count; w += waves) {
+        const int k = w * G + grp;
+        if (grp >= G || k >= count) continue;  // whole groups: no shuffle crosses a group
+        const int4 it = order[k];
+        const int node = it.x, n0 = it.y;
+        const SoftNode nd = soft_node(g, a.nodes[node]);
+        const R via = R(a.vcost[cell_of(g, lane, nd.x, nd.y)]);
+        R D[L];
+        {
+            R s = R(0);
+#pragma unroll
+            for (int m = 0; m < L; ++m) {
+                if (m) s += from_lane(via, lane + m <= L ? wl + m - 1 : wl);
+                const bool out = nd.fixed < L && (lane > nd.fixed || lane + m < nd.fixed);
+                D[m] = out ? R(kSoftInf) : s;
+            }
+        }
+        for (int c = (a.link[node] & 0xFFFF) - 1; c >= 0; c = (a.link[n0 + c] >> 16) - 1) {
+            const R dl = t.diag[size_t(n0 + c - a.node0) * L + lane];
+            closure_row<L>(dl, lane, wl, tau, [&](int m, R cv) {
+                D[m] = (!(D[m] < R(kSoftBig)) || !(cv < R(kSoftBig))) ? R(kSoftInf) : D[m] + cv;
+            });
+        }
+        R* Dn = t.D + size_t(node - a.node0) * T + (lane * (2 * L - lane + 1)) / 2;
+#pragma unroll
+        for (int m = 0; m < L; ++m)
+            if (lane + m < L) Dn[m] = D[m];
+        // S[m] = soft minimum over the row's intervals [lo, hi >= lo + m]
+        Lse<R> S[L];
+        {
+            Lse<R> st = lse_empty<R>();
+#pragma unroll
+            for (int m = L - 1; m >= 0; --m) {
+                if (lane + m < L) lse_push(st, D[m], tau);
+                S[m] = st;
+            }
+        }
+        if (it.w < 0) {  // root: over every interval
+            Lse<R> st = S[0];
+            for (int j = 1; j < L; ++j) {
+                const int src = lane == 0 ? wl + j : wl;
+                const Lse<R> o{from_lane(S[0].mn, src), from_lane(S[0].s, src)};
+                if (lane == 0) st = lse_merge(st, o, tau);
+            }
+            if (lane == 0) a.value[it.z] = double(lse_value(st, tau));
+            continue;
+        }
+        // layer k: rows k - m, intervals reaching at least k
+        Lse<R> bs = S[0];
+#pragma unroll
+        for (int m = 1; m < L; ++m) {
+            const int src = lane >= m ? wl - m : wl;
+            const Lse<R> o{from_lane(S[m].mn, src), from_lane(S[m].s, src)};
+            if (lane >= m) bs = lse_merge(bs, o, tau);
+        }
+        const R best = lse_value(bs, tau);
+        const size_t row = size_t(node - a.node0) * L + lane;
+        t.best[row] = best;
+        if (K == 0) {
+            const SoftNode pn = soft_node(g, a.nodes[n0 + it.w]);
+            const EdgeCosts ec = edge_costs(a, lane, nd.x, nd.y, pn.x, pn.y);
+            Lse<R> st = lse_empty<R>();
+            if (ec.straight) {
+                if (ec.along && best < R(kSoftBig)) lse_push(st, best + R(ec.w1), tau);
+            } else {
+                bent_candidates<L>(g, ec, lane, wl, [&](int d, bool down, bool valid, int, double sum) {
+                    const R b = from_lane(best, valid ? (down ? wl - d : wl + d) : wl);
+                    if (valid && b < R(kSoftBig)) lse_push(st, b + R(sum), tau);
+                });
+            }
+            t.diag[row] = lse_value(st, tau);
+        }
+    }
+}
+
+namespace {
+
+// ---- kind 1 edges on 16 lanes ----
+constexpr int kZGroup = 16;
+
+// Minimum / sum over a row of 16 lanes, the same in each of them.
+template <class R, class Op>
+__device__ __forceinline__ R row_reduce(R v, Op&& op) {
+#pragma unroll
+    for (int o = 1; o < kZGroup; o <<= 1) v = op(v, __shfl_xor(v, o, kWave));
+    return v;
+}
+
+// sum[s][m] of the via stacks between every pair of layers of opposite
+// direction at one place: f(lower, upper, sum), sums running upwards from
+// the lower layer.
+template <int L, class F>
+__device__ __forceinline__ void stack_pairs(const double* v, F&& f) {
+#pragma unroll
+    for (int lo = 0; lo < L; ++lo) {
+        double s = 0.0;
+#pragma unroll
+        for (int hi = lo + 1; hi < L; ++hi) {
+            s += v[hi - 1];
+            if ((hi - lo) & 1) f(lo, hi, s);
+        }
+    }
+}
+
+// One bend of an edge: the layers' legs and the two stacks' via costs.  P:
+// parity of the layers of the first and last legs.  The corner bend (bend ==
+// the child's own row or column) has no first leg and no first stack: the
+// middle leg starts at the child.
+template <int V>
+struct ZParity {
+    static constexpr int value = V;
+};
+template <int L>
+struct ZBend {
+    double legs[L];  // first leg on layers of parity P, middle leg on the others
+    double last[L];  // last leg (parity P)
+    double va[L], vb[L];
+    bool corner;
+};
+template <int L, int P>
+__device__ __forceinline__ void load_bend(const SoftArgs& a, const Edge& E, int d1, int b, ZBend<L>& z) {
+    const int ax = d1 ? E.x : b, ay = d1 ? b : E.y, bx = d1 ? E.px : b, by = d1 ? b : E.py;
+    const bool along = d1 ? E.py > E.y : E.px > E.x, across = d1 ? E.px > E.x : E.py > E.y;
+    z.corner = b == (d1 ? E.y : E.x);
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+        const int ca = cell_of(a.g, l, ax, ay), cb = cell_of(a.g, l, bx, by);
+        const double pa = a.presum[ca], pb = a.presum[cb];
+        if ((l & 1) == P) {
+            const double pc = a.presum[cell_of(a.g, l, E.x, E.y)], pp = a.presum[cell_of(a.g, l, E.px, E.py)];
+            z.legs[l] = along ? pa - pc : pc - pa;
+            z.last[l] = along ? pp - pb : pb - pp;
+        } else {
+            z.legs[l] = across ? pb - pa : pa - pb;
+            z.last[l] = 0.0;
+        }
+        z.va[l] = a.vcost[ca];
+        z.vb[l] = a.vcost[cb];
+    }
+}
+
+// Soft minima of a bend's routes from the leaving layers: f1[m] per middle
+// layer (before the middle leg), mv[e] per arriving layer (before the last
+// leg).
+template <class R, int L, int P>
+__device__ __forceinline__ void bend_minima(const ZBend<L>& z, const R* best, R tau, R* f1, R* mv) {
+    Lse<R> s1[L], s2[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) s1[l] = s2[l] = lse_empty<R>();
+    stack_pairs<L>(z.va, [&](int lo, int hi, double s) {
+        const int from = (lo & 1) == P ? lo : hi, to = (lo & 1) == P ? hi : lo;
+        if (best[from] < R(kSoftBig)) lse_push(s1[to], best[from] + R(z.legs[from] + s), tau);
+    });
+#pragma unroll
+    for (int m = 0; m < L; ++m)
+        if ((m & 1) != P) f1[m] = z.corner ? best[m] : lse_value(s1[m], tau);
+    stack_pairs<L>(z.vb, [&](int lo, int hi, double s) {
+        const int e = (lo & 1) == P ? lo : hi, m = (lo & 1) == P ? hi : lo;
+        if (f1[m] < R(kSoftBig)) lse_push(s2[e], f1[m] + R(z.legs[m] + s), tau);
+    });
+#pragma unroll
+    for (int e = 0; e < L; ++e)
+        if ((e & 1) == P) mv[e] = lse_value(s2[e], tau);
+}
+
+// The bends of one orientation (d1 = direction of the first leg) of an edge,
+// kZGroup at a time: the child's own row (column) and those strictly between.
+template <int L, int P, class F>
+__device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, int d1, int lane, F&& f) {
+    const int from = d1 ? E.y : E.x, to = d1 ? E.py : E.px, n = abs(to - from);
+    for (int b0 = 0; b0 < n; b0 += kZGroup) {
+        const int k = b0 + lane;
+        const bool live = k < n;
+        ZBend<L> z;
+        const int b = to > from ? from + (live ? k : 0) : from - (live ? k : 0);
+        load_bend<L, P>(a, E, d1, b, z);
+        f(z, b, live, b0);
+    }
+}
+
+}  // namespace
+
+// Kind 1: one level's edges, 16 lanes each: lane = bend, the lanes' soft
+// minima per arriving layer merged over the row (the minimum first, then one
+// exponential per lane and layer).  Every via cost and prefix sum of a bend is
+// loaded once into registers, where the one-wavefront-per-net form read each
+// stack's costs again for every pair of layers.  Bound by the exponentials
+// (about L^2 / 2 per bend) at three wavefronts per SIMD.  16 lanes an edge:
+// 8 and 4 lanes leave fewer idle on the usual box of 5 x 5 cells but make the
+// long edges the tail (forward over 188k nodes, 8 layers, binary32, tau =
+// 0.1: 0.66 ms at 16, 0.80 at 8, 0.97 at 4; before, 1.33).
+template <class R, int L>
+__global__ __launch_bounds__(256) void soft_zedge_level_kernel(SoftArgs a, const int4* order, int count) {
+    const DeviceGrid& g = a.g;
+    const R tau = R(a.tau);
+    const int lane = threadIdx.x % kZGroup;
+    const SoftTables<R> t = soft_tables<R>(a);
+    const int groups = gridDim.x * (256 / kZGroup);
+    for (int k = blockIdx.x * (256 / kZGroup) + threadIdx.x / kZGroup; k < count; k += groups) {
+        const int4 it = order[k];
+        if (it.w < 0) continue;
+        const SoftNode c = soft_node(g, a.nodes[it.x]), p = soft_node(g, a.nodes[it.y + it.w]);
+        const Edge E{c.x, c.y, p.x, p.y};
+        const R* bn = t.best + size_t(it.x - a.node0) * L;
+        R* out = t.diag + size_t(it.x - a.node0) * L;
+        if (E.x == E.px || E.y == E.py) {
+            const int d = E.x == E.px;  // a column (also when both coordinates agree)
+            if (lane < L) {
+                R v = R(kSoftInf);
+                if (layer_dir(g, lane) == d && bn[lane] < R(kSoftBig))
+                    v = bn[lane] + R(d ? leg(a, lane, 1, E.x, E.y, E.py) : leg(a, lane, 0, E.y, E.x, E.px));
+                out[lane] = v;
+            }
+            continue;
+        }
+        R best[L];
+        Lse<R> st[L];
+#pragma unroll
+        for (int l = 0; l < L; ++l) best[l] = bn[l], st[l] = lse_empty<R>();
+        auto pass = [&](auto par, int d1) {
+            constexpr int P = decltype(par)::value;
+            for_each_bend<L, P>(a, E, d1, lane, [&](const ZBend<L>& z, int, bool live, int) {
+                R f1[L], mv[L];
+                bend_minima<R, L, P>(z, best, tau, f1, mv);
+#pragma unroll
+                for (int e = 0; e < L; ++e)
+                    if ((e & 1) == P && live && mv[e] < R(kSoftBig)) lse_push(st[e], mv[e] + R(z.last[e]), tau);
+            });
+        };
+        // layer l runs along y (direction 1) where its parity differs from DIR
+        if (g.DIR) {
+            pass(ZParity<0>{}, 1);
+            pass(ZParity<1>{}, 0);
+        } else {
+            pass(ZParity<1>{}, 1);
+            pass(ZParity<0>{}, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < L; ++e) {
+            const R mn = row_reduce(st[e].mn, [](R u, R v) { return v < u ? v : u; });
+            const R s = st[e].mn < R(kSoftBig) ? st[e].s * r_exp<R>(-(st[e].mn - mn) / tau) : R(0);
+            const Lse<R> m{mn, row_reduce(s, [](R u, R v) { return u + v; })};
+            if (lane == e) out[e] = lse_value(m, tau);
+        }
+    }
+}
+
+// One wavefront per net (grid-stride over the slots [begin, begin + count)).
 template <class R, int K>
 __global__ __launch_bounds__(kWave) void soft_backward_kernel(SoftArgs a) {
     __shared__ unsigned char s_lo[kSoftMaxT], s_hi[kSoftMaxT];
@@ -599,7 +869,7 @@ __global__ __launch_bounds__(kWave) void soft_backward_kernel(SoftArgs a) {
         const int n0 = a.node_off[slot], n = a.node_off[slot + 1] - n0;
         const int* nodes = a.nodes + n0;
         const int* parents = a.parents + n0;
-        const NetTables<R> t = net_tables<R>(a, slot);
+        const SoftTables<R> t = net_tables<R>(a, slot);
         const R F = R(a.value[slot - a.begin]);
         if (!(F < R(kSoftBig))) continue;  // uniform over the wave
         for (int e = lane; e < T; e += kWave) t.gD[e] = soft_weight<R>(t.D[e], F, tau);
@@ -763,21 +1033,53 @@ __global__ __launch_bounds__(256) void soft_params_kernel(SoftCostArgs c, const 
 
 size_t soft_scratch_bytes(int L, long long nodes, int precision) {
     const int T = L * (L + 1) / 2;
-    return size_t(nodes) * size_t(2 * T + 4 * L) * (precision == 64 ? 8 : 4);
+    return size_t(nodes) * size_t(2 * T + 2 * L) * (precision == 64 ? 8 : 4);
+}
+
+void launch_soft_levels(const SoftLevelArgs& a, int nodes, int cus, hipStream_t st) {
+    const int blocks = std::max(1, std::min((nodes + kLevelThreads - 1) / kLevelThreads, std::max(1, cus) * 4));
+    hipLaunchKernelGGL(fill_int_kernel, dim3((a.levels + 255) / 256), dim3(256), 0, st, a.cursor, 0, (long long)a.levels);
+    hipLaunchKernelGGL(soft_level_count_kernel, dim3(blocks), dim3(kLevelThreads), 0, st, a);
+    hipLaunchKernelGGL(soft_level_scan_kernel, dim3(1), dim3(kLevelThreads), 0, st, a);
+    hipLaunchKernelGGL(soft_level_place_kernel, dim3((a.count + kLevelThreads - 1) / kLevelThreads), dim3(kLevelThreads),
+                       0, st, a);
 }
 
 namespace {
 int soft_grid(const SoftArgs& a, int cus) { return std::max(1, std::min(a.count, std::max(1, cus) * 32)); }
+
+// workgroups for `count` items of `per` items a workgroup, at most 16 a CU
+int level_grid(int count, int per, int cus) { return std::max(1, std::min((count + per - 1) / per, std::max(1, cus) * 16)); }
+
+template <class R, int L>
+void forward_levels(const SoftArgs& a, const SoftLevels& lv, int kind, int cus, hipStream_t st) {
+    for (int h = 0; h + 1 < int(lv.start.size()); ++h) {
+        const int count = lv.start[h + 1] - lv.start[h];
+        if (!count) continue;
+        const int4* order = lv.order + lv.start[h];
+        const dim3 grid(level_grid(count, 256 / kWave * kNodesPerWave<L>, cus));
+        if (kind) {
+            hipLaunchKernelGGL((soft_forward_level_kernel<R, L, 1>), grid, dim3(256), 0, st, a, order, count);
+            hipLaunchKernelGGL((soft_zedge_level_kernel<R, L>), dim3(level_grid(count, 256 / kZGroup, cus)), dim3(256), 0,
+                               st, a, order, count);
+        } else {
+            hipLaunchKernelGGL((soft_forward_level_kernel<R, L, 0>), grid, dim3(256), 0, st, a, order, count);
+        }
+    }
+}
 }  // namespace
 
-void launch_soft_forward(const SoftArgs& a, int precision, int kind, int cus, hipStream_t st) {
-    const dim3 grid(soft_grid(a, cus));
-    if (precision == 64) {
-        if (kind) hipLaunchKernelGGL((soft_forward_kernel<double, 1>), grid, dim3(kWave), 0, st, a);
-        else hipLaunchKernelGGL((soft_forward_kernel<double, 0>), grid, dim3(kWave), 0, st, a);
-    } else {
-        if (kind) hipLaunchKernelGGL((soft_forward_kernel<float, 1>), grid, dim3(kWave), 0, st, a);
-        else hipLaunchKernelGGL((soft_forward_kernel<float, 0>), grid, dim3(kWave), 0, st, a);
+void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, int cus, hipStream_t st) {
+    switch (a.g.L) {
+#define GR_SOFT_CASE(n)                                                        \
+    case n:                                                                    \
+        if (precision == 64) forward_levels<double, n>(a, lv, kind, cus, st);  \
+        else forward_levels<float, n>(a, lv, kind, cus, st);                   \
+        break;
+        GR_SOFT_CASE(1) GR_SOFT_CASE(2) GR_SOFT_CASE(3) GR_SOFT_CASE(4) GR_SOFT_CASE(5)
+        GR_SOFT_CASE(6) GR_SOFT_CASE(7) GR_SOFT_CASE(8) GR_SOFT_CASE(9) GR_SOFT_CASE(10)
+#undef GR_SOFT_CASE
+        default: break;
     }
 }
 
