@@ -177,8 +177,8 @@ struct gr_ctx {
     std::vector<int> geom_pt_off;  // host copy of the point offsets
     // soft DP: cost arrays, per-cell gradients, checkpointed tables
     Workspace soft_ws, soft_tables, soft_level_ws;
-    // the nodes of the last call's slot range by height, kept while the range
-    // and the uploaded stage stay the same
+    // the level order of the last call's slot range, kept while the range and
+    // the uploaded stage stay the same
     SoftLevels soft_levels;
     std::vector<int> soft_levels_key;  // stage generation, begin, count
     SoftCostArgs soft_cost{};
@@ -1078,17 +1078,17 @@ void ensure_soft_levels(gr_ctx* c, int begin, int count, int nodes) {
     c->soft_levels_key.clear();
     int levels = 1;
     for (int s = begin; s < begin + count; ++s) levels = std::max(levels, c->height_h[s] + 1);
-    SoftLevelArgs a{c->node_off, c->parents, c->lvl, begin, count, levels, nullptr, nullptr, nullptr};
+    SoftLevelArgs a{c->node_off, c->parents, c->lvl, begin, count, 1, levels, nullptr, nullptr};
+    // four workgroups a CU where there are nets for them (measured in soft.hip)
+    a.chunk = std::max(1, std::min(kSoftChunkNets, count / std::max(1, c->cus * 4)));
+    const int chunks = (count + a.chunk - 1) / a.chunk, bins = soft_level_bins(levels);
     c->soft_level_ws.carve([&](auto& cv) {
-        a.cursor = cv.template take<int>(levels);
-        a.start = cv.template take<int>(levels + 1);
+        a.start = cv.template take<int>(size_t(chunks) * (bins + 1));
         a.order = cv.template take<int4>(nodes);
     });
-    launch_soft_levels(a, nodes, c->cus, c->stream);
+    launch_soft_chunks(a, c->stream);
+    c->soft_levels = SoftLevels{a.order, a.start, a.chunk, bins};
     hip_check(hipGetLastError(), "soft level kernels");
-    c->soft_levels.start.resize(levels + 1);
-    c->soft_levels.order = a.order;
-    download(c->soft_levels.start.data(), a.start, sizeof(int) * (levels + 1), c->stream);
     c->soft_levels_key = key;
 }
 
@@ -1160,7 +1160,7 @@ void soft_forward(gr_ctx* c, int begin, int count, double slope, double zero_slo
         hipLaunchKernelGGL(soft_prefix_kernel, dim3(c->tracks), dim3(256), 0, c->stream, c->g, sc.wcost, sc.presum);
     else
         hipLaunchKernelGGL(soft_costs_kernel, dim3(c->tracks), dim3(256), 0, c->stream, sc);
-    if (count) launch_soft_forward(a, c->soft_levels, precision, c->soft_kind, c->cus, c->stream);
+    if (count) launch_soft_forward(a, c->soft_levels, precision, c->soft_kind, c->stream);
     hip_check(hipEventRecord(e1, c->stream), "hipEventRecord");
     hip_check(hipGetLastError(), "soft forward kernels");
     std::vector<double> v(std::max(count, 1));
@@ -2666,7 +2666,7 @@ int gr_soft_backward(gr_ctx* c, double* grad_params, double* elapsed_ms) {
                   "clear parameter gradients");
         hipEvent_t e0 = take_event(c), e1 = take_event(c);
         hip_check(hipEventRecord(e0, c->stream), "hipEventRecord");
-        if (a.count) launch_soft_backward(a, c->soft_precision, c->soft_kind, c->cus, c->stream);
+        if (a.count) launch_soft_backward(a, c->soft_levels, c->soft_precision, c->soft_kind, c->stream);
         const int blocks = int(std::min<size_t>(1024, (cells + 255) / 256));
         if (!c->soft_given)  // the cost-model parameters exist only for model costs
             hipLaunchKernelGGL(soft_params_kernel, dim3(blocks), dim3(256), 0, c->stream, c->soft_cost, a.gw, a.gv,

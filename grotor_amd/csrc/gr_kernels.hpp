@@ -1,8 +1,6 @@
 // Kernel declarations and launch-argument structures of the gfx950 hot path.
 #pragma once
 
-#include <vector>
-
 #include "gr_device.hpp"
 
 namespace grotor {
@@ -303,25 +301,28 @@ __global__ void soft_params_kernel(SoftCostArgs c, const double* gw, const doubl
 __global__ void soft_prefix_kernel(DeviceGrid g, const double* wcost, double* presum);
 constexpr int kSoftLayers = 10;  // routing layers the soft DP supports
 size_t soft_scratch_bytes(int L, long long nodes, int precision);
-// The nodes of the slots [begin, begin + count) by height: `levels` heights,
-// order[start[h] .. start[h + 1]) the nodes of height h.
+// The slots [begin, begin + count) in chunks of `chunk` nets, each chunk's nodes
+// by height (soft.hip).
+constexpr int kSoftChunkNets = 64;
 struct SoftLevelArgs {
     const int* node_off;
     const int* parents;
     const int* lvl;  // per net position: node | height << 16
-    int begin, count, levels;
-    int* cursor;  // [levels]
-    int* start;   // [levels + 1]
-    int4* order;  // {node, first node of its net, slot - begin, parent (-1: root)}
+    int begin, count;
+    int chunk, levels;  // nets per chunk (at most kSoftChunkNets), heights of the tallest net
+    int* start;         // per chunk soft_level_bins(levels) + 1 level starts
+    int4* order;        // {node, first node of its net, slot - begin, parent (-1: root)}
 };
-void launch_soft_levels(const SoftLevelArgs& a, int nodes, int cus, hipStream_t stream);
+int soft_level_bins(int levels);
+void launch_soft_chunks(const SoftLevelArgs& a, hipStream_t stream);
 struct SoftLevels {
-    std::vector<int> start;  // host copy
     const int4* order = nullptr;
+    const int* dstart = nullptr;
+    int chunk = 1, bins = 1;
 };
 // kind 0: L-shape edges, 1: the Z-shape route family
-void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, int cus, hipStream_t stream);
-void launch_soft_backward(const SoftArgs& a, int precision, int kind, int cus, hipStream_t stream);
+void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, hipStream_t stream);
+void launch_soft_backward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, hipStream_t stream);
 
 // Evaluator-equivalent score (resources/evaluator.cpp:458-675)
 struct ScoreArgs {

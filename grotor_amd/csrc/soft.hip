@@ -32,11 +32,10 @@
 // scatters dF/dwcost (expected wire edge use) and dF/dvcost (expected via
 // landings) into FP64 accumulators.
 //
-// The forward pass runs level by level over the nodes of all nets (see "level
-// order" below), L lanes per node, and for kind 1 over the edges of a level,
-// 16 lanes each, lane = bend position; the adjoint one wavefront per net.  R,
-// the type of the tables and of exp / log, is float or double; costs and
-// gradients stay FP64.
+// Both passes run level by level over the nodes of a chunk of nets (see
+// "chunks of nets" below), L lanes per node, and for kind 1 over the edges of
+// a level, 16 lanes each, lane = bend position.  R, the type of the tables and of exp /
+// log, is float or double; costs and gradients stay FP64.
 #include "gr_kernels.hpp"
 
 namespace grotor {
@@ -45,7 +44,6 @@ namespace {
 
 constexpr double kSoftInf = 1e22;
 constexpr double kSoftBig = 1e20;
-constexpr int kSoftMaxT = kSoftLayers * (kSoftLayers + 1) / 2;
 
 __device__ __forceinline__ double soft_e(double cap, double dem, double s, double z, double& ds, double& dz) {
     ds = dz = 0.0;
@@ -103,33 +101,11 @@ __device__ __forceinline__ Lse<R> lse_empty() {
 }
 
 template <class R>
-__device__ __forceinline__ void lse_add(Lse<R>& a, R x, R tau) {
-    if (!(x < R(kSoftBig))) return;
-    if (x < a.mn) {
-        a.s = (a.mn < R(kSoftBig) ? a.s * r_exp<R>(-(a.mn - x) / tau) : R(0)) + R(1);
-        a.mn = x;
-    } else {
-        a.s += r_exp<R>(-(x - a.mn) / tau);
-    }
-}
-
-template <class R>
 __device__ __forceinline__ Lse<R> lse_merge(const Lse<R>& a, const Lse<R>& b, R tau) {
     if (!(b.mn < R(kSoftBig))) return a;
     if (!(a.mn < R(kSoftBig))) return b;
     const R m = a.mn < b.mn ? a.mn : b.mn;
     return Lse<R>{m, a.s * r_exp<R>(-(a.mn - m) / tau) + b.s * r_exp<R>(-(b.mn - m) / tau)};
-}
-
-// every lane receives the merge of all lanes' states (the butterfly adds
-// the same two terms on both partners, so all lanes agree bit for bit)
-template <class R>
-__device__ __forceinline__ Lse<R> lse_wave(Lse<R> a, R tau) {
-    for (int off = kWave / 2; off; off >>= 1) {
-        const Lse<R> b{__shfl_xor(a.mn, off, kWave), __shfl_xor(a.s, off, kWave)};
-        a = lse_merge(a, b, tau);
-    }
-    return a;
 }
 
 template <class R>
@@ -143,43 +119,19 @@ __device__ __forceinline__ R soft_weight(R x, R y, R tau) {
     return r_exp<R>(-(x - y) / tau);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = kWave / 2; off; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
-}
-
-__device__ __forceinline__ int tri_index(int L, int lo, int hi) { return lo * (2 * L - lo + 1) / 2 + (hi - lo); }
-
 // Wire cost of layer l along its track between positions p0 and p1 of the
-// track through `fixed` (x for along_y, else y), from the prefix sums; the
-// gradient variant adds gr to each edge cell [min, max) of the leg.
+// track through `fixed` (x for along_y, else y), from the prefix sums.
 __device__ __forceinline__ double leg(const SoftArgs& a, int l, int along_y, int fixed, int p0, int p1) {
     const int lo = min(p0, p1), hi = max(p0, p1);
     const int c0 = along_y ? cell_of(a.g, l, fixed, lo) : cell_of(a.g, l, lo, fixed);
     const int c1 = along_y ? cell_of(a.g, l, fixed, hi) : cell_of(a.g, l, hi, fixed);
     return a.presum[c1] - a.presum[c0];
 }
-__device__ __forceinline__ void leg_grad(const SoftArgs& a, int l, int along_y, int fixed, int p0, int p1, double gr) {
-    if (gr == 0.0) return;
-    const int lo = min(p0, p1), hi = max(p0, p1);
-    for (int p = lo; p < hi; ++p) atomicAdd(a.gw + (along_y ? cell_of(a.g, l, fixed, p) : cell_of(a.g, l, p, fixed)), gr);
-}
-// via stack at (x, y) between layers l0 and l1: vcost(k), min <= k < max
-__device__ __forceinline__ double stack(const SoftArgs& a, int x, int y, int l0, int l1) {
-    double s = 0.0;
-    for (int k = min(l0, l1); k < max(l0, l1); ++k) s += a.vcost[cell_of(a.g, k, x, y)];
-    return s;
-}
-__device__ __forceinline__ void stack_grad(const SoftArgs& a, int x, int y, int l0, int l1, double gr) {
-    if (gr == 0.0) return;
-    for (int k = min(l0, l1); k < max(l0, l1); ++k) atomicAdd(a.gv + cell_of(a.g, k, x, y), gr);
-}
-
 // Checkpointed tables of the nodes [node0, node0 + table_nodes) of the call,
 // node by node.
 template <class R>
 struct SoftTables {
-    R *D, *gD, *best, *diag;
+    R *D, *best, *diag, *gdiag, *gbest;
 };
 
 template <class R>
@@ -188,170 +140,17 @@ __device__ __forceinline__ SoftTables<R> soft_tables(const SoftArgs& a) {
     const size_t N = size_t(a.table_nodes);
     SoftTables<R> t;
     t.D = reinterpret_cast<R*>(a.scratch);
-    t.gD = t.D + N * T;
-    t.best = t.gD + N * T;
+    t.best = t.D + N * T;
     t.diag = t.best + N * L;
+    t.gdiag = t.diag + N * L;
+    t.gbest = t.gdiag + N * L;
     return t;
-}
-
-template <class R>
-__device__ __forceinline__ SoftTables<R> net_tables(const SoftArgs& a, int slot) {
-    const int L = a.g.L, T = L * (L + 1) / 2;
-    const size_t n0 = size_t(a.node_off[slot] - a.node0);
-    SoftTables<R> t = soft_tables<R>(a);
-    t.D += n0 * T;
-    t.gD += n0 * T;
-    t.best += n0 * L;
-    t.diag += n0 * L;
-    return t;
-}
-
-// Interval table of a workgroup: s_lo[e], s_hi[e] for e = tri_index(L, lo, hi).
-__device__ __forceinline__ void interval_table(int L, unsigned char* s_lo, unsigned char* s_hi) {
-    const int T = L * (L + 1) / 2;
-    for (int e = threadIdx.x; e < T; e += blockDim.x) {
-        int lo = 0, rem = e;
-        while (rem >= L - lo) rem -= L - lo, ++lo;
-        s_lo[e] = (unsigned char)lo;
-        s_hi[e] = (unsigned char)(lo + rem);
-    }
 }
 
 // Geometry of a tree edge from child (x, y) to parent (px, py).
 struct Edge {
     int x, y, px, py;
 };
-
-// ---- kind 1: the Z-shape route family ----
-//
-// zedge() visits every route of the edge as (leaving layer s, arriving
-// layer e, cost): straight and L-shape routes are split over the lanes by
-// arriving layer, the Z-shapes by bend position.  Visit(s, e, cost,
-// scatter) is called with the route's cost; in the adjoint pass it returns
-// the route's weight and then scatter(w) adds w to the route's cells.  The
-// Z-shapes are visited through their nested soft minima: per bend, F1 over
-// the leaving layer, M over the middle layer, then the arriving layer.
-
-// Adjoint of zedge_forward: gdiag[e] = dF/d diag[e]; adds each route's
-// weight to gb[s] (this lane's share of dF/d best[s]) and its cells.
-template <class R>
-__device__ __forceinline__ void zedge_backward(const SoftArgs& a, const Edge& E, const R* best, const R* diag,
-                                               const R* gdiag, R tau, double* gb) {
-    const DeviceGrid& g = a.g;
-    const int L = g.L, lane = threadIdx.x;
-    const int x = E.x, y = E.y, px = E.px, py = E.py;
-    if (x == px || y == py) {
-        const int e = lane;
-        const int dv = x == px;
-        if (e < L && layer_dir(g, e) == dv && gdiag[e] != R(0) && best[e] < R(kSoftBig)) {
-            const double c = dv ? leg(a, e, 1, x, y, py) : leg(a, e, 0, y, x, px);
-            const double w = double(gdiag[e] * soft_weight<R>(best[e] + R(c), diag[e], tau));
-            gb[e] += w;
-            if (dv) leg_grad(a, e, 1, x, y, py, w);
-            else leg_grad(a, e, 0, y, x, px, w);
-        }
-        return;
-    }
-    {
-        const int e = lane;
-        if (e < L && gdiag[e] != R(0)) {
-            const int h = layer_dir(g, e) == 0;  // arriving horizontal: first leg vertical through (x, py)
-            const double last = h ? leg(a, e, 0, py, x, px) : leg(a, e, 1, px, y, py);
-            double wl = 0.0;
-            for (int s = 0; s < L; ++s) {
-                if (layer_dir(g, s) != (h ? 1 : 0) || !(best[s] < R(kSoftBig))) continue;
-                const double first = h ? leg(a, s, 1, x, y, py) : leg(a, s, 0, y, x, px);
-                const double c = first + (h ? stack(a, x, py, s, e) : stack(a, px, y, s, e)) + last;
-                const double w = double(gdiag[e] * soft_weight<R>(best[s] + R(c), diag[e], tau));
-                if (w == 0.0) continue;
-                gb[s] += w;
-                wl += w;
-                if (h) {
-                    leg_grad(a, s, 1, x, y, py, w);
-                    stack_grad(a, x, py, s, e, w);
-                } else {
-                    leg_grad(a, s, 0, y, x, px, w);
-                    stack_grad(a, px, y, s, e, w);
-                }
-            }
-            if (h) leg_grad(a, e, 0, py, x, px, wl);
-            else leg_grad(a, e, 1, px, y, py, wl);
-        }
-    }
-    for (int pass = 0; pass < 2; ++pass) {
-        const int lo = pass == 0 ? min(y, py) : min(x, px), hi = pass == 0 ? max(y, py) : max(x, px);
-        const int d1 = pass == 0 ? 1 : 0;
-        for (int b0 = lo + 1; b0 < hi; b0 += kWave) {
-            const int b = b0 + lane;
-            if (b >= hi) continue;
-            const int ax = pass == 0 ? x : b, ay = pass == 0 ? b : y;
-            const int bx = pass == 0 ? px : b, by = pass == 0 ? b : py;
-            R f1[kSoftLayers], mv[kSoftLayers];
-            double gf1[kSoftLayers], gm[kSoftLayers];
-            for (int m = 0; m < L; ++m) {
-                Lse<R> s1 = lse_empty<R>();
-                if (layer_dir(g, m) != d1)
-                    for (int s = 0; s < L; ++s)
-                        if (layer_dir(g, s) == d1 && best[s] < R(kSoftBig)) {
-                            const double c = (pass == 0 ? leg(a, s, 1, x, y, b) : leg(a, s, 0, y, x, b)) +
-                                             stack(a, ax, ay, s, m);
-                            lse_add(s1, best[s] + R(c), tau);
-                        }
-                f1[m] = lse_value(s1, tau);
-                gf1[m] = 0.0;
-            }
-            for (int e = 0; e < L; ++e) {
-                gm[e] = 0.0;
-                mv[e] = R(kSoftInf);
-                if (layer_dir(g, e) != d1) continue;
-                Lse<R> s2 = lse_empty<R>();
-                for (int m = 0; m < L; ++m)
-                    if (layer_dir(g, m) != d1 && f1[m] < R(kSoftBig)) {
-                        const double c = (pass == 0 ? leg(a, m, 0, b, x, px) : leg(a, m, 1, b, y, py)) +
-                                         stack(a, bx, by, m, e);
-                        lse_add(s2, f1[m] + R(c), tau);
-                    }
-                mv[e] = lse_value(s2, tau);
-                if (mv[e] < R(kSoftBig) && gdiag[e] != R(0)) {
-                    const double c = pass == 0 ? leg(a, e, 1, px, b, py) : leg(a, e, 0, py, b, px);
-                    gm[e] = double(gdiag[e] * soft_weight<R>(mv[e] + R(c), diag[e], tau));
-                    if (pass == 0) leg_grad(a, e, 1, px, b, py, gm[e]);
-                    else leg_grad(a, e, 0, py, b, px, gm[e]);
-                }
-            }
-            // middle legs and the second bend's stacks
-            for (int m = 0; m < L; ++m) {
-                if (layer_dir(g, m) == d1 || !(f1[m] < R(kSoftBig))) continue;
-                const double mid = pass == 0 ? leg(a, m, 0, b, x, px) : leg(a, m, 1, b, y, py);
-                for (int e = 0; e < L; ++e) {
-                    if (layer_dir(g, e) != d1 || gm[e] == 0.0) continue;
-                    const double c = mid + stack(a, bx, by, m, e);
-                    const double w = gm[e] * double(soft_weight<R>(f1[m] + R(c), mv[e], tau));
-                    gf1[m] += w;
-                    stack_grad(a, bx, by, m, e, w);
-                }
-                if (pass == 0) leg_grad(a, m, 0, b, x, px, gf1[m]);
-                else leg_grad(a, m, 1, b, y, py, gf1[m]);
-            }
-            // first legs and the first bend's stacks
-            for (int s = 0; s < L; ++s) {
-                if (layer_dir(g, s) != d1 || !(best[s] < R(kSoftBig))) continue;
-                const double first = pass == 0 ? leg(a, s, 1, x, y, b) : leg(a, s, 0, y, x, b);
-                double ws = 0.0;
-                for (int m = 0; m < L; ++m) {
-                    if (layer_dir(g, m) == d1 || gf1[m] == 0.0) continue;
-                    const double c = first + stack(a, ax, ay, s, m);
-                    const double w = gf1[m] * double(soft_weight<R>(best[s] + R(c), f1[m], tau));
-                    ws += w;
-                    stack_grad(a, ax, ay, s, m, w);
-                }
-                gb[s] += ws;
-                if (pass == 0) leg_grad(a, s, 1, x, y, b, ws);
-                else leg_grad(a, s, 0, y, x, b, ws);
-            }
-        }
-    }
-}
 
 }  // namespace
 
@@ -417,86 +216,10 @@ __global__ __launch_bounds__(256) void soft_costs_kernel(SoftCostArgs a) {
 }
 
 
-// ---- level order ----
-//
-// Both passes run over the nodes of all nets of the call level by level: a
-// node's level is its height in its tree, so a level's nodes depend on lower
-// levels only (forward) or on higher ones only (adjoint), and every launch
-// has the whole batch's nodes of a level to fill the chip with.  One
-// wavefront per net, its nodes one after another, kept 8 of 64 lanes busy and
-// every table a dependent round trip away.
-//
-// The order is three small kernels per (stage, slot range): count the nodes
-// per height, scan, place.  Blocks gather their counts in LDS (heights below
-// kLevelBins), one atomic per block and height.
+// Level order: a node's level is its height in its tree, so a level's nodes
+// depend on lower levels only (forward) or on higher ones only (adjoint).
 constexpr int kLevelBins = 256;
 constexpr int kLevelThreads = 256;
-
-__global__ __launch_bounds__(kLevelThreads) void soft_level_count_kernel(SoftLevelArgs a) {
-    __shared__ int s_bin[kLevelBins];
-    for (int h = threadIdx.x; h < kLevelBins; h += kLevelThreads) s_bin[h] = 0;
-    __syncthreads();
-    const int q0 = a.node_off[a.begin], q1 = a.node_off[a.begin + a.count];
-    for (int q = q0 + blockIdx.x * kLevelThreads + threadIdx.x; q < q1; q += gridDim.x * kLevelThreads) {
-        const int h = a.lvl[q] >> 16;
-        atomicAdd(h < kLevelBins ? s_bin + h : a.cursor + h, 1);
-    }
-    __syncthreads();
-    for (int h = threadIdx.x; h < min(kLevelBins, a.levels); h += kLevelThreads)
-        if (s_bin[h]) atomicAdd(a.cursor + h, s_bin[h]);
-}
-
-// cursor[h]: counts in, exclusive prefix out; start[0 .. levels] the same
-// with the total at the end.  One workgroup.
-__global__ __launch_bounds__(kLevelThreads) void soft_level_scan_kernel(SoftLevelArgs a) {
-    __shared__ int s_part[kLevelThreads];
-    const int k = (a.levels + kLevelThreads - 1) / kLevelThreads;
-    const int p0 = min(a.levels, int(threadIdx.x) * k), p1 = min(a.levels, p0 + k);
-    int sum = 0;
-    for (int p = p0; p < p1; ++p) sum += a.cursor[p];
-    s_part[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int t = 0; t < kLevelThreads; ++t) {
-            const int v = s_part[t];
-            s_part[t] = run;
-            run += v;
-        }
-        a.start[a.levels] = run;
-    }
-    __syncthreads();
-    int run = s_part[threadIdx.x];
-    for (int p = p0; p < p1; ++p) {
-        const int v = a.cursor[p];
-        a.cursor[p] = a.start[p] = run;
-        run += v;
-    }
-}
-
-// order[...] = {node, first node of its net, slot - begin, parent (-1: root)};
-// one thread per slot
-__global__ __launch_bounds__(kLevelThreads) void soft_level_place_kernel(SoftLevelArgs a) {
-    __shared__ int s_bin[kLevelBins];
-    const int k = blockIdx.x * kLevelThreads + threadIdx.x;
-    const int n0 = k < a.count ? a.node_off[a.begin + k] : 0;
-    const int n = k < a.count ? a.node_off[a.begin + k + 1] - n0 : 0;
-    for (int h = threadIdx.x; h < kLevelBins; h += kLevelThreads) s_bin[h] = 0;
-    __syncthreads();
-    for (int i = 0; i < n; ++i) {
-        const int h = a.lvl[n0 + i] >> 16;
-        if (h < kLevelBins) atomicAdd(s_bin + h, 1);
-    }
-    __syncthreads();
-    for (int h = threadIdx.x; h < min(kLevelBins, a.levels); h += kLevelThreads)
-        if (s_bin[h]) s_bin[h] = atomicAdd(a.cursor + h, s_bin[h]);
-    __syncthreads();
-    for (int i = 0; i < n; ++i) {
-        const int q = a.lvl[n0 + i], h = q >> 16, v = q & 0xFFFF;
-        const int at = atomicAdd(h < kLevelBins ? s_bin + h : a.cursor + h, 1);
-        a.order[at] = make_int4(n0 + v, n0, k, a.parents[n0 + v]);
-    }
-}
 
 namespace {
 
@@ -592,21 +315,20 @@ __device__ __forceinline__ void bent_candidates(const DeviceGrid& g, const EdgeC
 
 }  // namespace
 
-// One level of the forward pass: per node its intervals (via stack plus the
-// closures of its children), the soft minima per layer, and for kind 0 the
-// edge to its parent; a root's value.  L lanes per node.  Bound by the
+// Nodes of one level of the forward pass: per node its intervals (via stack
+// plus the closures of its children), the soft minima per layer, and for kind
+// 0 the edge to its parent; a root's value.  L lanes per node.  Bound by the
 // instruction issue of the exponentials and logarithms (about 4 L per lane)
-// and, on the upper levels, by the launch itself.  Against one wavefront per
-// net, forward over 465k nodes of 8 layers in binary32: 1.61 -> 0.33 ms.
+// and the latency of the gathers.  Against one wavefront per net, 465k nodes
+// of 8 layers in binary32: 1.61 -> 0.25 ms.
 template <class R, int L, int K>
-__global__ __launch_bounds__(256) void soft_forward_level_kernel(SoftArgs a, const int4* order, int count) {
+__device__ __forceinline__ void forward_nodes(const SoftArgs& a, const int4* order, int count, int first, int waves) {
     constexpr int T = L * (L + 1) / 2, G = kNodesPerWave<L>;
     const DeviceGrid& g = a.g;
     const R tau = R(a.tau);
     const int wl = threadIdx.x & (kWave - 1), grp = wl / L, lane = wl % L;
     const SoftTables<R> t = soft_tables<R>(a);
-    const int waves = gridDim.x * (256 / kWave);
-    for (int w = blockIdx.x * (256 / kWave) + threadIdx.x / kWave; w * G < count; w += waves) {
+    for (int w = first; w * G < count; w += waves) {
         const int k = w * G + grp;
         if (grp >= G || k >= count) continue;  // whole groups: no shuffle crosses a group
         const int4 it = order[k];
@@ -788,7 +510,7 @@ __device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, 
 
 }  // namespace
 
-// Kind 1: one level's edges, 16 lanes each: lane = bend, the lanes' soft
+// Kind 1: edges of one level, 16 lanes each: lane = bend, the lanes' soft
 // minima per arriving layer merged over the row (the minimum first, then one
 // exponential per lane and layer).  Every via cost and prefix sum of a bend is
 // loaded once into registers, where the one-wavefront-per-net form read each
@@ -796,15 +518,15 @@ __device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, 
 // (about L^2 / 2 per bend) at three wavefronts per SIMD.  16 lanes an edge:
 // 8 and 4 lanes leave fewer idle on the usual box of 5 x 5 cells but make the
 // long edges the tail (forward over 188k nodes, 8 layers, binary32, tau =
-// 0.1: 0.66 ms at 16, 0.80 at 8, 0.97 at 4; before, 1.33).
+// 0.1: 0.66 ms at 16, 0.80 at 8, 0.97 at 4, one launch per level; 0.53 by
+// chunks; before, 1.33).
 template <class R, int L>
-__global__ __launch_bounds__(256) void soft_zedge_level_kernel(SoftArgs a, const int4* order, int count) {
+__device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* order, int count, int first, int groups) {
     const DeviceGrid& g = a.g;
     const R tau = R(a.tau);
     const int lane = threadIdx.x % kZGroup;
     const SoftTables<R> t = soft_tables<R>(a);
-    const int groups = gridDim.x * (256 / kZGroup);
-    for (int k = blockIdx.x * (256 / kZGroup) + threadIdx.x / kZGroup; k < count; k += groups) {
+    for (int k = first; k < count; k += groups) {
         const int4 it = order[k];
         if (it.w < 0) continue;
         const SoftNode c = soft_node(g, a.nodes[it.x]), p = soft_node(g, a.nodes[it.y + it.w]);
@@ -853,122 +575,443 @@ __global__ __launch_bounds__(256) void soft_zedge_level_kernel(SoftArgs a, const
     }
 }
 
-// One wavefront per net (grid-stride over the slots [begin, begin + count)).
-template <class R, int K>
-__global__ __launch_bounds__(kWave) void soft_backward_kernel(SoftArgs a) {
-    __shared__ unsigned char s_lo[kSoftMaxT], s_hi[kSoftMaxT];
-    __shared__ R s_C[kSoftMaxT], s_gC[kSoftMaxT];
-    __shared__ R s_best[kSoftLayers], s_diag[kSoftLayers], s_gdiag[kSoftLayers], s_gbest[kSoftLayers];
-    const int lane = threadIdx.x;
-    const DeviceGrid& g = a.g;
-    const int L = g.L, X = g.X, Y = g.Y, T = L * (L + 1) / 2;
-    const R tau = R(a.tau);
-    interval_table(L, s_lo, s_hi);
-    __syncthreads();
-    for (int slot = a.begin + blockIdx.x; slot < a.begin + a.count; slot += gridDim.x) {
-        const int n0 = a.node_off[slot], n = a.node_off[slot + 1] - n0;
-        const int* nodes = a.nodes + n0;
-        const int* parents = a.parents + n0;
-        const SoftTables<R> t = net_tables<R>(a, slot);
-        const R F = R(a.value[slot - a.begin]);
-        if (!(F < R(kSoftBig))) continue;  // uniform over the wave
-        for (int e = lane; e < T; e += kWave) t.gD[e] = soft_weight<R>(t.D[e], F, tau);
-        __syncthreads();
-        for (int c = 1; c < n; ++c) {
-            const int p = parents[c];
-            const Edge E{nodes[c] / Y % X, nodes[c] % Y, nodes[p] / Y % X, nodes[p] % Y};
-            const R* dg = t.diag + size_t(c) * L;
-            const R* gC = t.gD + size_t(p) * T;
-            for (int e = lane; e < T; e += kWave) {
-                Lse<R> st = lse_empty<R>();
-                for (int h = s_lo[e]; h <= s_hi[e]; ++h) lse_add(st, dg[h], tau);
-                s_C[e] = lse_value(st, tau);
-                s_gC[e] = gC[e];
-            }
-            if (lane < L) {
-                s_best[lane] = t.best[size_t(c) * L + lane];
-                s_diag[lane] = dg[lane];
-            }
-            __syncthreads();
-            if (lane < L) {
-                const int h = lane;
-                R s = 0;
-                for (int lo = 0; lo <= h; ++lo)
-                    for (int hi = h; hi < L; ++hi) {
-                        const int e = tri_index(L, lo, hi);
-                        if (s_gC[e] != R(0)) s += s_gC[e] * soft_weight<R>(s_diag[h], s_C[e], tau);
-                    }
-                s_gdiag[h] = s;
-            }
-            __syncthreads();
-            double gb[kSoftLayers];
+namespace {
+
+// gr added to the wire cells [lo, hi) of layer l's track through `fixed`,
+// spread over `width` lanes: consecutive lanes take consecutive cells, which
+// is one 64-byte segment for eight of them (scattered atomics run at 24 G/s
+// here, eight to a segment at 180 G/s).  Every lane of the group calls it.
+__device__ __forceinline__ void spread_leg(const SoftArgs& a, int l, int along_y, int fixed, int p0, int p1, double gr,
+                                           int lane, int width) {
+    if (gr == 0.0) return;
+    const int lo = min(p0, p1), hi = max(p0, p1);
+    double* base = a.gw + (along_y ? cell_of(a.g, l, fixed, 0) : cell_of(a.g, l, 0, fixed));
+    for (int p = lo + lane; p < hi; p += width) atomicAdd(base + p, gr);
+}
+
+// Layer k's sum over the rows that contain it: v[m] of lane k - m, m = 0 ..
+// k (row k - m, intervals reaching at least k).
+template <int L, class R>
+__device__ __forceinline__ R gather_rows(const R (&v)[L], int lane, int wl) {
+    R s = v[0];
 #pragma unroll
-            for (int k = 0; k < kSoftLayers; ++k) gb[k] = 0.0;
+    for (int m = 1; m < L; ++m) {
+        const R o = from_lane(v[m], lane >= m ? wl - m : wl);
+        s += lane >= m ? o : R(0);
+    }
+    return s;
+}
+
+}  // namespace
+
+// Nodes of one level of the adjoint: for kind 0 the edge of each node to its parent
+// (gdiag -> gbest, wires and corner vias), then the node itself: dF/dD of its
+// intervals in registers, its via stack, and its children's gdiag.  A root
+// starts from its value.  L lanes per node, as in the forward pass.
+//  - gD[lo][hi] = sum over k in [lo, hi] of gbest[k] exp(-(D - best[k]) / tau)
+//    runs along hi with the terms scaled by the largest best so far (two
+//    exponentials an entry instead of one per layer of the interval), and
+//    gdiag of a child along hi downwards, its closures growing: every factor
+//    stays within (0, 1].
+//  - a layer's first legs of all its routes end in one weight, so a leg's
+//    cells are added once per layer, by the group's lanes side by side.
+// Bound by the atomics' 64-byte segments and the latency of the gathers.
+// Against one wavefront per net with an atomic per route and cell from one
+// lane, 465k nodes of 8 layers in binary32: 1.78 -> 0.48 ms.
+template <class R, int L, int K>
+__device__ __forceinline__ void backward_nodes(const SoftArgs& a, const int4* order, int count, int first, int waves) {
+    constexpr int T = L * (L + 1) / 2, G = kNodesPerWave<L>;
+    const DeviceGrid& g = a.g;
+    const R tau = R(a.tau);
+    const int wl = threadIdx.x & (kWave - 1), grp = wl / L, lane = wl % L;
+    const SoftTables<R> t = soft_tables<R>(a);
+    for (int w = first; w * G < count; w += waves) {
+        const int k = w * G + grp;
+        if (grp >= G || k >= count) continue;  // whole groups: no shuffle crosses a group
+        const int4 it = order[k];
+        const int node = it.x, n0 = it.y;
+        const SoftNode nd = soft_node(g, a.nodes[node]);
+        const size_t row = size_t(node - a.node0) * L + lane;
+        const R* Dn = t.D + size_t(node - a.node0) * T + (lane * (2 * L - lane + 1)) / 2;
+        R D[L], gD[L];
+#pragma unroll
+        for (int m = 0; m < L; ++m) D[m] = lane + m < L ? Dn[m] : R(kSoftInf);
+        if (it.w < 0) {
+            const R F = R(a.value[it.z]);
+#pragma unroll
+            for (int m = 0; m < L; ++m) gD[m] = soft_weight<R>(D[m], F, tau);
+        } else {
+            const R best = t.best[row];
+            R gbest;
             if (K == 0) {
-                const int x = E.x, y = E.y, px = E.px, py = E.py;
-                const bool straight = x == px || y == py;
-                if (lane < L && s_gdiag[lane] != R(0)) {
-                    const int pl = lane, d = layer_dir(g, pl);
-                    if (straight) {
-                        if (d ? x == px : y == py) {
-                            gb[pl] += double(s_gdiag[pl]);
-                            if (d) leg_grad(a, pl, 1, x, y, py, double(s_gdiag[pl]));
-                            else leg_grad(a, pl, 0, y, x, px, double(s_gdiag[pl]));
+                const R diag = t.diag[row], gdiag = t.gdiag[row];
+                const SoftNode pn = soft_node(g, a.nodes[n0 + it.w]);
+                const int x = nd.x, y = nd.y, px = pn.x, py = pn.y;
+                const EdgeCosts ec = edge_costs(a, lane, x, y, px, py);
+                double g1 = 0.0, g2 = 0.0;  // weights of this layer's first and second legs
+                if (ec.straight) {
+                    g1 = ec.along ? double(gdiag) : 0.0;
+                } else {
+                    // corner vias of layer l lie strictly inside the candidates
+                    // between a lane below and a lane above it; their column
+                    // follows the leaving layer's direction, which is l's own
+                    // for an arriving layer at odd distance
+                    double same = 0.0, other = 0.0;
+                    bent_candidates<L>(g, ec, lane, wl, [&](int d, bool down, bool valid, int, double sum) {
+                        const R b = from_lane(best, valid ? (down ? wl - d : wl + d) : wl);
+                        double gr = 0.0;
+                        if (valid && b < R(kSoftBig) && gdiag != R(0))
+                            gr = double(gdiag * soft_weight<R>(b + R(sum), diag, tau));
+                        g2 += gr;
+                        // the leaving lane takes the weight of its first leg
+                        const bool has = down ? lane + d < L : lane >= d;
+                        const double in = from_lane(gr, has ? (down ? wl + d : wl - d) : wl);
+                        g1 += has ? in : 0.0;
+#pragma unroll
+                        for (int j = 1; j < L; ++j) {
+                            if (j >= d) continue;
+                            // arriving lane j above (down) or below, reaching past this layer
+                            const bool in_range = down ? lane + j < L && lane + j >= d : lane >= j && lane - j + d < L;
+                            const double v = from_lane(gr, in_range ? (down ? wl + j : wl - j) : wl);
+                            if (j % 2) same += in_range ? v : 0.0;
+                            else other += in_range ? v : 0.0;
                         }
-                    } else {
-                        // the forward's candidate values, recomputed the same way
-                        const double wpl = d ? leg(a, pl, 1, px, y, py) : leg(a, pl, 0, py, x, px);
-                        double w2 = 0.0;
-                        for (int cl = (pl & 1) ^ 1; cl < L; cl += 2) {
-                            if (!(s_best[cl] < R(kSoftBig))) continue;
-                            const int lo = min(cl, pl), hi = max(cl, pl);
-                            const int dcl = layer_dir(g, cl);
-                            double f = 0.0;
-                            for (int l = lo + 1; l < hi; ++l)
-                                f += dcl ? a.vcost[cell_of(g, l, x, py)] : a.vcost[cell_of(g, l, px, y)];
-                            const double wcl = dcl ? leg(a, cl, 1, x, y, py) : leg(a, cl, 0, y, x, px);
-                            const R tc = s_best[cl] + R(wcl + f + wpl);
-                            const double gr = double(s_gdiag[pl] * soft_weight<R>(tc, s_diag[pl], tau));
-                            if (gr == 0.0) continue;
-                            gb[cl] += gr;
-                            w2 += gr;
-                            if (dcl) leg_grad(a, cl, 1, x, y, py, gr);
-                            else leg_grad(a, cl, 0, y, x, px, gr);
-                            for (int l = lo + 1; l < hi; ++l)
-                                atomicAdd(a.gv + (dcl ? cell_of(g, l, x, py) : cell_of(g, l, px, y)), gr);
-                        }
-                        if (d) leg_grad(a, pl, 1, px, y, py, w2);
-                        else leg_grad(a, pl, 0, py, x, px, w2);
+                    });
+                    const bool v = layer_dir(g, lane) != 0;
+                    const double ga = v ? same : other, gb = v ? other : same;  // corners (x, py), (px, y)
+                    if (ga != 0.0) atomicAdd(a.gv + cell_of(g, lane, x, py), ga);
+                    if (gb != 0.0) atomicAdd(a.gv + cell_of(g, lane, px, y), gb);
+                }
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    const int src = wl - lane + l, d = layer_dir(g, l);
+                    const double v1 = from_lane(g1, src), v2 = from_lane(g2, src);
+                    spread_leg(a, l, d, d ? x : y, d ? y : x, d ? py : px, v1, lane, L);
+                    spread_leg(a, l, d, d ? px : py, d ? y : x, d ? py : px, v2, lane, L);
+                }
+                gbest = R(g1);
+            } else {
+                gbest = t.gbest[row];
+            }
+            R mx = -R(kSoftInf), run = R(0);
+#pragma unroll
+            for (int m = 0; m < L; ++m) {
+                const int src = lane + m < L ? wl + m : wl;
+                const R b = from_lane(best, src), gb = from_lane(gbest, src);
+                gD[m] = R(0);
+                if (lane + m < L && b < R(kSoftBig)) {
+                    if (gb != R(0)) {
+                        const R e = r_exp<R>(-(b < mx ? mx - b : b - mx) / tau);
+                        run = b > mx ? run * e + gb : run + gb * e;
+                        mx = b > mx ? b : mx;
                     }
                 }
+                if (lane + m < L && run != R(0) && D[m] < R(kSoftBig)) gD[m] = run * r_exp<R>(-(D[m] - mx) / tau);
+            }
+        }
+        // via stacks: D[lo][hi] holds vcost(l) for lo <= l < hi
+        {
+            R Q[L], s = R(0);
+#pragma unroll
+            for (int m = L - 1; m >= 0; --m) {
+                Q[m] = s;
+                s += gD[m];
+            }
+            const R v = gather_rows<L>(Q, lane, wl);
+            if (lane < L - 1 && v != R(0)) atomicAdd(a.gv + cell_of(g, lane, nd.x, nd.y), double(v));
+        }
+        // children: dF/d diag[h] = sum over the intervals containing h of
+        // gD exp(-(diag[h] - C) / tau)
+        for (int c = (a.link[node] & 0xFFFF) - 1; c >= 0; c = (a.link[n0 + c] >> 16) - 1) {
+            const size_t crow = size_t(n0 + c - a.node0) * L + lane;
+            const R dl = t.diag[crow];
+            R C[L], P[L];
+#pragma unroll
+            for (int m = 0; m < L; ++m) C[m] = R(kSoftInf);
+            closure_row<L>(dl, lane, wl, tau, [&](int m, R v) { C[m] = v; });
+            R run = R(0), ref = R(kSoftInf);
+#pragma unroll
+            for (int m = L - 1; m >= 0; --m) {
+                const R d = from_lane(dl, lane + m < L ? wl + m : wl);
+                P[m] = R(0);
+                if (lane + m >= L || !(C[m] < R(kSoftBig))) continue;
+                run = (ref < R(kSoftBig) ? run * r_exp<R>(-(C[m] - ref) / tau) : R(0)) + gD[m];
+                ref = C[m];
+                if (run != R(0) && d < R(kSoftBig)) P[m] = run * r_exp<R>(-(d - C[m]) / tau);
+            }
+            t.gdiag[crow] = gather_rows<L>(P, lane, wl);
+        }
+    }
+}
+
+namespace {
+
+// Over a row of 16 lanes: the sum up to and including the lane, the sum of
+// the lanes after it, and the total.
+__device__ __forceinline__ double prefix_sum16(double v, int lane, double& total) {
+#pragma unroll
+    for (int o = 1; o < kZGroup; o <<= 1) {
+        const double u = __shfl_up(v, o, kZGroup);
+        v += lane >= o ? u : 0.0;
+    }
+    total = __shfl(v, kZGroup - 1, kZGroup);
+    return v;
+}
+__device__ __forceinline__ double suffix_sum16(double v, int lane, double& total) {
+#pragma unroll
+    for (int o = 1; o < kZGroup; o <<= 1) {
+        const double u = __shfl_down(v, o, kZGroup);
+        v += lane + o < kZGroup ? u : 0.0;
+    }
+    total = __shfl(v, 0, kZGroup);
+    const double after = __shfl_down(v, 1, kZGroup);
+    return lane + 1 < kZGroup ? after : 0.0;
+}
+
+}  // namespace
+
+// Kind 1: edges of one level of the adjoint, 16 lanes each, lane = bend:
+// gdiag -> gbest, and the weights of every route's cells.  The first and last
+// legs of the bends cover nested runs of one track per layer, so a cell's
+// weight is a running sum over the bends, taken across the lanes, and each
+// cell of those tracks is added once per layer by consecutive lanes; a bend's
+// middle leg is added by the whole row, bend after bend; a via cell's weight is
+// summed over the pairs of layers that pass it before it is added.  Bound by
+// latency at two wavefronts per SIMD (binary32; one in binary64) and, on large
+// boxes, by the middle legs' atomics.  Against one wavefront per net with an
+// atomic per route and cell (8 layers, binary32): 188k nodes, tau = 0.1 1.91
+// -> 0.87 ms; 465k nodes, tau = 10 8.0 -> 2.2 ms.
+template <class R, int L>
+__device__ __forceinline__ void backward_zedges(const SoftArgs& a, const int4* order, int count, int first, int groups) {
+    const DeviceGrid& g = a.g;
+    const R tau = R(a.tau);
+    const int lane = threadIdx.x % kZGroup;
+    const SoftTables<R> t = soft_tables<R>(a);
+    for (int k = first; k < count; k += groups) {
+        const int4 it = order[k];
+        if (it.w < 0) continue;
+        const SoftNode c = soft_node(g, a.nodes[it.x]), p = soft_node(g, a.nodes[it.y + it.w]);
+        const Edge E{c.x, c.y, p.x, p.y};
+        const size_t base = size_t(it.x - a.node0) * L;
+        if (E.x == E.px || E.y == E.py) {
+            const int d = E.x == E.px;
+#pragma unroll
+            for (int l = 0; l < L; ++l) {
+                R w = R(0);
+                if (layer_dir(g, l) == d) {
+                    w = t.gdiag[base + l];
+                    spread_leg(a, l, d, d ? E.x : E.y, d ? E.y : E.x, d ? E.py : E.px, double(w), lane, kZGroup);
+                }
+                if (lane == l) t.gbest[base + l] = w;
+            }
+            continue;
+        }
+        const R *diag = t.diag + base, *gdiag = t.gdiag + base;  // read at their use: registers are short here
+        R best[L];
+        double gb[L];  // this lane's share of dF/d best
+        bool any = false;
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            best[l] = t.best[base + l];
+            gb[l] = 0.0;
+            any |= gdiag[l] != R(0);
+        }
+        auto pass = [&](auto par, int d1) {
+            constexpr int P = decltype(par)::value;
+            const int from = d1 ? E.y : E.x, to = d1 ? E.py : E.px, n = abs(to - from);
+            const bool up = to > from;
+            double before[L];  // last-leg weights of the bends nearer the child
+#pragma unroll
+            for (int l = 0; l < L; ++l) before[l] = 0.0;
+            for_each_bend<L, P>(a, E, d1, lane, [&](const ZBend<L>& z, int b, bool live, int b0) {
+                const int ax = d1 ? E.x : b, ay = d1 ? b : E.y, bx = d1 ? E.px : b, by = d1 ? b : E.py;
+                const int cell = up ? b : b - 1;  // this lane's cell of the first and last legs' tracks
+                R f1[L], mv[L];
+                bend_minima<R, L, P>(z, best, tau, f1, mv);
+                double gm[L], gf[L], gs[L], via[L];
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    gm[l] = gf[l] = gs[l] = via[l] = 0.0;
+                    if ((l & 1) != P) continue;
+                    const R gd = gdiag[l], dg = diag[l];
+                    if (live && mv[l] < R(kSoftBig) && gd != R(0))
+                        gm[l] = double(gd * soft_weight<R>(mv[l] + R(z.last[l]), dg, tau));
+                }
+                // second bend: the middle layers' weights and its via cells
+                stack_pairs<L>(z.vb, [&](int lo, int hi, double s) {
+                    const int e = (lo & 1) == P ? lo : hi, m = (lo & 1) == P ? hi : lo;
+                    double w = 0.0;
+                    if (gm[e] != 0.0 && f1[m] < R(kSoftBig))
+                        w = gm[e] * double(soft_weight<R>(f1[m] + R(z.legs[m] + s), mv[e], tau));
+                    gf[m] += w;
+#pragma unroll
+                    for (int l = 0; l < L; ++l)
+                        if (l >= lo && l < hi) via[l] += w;
+                });
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    if (via[l] != 0.0) atomicAdd(a.gv + cell_of(g, l, bx, by), via[l]);
+                    via[l] = 0.0;
+                }
+                // first bend: the leaving layers' weights and its via cells
+                stack_pairs<L>(z.va, [&](int lo, int hi, double s) {
+                    const int f = (lo & 1) == P ? lo : hi, m = (lo & 1) == P ? hi : lo;
+                    double w = 0.0;
+                    if (!z.corner && gf[m] != 0.0 && best[f] < R(kSoftBig))
+                        w = gf[m] * double(soft_weight<R>(best[f] + R(z.legs[f] + s), f1[m], tau));
+                    gs[f] += w;
+#pragma unroll
+                    for (int l = 0; l < L; ++l)
+                        if (l >= lo && l < hi) via[l] += w;
+                });
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    if (via[l] != 0.0) atomicAdd(a.gv + cell_of(g, l, ax, ay), via[l]);
+                    gb[l] += (l & 1) == P ? gs[l] : z.corner ? gf[l] : 0.0;
+                }
+                const int bends = min(kZGroup, n - b0);
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    if ((l & 1) == P) {
+                        // cell k of the last leg's track is passed by the bends
+                        // up to k, cell k of the first leg's by those after k
+                        double total;
+                        const double w2 = before[l] + prefix_sum16(gm[l], lane, total);
+                        before[l] += total;
+                        const double w1 = suffix_sum16(gs[l], lane, total);
+                        if (live && w2 != 0.0)
+                            atomicAdd(a.gw + (d1 ? cell_of(g, l, E.px, cell) : cell_of(g, l, cell, E.py)), w2);
+                        if (live && w1 != 0.0)
+                            atomicAdd(a.gw + (d1 ? cell_of(g, l, E.x, cell) : cell_of(g, l, cell, E.y)), w1);
+                        // the cells before these 16 bends
+                        if (b0) spread_leg(a, l, d1, d1 ? E.x : E.y, from, up ? from + b0 : from - b0, total, lane, kZGroup);
+                    } else {
+                        for (int q = 0; q < bends; ++q) {
+                            const double w = __shfl(gf[l], q, kZGroup);
+                            const int bq = __shfl(b, q, kZGroup);
+                            spread_leg(a, l, d1 ^ 1, bq, d1 ? E.x : E.y, d1 ? E.px : E.py, w, lane, kZGroup);
+                        }
+                    }
+                }
+            });
+        };
+        if (any) {
+            if (g.DIR) {
+                pass(ZParity<0>{}, 1);
+                pass(ZParity<1>{}, 0);
             } else {
-                zedge_backward<R>(a, E, s_best, s_diag, s_gdiag, tau, gb);
+                pass(ZParity<1>{}, 1);
+                pass(ZParity<0>{}, 0);
             }
-            for (int k = 0; k < L; ++k) {
-                const double v = wave_sum(gb[k]);
-                if (lane == k) s_gbest[k] = R(v);
+        }
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            const double s = row_reduce(gb[l], [](double u, double v) { return u + v; });
+            if (lane == l) t.gbest[base + l] = R(s);
+        }
+    }
+}
+
+// ---- chunks of nets ----
+//
+// Each pass is one launch: a workgroup of four wavefronts takes a chunk of
+// nets through their levels, a level's nodes of all its nets at a time, with
+// barriers between the levels.  One wavefront per net, its nodes one after
+// another, kept 8 of 64 lanes busy; one launch per level over all nets fills
+// the chip on the low levels but pays a launch for each of the few nodes of
+// the high ones (forward and adjoint of 2k nets, 6k nodes, Z-shape, binary64:
+// 0.53 ms against 0.21 here; of 96k nets, 465k nodes, L-shape, binary32 0.86
+// against 0.72; before, 0.37 and 3.47).  Nets per chunk: four workgroups a CU
+// where the call has that many nets (at least one net, at most 64), between
+// the small calls, which want every net on its own (eight a CU: 0.21 ms there
+// too), and the large, which want full levels (11k nets, Z-shape, binary32:
+// 0.77 ms at four a CU, 1.00 at eight, 1.18 at two).
+
+// The order of a chunk: its nodes by height; those of height kLevelBins - 1
+// and above net by net (each net's by height), which the passes take one at a
+// time.  start: a row of bins + 1 per chunk.
+__global__ __launch_bounds__(kLevelThreads) void soft_chunk_order_kernel(SoftLevelArgs a) {
+    __shared__ int s_off[kSoftChunkNets + 1], s_bin[kLevelBins + 1];
+    const int k0 = blockIdx.x * a.chunk, nets = min(a.chunk, a.count - k0);
+    const int bins = min(a.levels, kLevelBins);
+    for (int i = threadIdx.x; i <= nets; i += kLevelThreads) s_off[i] = a.node_off[a.begin + k0 + i];
+    for (int h = threadIdx.x; h <= kLevelBins; h += kLevelThreads) s_bin[h] = 0;
+    __syncthreads();
+    const int q0 = s_off[0], q1 = s_off[nets];
+    for (int q = q0 + threadIdx.x; q < q1; q += kLevelThreads) atomicAdd(s_bin + min(a.lvl[q] >> 16, kLevelBins - 1), 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int run = 0;
+        for (int h = 0; h < bins; ++h) {
+            const int v = s_bin[h];
+            s_bin[h] = run;
+            run += v;
+        }
+        s_bin[bins] = run;
+    }
+    __syncthreads();
+    int* row = a.start + size_t(blockIdx.x) * (bins + 1);
+    for (int h = threadIdx.x; h <= bins; h += kLevelThreads) row[h] = s_bin[h];
+    __syncthreads();
+    int4* order = a.order + (q0 - a.node_off[a.begin]);
+    for (int q = q0 + threadIdx.x; q < q1; q += kLevelThreads) {
+        const int h = a.lvl[q] >> 16, v = a.lvl[q] & 0xFFFF;
+        if (h >= kLevelBins - 1) continue;
+        int lo = 0, hi = nets - 1;  // last net that starts at or before q
+        while (lo < hi) {
+            const int m = (lo + hi + 1) >> 1;
+            if (s_off[m] <= q) lo = m;
+            else hi = m - 1;
+        }
+        const int n0 = s_off[lo];
+        order[atomicAdd(s_bin + h, 1)] = make_int4(n0 + v, n0, k0 + lo, a.parents[n0 + v]);
+    }
+    if (threadIdx.x == 0 && bins == kLevelBins) {
+        int at = s_bin[kLevelBins - 1];
+        for (int i = 0; i < nets; ++i) {
+            const int n0 = s_off[i], n = s_off[i + 1] - n0;
+            int q = n;  // a net's level order is by height: its tall nodes end it
+            while (q > 0 && a.lvl[n0 + q - 1] >> 16 >= kLevelBins - 1) --q;
+            for (; q < n; ++q) {
+                const int v = a.lvl[n0 + q] & 0xFFFF;
+                order[at++] = make_int4(n0 + v, n0, k0 + i, a.parents[n0 + v]);
             }
-            __syncthreads();
-            const R* Dc = t.D + size_t(c) * T;
-            R* gDc = t.gD + size_t(c) * T;
-            for (int e = lane; e < T; e += kWave) {
-                R s = 0;
-                const R d = Dc[e];
-                for (int k = s_lo[e]; k <= s_hi[e]; ++k)
-                    if (s_gbest[k] != R(0)) s += s_gbest[k] * soft_weight<R>(d, s_best[k], tau);
-                gDc[e] = s;
-            }
+        }
+    }
+}
+
+template <class R, int L, int K>
+__global__ __launch_bounds__(256) void soft_forward_chunk_kernel(SoftArgs a, SoftLevels lv) {
+    const int* start = lv.dstart + size_t(blockIdx.x) * (lv.bins + 1);
+    const int4* order = lv.order + (a.node_off[a.begin + blockIdx.x * lv.chunk] - a.node0);
+    const int wave = threadIdx.x / kWave, group = threadIdx.x / kZGroup;
+    const int bins = min(lv.bins, kLevelBins - 1), tall = lv.bins == kLevelBins ? start[bins + 1] - start[bins] : 0;
+    for (int h = 0; h < bins + tall; ++h) {
+        const int b = h < bins ? start[h] : start[bins] + h - bins, e = h < bins ? start[h + 1] : b + 1;
+        if (b == e) break;  // heights are contiguous
+        forward_nodes<R, L, K>(a, order + b, e - b, wave, 256 / kWave);
+        __syncthreads();
+        if (K) {
+            forward_zedges<R, L>(a, order + b, e - b, group, 256 / kZGroup);
             __syncthreads();
         }
-        // via stacks: D_i[lo][hi] holds vcost(l) for lo <= l < hi
-        for (int q = lane; q < n * (L - 1); q += kWave) {
-            const int i = q / (L - 1), l = q % (L - 1);
-            const int x = nodes[i] / Y % X, y = nodes[i] % Y;
-            R s = 0;
-            for (int lo = 0; lo <= l; ++lo)
-                for (int hi = l + 1; hi < L; ++hi) s += t.gD[size_t(i) * T + tri_index(L, lo, hi)];
-            if (s != R(0)) atomicAdd(a.gv + cell_of(g, l, x, y), double(s));
+    }
+}
+
+template <class R, int L, int K>
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? 2 : 1) void soft_backward_chunk_kernel(SoftArgs a, SoftLevels lv) {
+    const int* start = lv.dstart + size_t(blockIdx.x) * (lv.bins + 1);
+    const int4* order = lv.order + (a.node_off[a.begin + blockIdx.x * lv.chunk] - a.node0);
+    const int wave = threadIdx.x / kWave, group = threadIdx.x / kZGroup;
+    const int bins = min(lv.bins, kLevelBins - 1), tall = lv.bins == kLevelBins ? start[bins + 1] - start[bins] : 0;
+    for (int h = bins + tall - 1; h >= 0; --h) {
+        const int b = h < bins ? start[h] : start[bins] + h - bins, e = h < bins ? start[h + 1] : b + 1;
+        if (b == e) continue;
+        if (K) {
+            backward_zedges<R, L>(a, order + b, e - b, group, 256 / kZGroup);
+            __syncthreads();
         }
+        backward_nodes<R, L, K>(a, order + b, e - b, wave, 256 / kWave);
         __syncthreads();
     }
 }
@@ -1033,48 +1076,36 @@ __global__ __launch_bounds__(256) void soft_params_kernel(SoftCostArgs c, const 
 
 size_t soft_scratch_bytes(int L, long long nodes, int precision) {
     const int T = L * (L + 1) / 2;
-    return size_t(nodes) * size_t(2 * T + 2 * L) * (precision == 64 ? 8 : 4);
+    return size_t(nodes) * size_t(T + 4 * L) * (precision == 64 ? 8 : 4);
 }
 
-void launch_soft_levels(const SoftLevelArgs& a, int nodes, int cus, hipStream_t st) {
-    const int blocks = std::max(1, std::min((nodes + kLevelThreads - 1) / kLevelThreads, std::max(1, cus) * 4));
-    hipLaunchKernelGGL(fill_int_kernel, dim3((a.levels + 255) / 256), dim3(256), 0, st, a.cursor, 0, (long long)a.levels);
-    hipLaunchKernelGGL(soft_level_count_kernel, dim3(blocks), dim3(kLevelThreads), 0, st, a);
-    hipLaunchKernelGGL(soft_level_scan_kernel, dim3(1), dim3(kLevelThreads), 0, st, a);
-    hipLaunchKernelGGL(soft_level_place_kernel, dim3((a.count + kLevelThreads - 1) / kLevelThreads), dim3(kLevelThreads),
-                       0, st, a);
+void launch_soft_chunks(const SoftLevelArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(soft_chunk_order_kernel, dim3((a.count + a.chunk - 1) / a.chunk), dim3(kLevelThreads), 0, st, a);
 }
+
+int soft_level_bins(int levels) { return std::min(levels, kLevelBins); }
 
 namespace {
-int soft_grid(const SoftArgs& a, int cus) { return std::max(1, std::min(a.count, std::max(1, cus) * 32)); }
-
-// workgroups for `count` items of `per` items a workgroup, at most 16 a CU
-int level_grid(int count, int per, int cus) { return std::max(1, std::min((count + per - 1) / per, std::max(1, cus) * 16)); }
-
 template <class R, int L>
-void forward_levels(const SoftArgs& a, const SoftLevels& lv, int kind, int cus, hipStream_t st) {
-    for (int h = 0; h + 1 < int(lv.start.size()); ++h) {
-        const int count = lv.start[h + 1] - lv.start[h];
-        if (!count) continue;
-        const int4* order = lv.order + lv.start[h];
-        const dim3 grid(level_grid(count, 256 / kWave * kNodesPerWave<L>, cus));
-        if (kind) {
-            hipLaunchKernelGGL((soft_forward_level_kernel<R, L, 1>), grid, dim3(256), 0, st, a, order, count);
-            hipLaunchKernelGGL((soft_zedge_level_kernel<R, L>), dim3(level_grid(count, 256 / kZGroup, cus)), dim3(256), 0,
-                               st, a, order, count);
-        } else {
-            hipLaunchKernelGGL((soft_forward_level_kernel<R, L, 0>), grid, dim3(256), 0, st, a, order, count);
-        }
-    }
+void forward_chunks(const SoftArgs& a, const SoftLevels& lv, int kind, hipStream_t st) {
+    const dim3 grid((a.count + lv.chunk - 1) / lv.chunk);
+    if (kind) hipLaunchKernelGGL((soft_forward_chunk_kernel<R, L, 1>), grid, dim3(256), 0, st, a, lv);
+    else hipLaunchKernelGGL((soft_forward_chunk_kernel<R, L, 0>), grid, dim3(256), 0, st, a, lv);
+}
+template <class R, int L>
+void backward_chunks(const SoftArgs& a, const SoftLevels& lv, int kind, hipStream_t st) {
+    const dim3 grid((a.count + lv.chunk - 1) / lv.chunk);
+    if (kind) hipLaunchKernelGGL((soft_backward_chunk_kernel<R, L, 1>), grid, dim3(256), 0, st, a, lv);
+    else hipLaunchKernelGGL((soft_backward_chunk_kernel<R, L, 0>), grid, dim3(256), 0, st, a, lv);
 }
 }  // namespace
 
-void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, int cus, hipStream_t st) {
+void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, hipStream_t st) {
     switch (a.g.L) {
 #define GR_SOFT_CASE(n)                                                        \
     case n:                                                                    \
-        if (precision == 64) forward_levels<double, n>(a, lv, kind, cus, st);  \
-        else forward_levels<float, n>(a, lv, kind, cus, st);                   \
+        if (precision == 64) forward_chunks<double, n>(a, lv, kind, st);  \
+        else forward_chunks<float, n>(a, lv, kind, st);                   \
         break;
         GR_SOFT_CASE(1) GR_SOFT_CASE(2) GR_SOFT_CASE(3) GR_SOFT_CASE(4) GR_SOFT_CASE(5)
         GR_SOFT_CASE(6) GR_SOFT_CASE(7) GR_SOFT_CASE(8) GR_SOFT_CASE(9) GR_SOFT_CASE(10)
@@ -1083,14 +1114,17 @@ void launch_soft_forward(const SoftArgs& a, const SoftLevels& lv, int precision,
     }
 }
 
-void launch_soft_backward(const SoftArgs& a, int precision, int kind, int cus, hipStream_t st) {
-    const dim3 grid(soft_grid(a, cus));
-    if (precision == 64) {
-        if (kind) hipLaunchKernelGGL((soft_backward_kernel<double, 1>), grid, dim3(kWave), 0, st, a);
-        else hipLaunchKernelGGL((soft_backward_kernel<double, 0>), grid, dim3(kWave), 0, st, a);
-    } else {
-        if (kind) hipLaunchKernelGGL((soft_backward_kernel<float, 1>), grid, dim3(kWave), 0, st, a);
-        else hipLaunchKernelGGL((soft_backward_kernel<float, 0>), grid, dim3(kWave), 0, st, a);
+void launch_soft_backward(const SoftArgs& a, const SoftLevels& lv, int precision, int kind, hipStream_t st) {
+    switch (a.g.L) {
+#define GR_SOFT_CASE(n)                                                         \
+    case n:                                                                     \
+        if (precision == 64) backward_chunks<double, n>(a, lv, kind, st);  \
+        else backward_chunks<float, n>(a, lv, kind, st);                   \
+        break;
+        GR_SOFT_CASE(1) GR_SOFT_CASE(2) GR_SOFT_CASE(3) GR_SOFT_CASE(4) GR_SOFT_CASE(5)
+        GR_SOFT_CASE(6) GR_SOFT_CASE(7) GR_SOFT_CASE(8) GR_SOFT_CASE(9) GR_SOFT_CASE(10)
+#undef GR_SOFT_CASE
+        default: break;
     }
 }
 

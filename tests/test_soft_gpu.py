@@ -154,3 +154,63 @@ def test_soft_dag_cost_gradients_match_finite_differences(ga, ora, kind):
         unused = np.flatnonzero(grad == 0)
         assert len(unused) > 0
     ctx.close()
+
+
+def _soft_trees(rng, L, X, Y):
+    """Trees with long, short, straight and zero-length edges, every node
+    degree, and one chain taller than 256 levels: (node_off, nodes, parents)."""
+    off, nodes, parents = [0], [], []
+    for n in (1, 2, 2, 3, 7, 20, 300):
+        par = [-1] + [i - 1 if n == 300 else int(rng.integers(0, i)) for i in range(1, n)]
+        x, y = rng.integers(0, X, n), rng.integers(0, Y, n)
+        if n == 300:  # short steps, so that the oracle's Z-shape edges stay small
+            x, y = np.arange(n) % 3 % X, np.arange(n) // 2 % Y
+        x[1:][rng.random(n - 1) < 0.2] = x[0]
+        if n > 3:
+            x[2], y[2] = x[par[2]], y[par[2]]
+        if n == 2:
+            x[:], y[:] = (0, X - 1), (Y - 1, 0)  # the whole grid, falling
+        layer = np.where(rng.random(n) < 0.5, L, rng.integers(0, L, n))
+        nodes += ((layer * X + x) * Y + y).tolist()
+        parents += par
+        off.append(len(nodes))
+    return np.array(off, np.int32), np.array(nodes, np.int32), np.array(parents, np.int32)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("L,X,Y", [(1, 5, 9), (2, 3, 40), (5, 37, 20), (9, 20, 70), (10, 18, 17)])
+def test_soft_trees_of_every_form_match_oracle(ga, ora, L, X, Y, kind):
+    """Every lane count (L lanes per node: 64, 32, 12, 7 and 6 nodes per
+    wavefront), edges of more bends than the 16 lanes of an edge, a slot range
+    that does not start at 0, given costs of either sign: FP64 equal to the
+    oracle as on the generated instance above."""
+    rng = np.random.default_rng(1000 * L + X)
+    off, nodes, parents = _soft_trees(rng, L, X, Y)
+    t = dict(L=L, X=X, Y=Y, DIR=L & 1, unit_length_wire_cost=0.01, unit_via_cost=0.5,
+             unit_length_short_costs=np.full(L, 0.3), x_edge_len=np.full(X - 1, 30, np.int32),
+             y_edge_len=np.full(Y - 1, 30, np.int32), capacity=rng.integers(0, 6, L * X * Y).astype(np.float32))
+    n = len(off) - 1
+    ctx = ga.Context(t)
+    ctx.set_routes(off)
+    ctx.lshape_upload(np.arange(n), off, nodes, parents)
+    demand = random_demand(t, 3, high=4)
+    ctx.upload_demand(demand)
+    ctx.set_soft_kind(kind)
+    grid = ora.Grid(t)
+    print(f"soft trees L={L} {X}x{Y} kind={kind}", flush=True)
+    for begin in (0, 2):
+        o = off[begin:] - off[begin]
+        F_o, gw_o, gv_o, gp_o = grid.soft_stage(demand, o, nodes[off[begin]:], parents[off[begin]:], 1.0, *THETA,
+                                                grads=True, kind=kind)
+        total, _, _ = ctx.soft_forward(begin, n - begin, *THETA, tau=1.0, precision=64)
+        gp, _ = ctx.soft_backward()
+        gw, gv = ctx.soft_edge_grads()
+        assert abs(total - F_o) <= 1e-10 * abs(F_o)
+        assert np.allclose(gw, gw_o, rtol=1e-8, atol=1e-10) and np.allclose(gv, gv_o, rtol=1e-8, atol=1e-10)
+        assert np.allclose(gp, gp_o, rtol=1e-8, atol=1e-10)
+    w, v = rng.normal(0.3, 0.5, L * X * Y), rng.normal(0.5, 0.5, L * X * Y)
+    want = sum(np.array(grid.soft_net(w, v, nodes[off[k]:off[k + 1]], parents[off[k]:off[k + 1]], 0.5, kind=kind))
+               for k in range(n))
+    total, _, _ = ctx.soft_forward_costs(0, n, w, v, 0.5, 64)
+    assert abs(total - want) <= 1e-10 * max(1.0, abs(want))
+    ctx.close()
