@@ -166,6 +166,9 @@ struct gr_ctx {
     size_t gscratch_bytes = 0;
     double* noalloc_scratch = nullptr;    // this device's `scratch` (gr_lshape_batch_noalloc)
     std::vector<int> noalloc_slots;       // sized at gr_lshape_upload
+    // grid arrays on their way between IDX and track-major order, and the
+    // recomputed costs of gr_cost_download
+    Workspace layout_ws, cost_ws;
     // rip-up
     int* of_sum = nullptr;
     unsigned char* of_flags = nullptr;
@@ -353,19 +356,86 @@ void download(void* dst, const void* src, size_t bytes, hipStream_t s) {
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 
-// IDX order <-> track-major order (host side, one pass)
+// Grids of fewer cells change their order on the host: the extra launch and
+// its wait for the copy cost more there (a demand upload and download of 16k
+// cells 41 us on the host, 62 on the device; 32k 48 and 66, but the two cost
+// arrays and gradients of the soft DP 175 and 186; 65k 137 and 75; 262k 577 and
+// 150).
+constexpr size_t kHostLayoutCells = 32768;
+
+// IDX order <-> track-major order on the host, one pass.
 template <class T>
-void to_track_major(const DeviceGrid& g, const T* src, std::vector<T>& dst) {
-    dst.resize(size_t(g.L) * g.XY);
+void host_to_track_major(const DeviceGrid& g, const T* src, T* dst) {
     for (int l = 0; l < g.L; ++l)
         for (int x = 0; x < g.X; ++x)
             for (int y = 0; y < g.Y; ++y) dst[cell_of(g, l, x, y)] = src[(size_t(l) * g.X + x) * g.Y + y];
 }
 template <class T>
-void from_track_major(const DeviceGrid& g, const std::vector<T>& src, T* dst) {
+void host_from_track_major(const DeviceGrid& g, const T* src, T* dst) {
     for (int l = 0; l < g.L; ++l)
         for (int x = 0; x < g.X; ++x)
             for (int y = 0; y < g.Y; ++y) dst[(size_t(l) * g.X + x) * g.Y + y] = src[cell_of(g, l, x, y)];
+}
+
+// Up to two grid arrays of the ABI (IDX order, host) into track-major device
+// arrays and back, through the context's layout buffer, in one layout launch;
+// a null host pointer skips its array.  An upload may still be enqueued on
+// return: the caller waits for the stream before the host arrays may go.
+template <class T>
+void upload_grids(gr_ctx* c, T* dst0, const T* src0, T* dst1 = nullptr, const T* src1 = nullptr) {
+    if (c->cells < kHostLayoutCells) {
+        std::vector<T> h(c->cells);
+        for (auto [dst, src] : {std::pair<T*, const T*>{dst0, src0}, {dst1, src1}}) {
+            if (!src) continue;
+            host_to_track_major(c->g, src, h.data());
+            upload(dst, h.data(), sizeof(T) * c->cells, c->stream);
+            hip_check(hipStreamSynchronize(c->stream), "grid upload");
+        }
+        return;
+    }
+    T* tmp = nullptr;
+    c->layout_ws.carve([&](auto& cv) { tmp = cv.template take<T>(c->cells * (src1 ? 2 : 1)); });
+    LayoutArrays<T> a{};
+    for (auto [dst, src] : {std::pair<T*, const T*>{dst0, src0}, {dst1, src1}}) {
+        if (!src) continue;
+        upload(tmp, src, sizeof(T) * c->cells, c->stream);
+        a.src[a.count] = tmp, a.dst[a.count++] = dst;
+        tmp += c->cells;
+    }
+    launch_layout(c->g, a, true, c->stream);
+    hip_check(hipGetLastError(), "layout kernel");
+}
+template <class T>
+void download_grids(gr_ctx* c, const T* src0, T* dst0, const T* src1 = nullptr, T* dst1 = nullptr) {
+    if (c->cells < kHostLayoutCells) {
+        std::vector<T> h(c->cells);
+        for (auto [src, dst] : {std::pair<const T*, T*>{src0, dst0}, {src1, dst1}}) {
+            if (!dst) continue;
+            download(h.data(), src, sizeof(T) * c->cells, c->stream);
+            host_from_track_major(c->g, h.data(), dst);
+        }
+        return;
+    }
+    T* tmp = nullptr;
+    c->layout_ws.carve([&](auto& cv) { tmp = cv.template take<T>(c->cells * (dst1 ? 2 : 1)); });
+    LayoutArrays<T> a{};
+    T* host[2];
+    for (auto [src, dst] : {std::pair<const T*, T*>{src0, dst0}, {src1, dst1}}) {
+        if (!dst) continue;
+        host[a.count] = dst;
+        a.src[a.count] = src, a.dst[a.count++] = tmp;
+        tmp += c->cells;
+    }
+    launch_layout(c->g, a, false, c->stream);
+    hip_check(hipGetLastError(), "layout kernel");
+    for (int k = 0; k < a.count; ++k) download(host[k], a.dst[k], sizeof(T) * c->cells, c->stream);
+}
+
+// Every track marked for the next refresh.
+void mark_tracks(gr_ctx* c) {
+    hipLaunchKernelGGL(fill_int_kernel, dim3((c->tracks + 255) / 256), dim3(256), 0, c->stream, (int*)c->track_dirty, 1,
+                       (long long)c->tracks);
+    hip_check(hipGetLastError(), "mark tracks");
 }
 
 Stats read_stats(gr_ctx* c) {
@@ -1132,13 +1202,7 @@ void soft_forward(gr_ctx* c, int begin, int count, double slope, double zero_slo
     sc.via_weight = via_weight;
     const bool given = wcost != nullptr;
     if (given) {
-        std::vector<double> h;
-        to_track_major(c->g, wcost, h);
-        upload(sc.wcost, h.data(), sizeof(double) * cells, c->stream);
-        hip_check(hipStreamSynchronize(c->stream), "soft cost upload");
-        to_track_major(c->g, vcost, h);
-        upload(sc.vcost, h.data(), sizeof(double) * cells, c->stream);
-        hip_check(hipStreamSynchronize(c->stream), "soft cost upload");
+        upload_grids<double>(c, sc.wcost, wcost, sc.vcost, vcost);
     }
     a.g = c->g;
     a.presum = sc.presum;
@@ -1249,15 +1313,12 @@ int gr_ctx_create(const gr_grid_desc* grid, gr_ctx** out) {
         c->refreshed = c->mem.alloc<unsigned long long>(kStatStripes * kCounterStride);
         hip_check(hipMemsetAsync(c->refreshed, 0, sizeof(unsigned long long) * kStatStripes * kCounterStride, c->stream),
                   "clear counter");
-        std::vector<float> cap;
-        to_track_major(g, grid->capacity, cap);
-        upload(c->capacity, cap.data(), sizeof(float) * c->cells, c->stream);
+        upload_grids<float>(c.get(), c->capacity, grid->capacity);
         hip_check(hipMemsetAsync(c->demand, 0, sizeof(float) * c->cells, c->stream), "clear demand");
         hip_check(hipMemsetAsync(c->timestamp, 0, sizeof(int) * c->cells, c->stream), "clear timestamps");
         hip_check(hipMemsetAsync(c->stats, 0, sizeof(Stats) * kStatStripes, c->stream), "clear statistics");
         hip_check(hipMemsetAsync(c->error, 0, sizeof(int), c->stream), "clear error");
-        std::vector<unsigned> ones(c->tracks, 1u);
-        upload(c->track_dirty, ones.data(), sizeof(unsigned) * c->tracks, c->stream);
+        mark_tracks(c.get());
         hip_check(hipStreamSynchronize(c->stream), "context setup");
         *out = c.release();
     });
@@ -1305,8 +1366,7 @@ int gr_ctx_set_cost_params(gr_ctx* c, double slope, double zero_slope, double vi
         c->cp.zero_slope = zero_slope;
         c->cp.via_weight = via_weight;
         c->cp.integer_wire = integer_wire ? 1 : 0;
-        std::vector<unsigned> ones(c->tracks, 1u);
-        upload(c->track_dirty, ones.data(), sizeof(unsigned) * c->tracks, c->stream);
+        mark_tracks(c);
         hip_check(hipStreamSynchronize(c->stream), "cost parameters");
     });
 }
@@ -1330,44 +1390,35 @@ int gr_cost_refresh_full(gr_ctx* c) {
 int gr_cost_download(gr_ctx* c, float* wcost, float* vcost, double* presum) {
     return guarded([&] {
         if (!c) throw GrError(GR_E_ARG, "null context");
+        float* tmp = nullptr;
         if (wcost) {
             // wcost is not kept resident: recompute it from the current demand
             // with the refresh kernel into temporaries, leaving the resident
             // costs and dirty flags untouched
-            DeviceArena scratch;
-            float* tmp = scratch.alloc<float>(c->cells);
-            float* tv = scratch.alloc<float>(c->cells);
-            double* tp = scratch.alloc<double>(c->cells);
-            unsigned* td = scratch.alloc<unsigned>(c->tracks);
+            float* tv = nullptr;
+            double* tp = nullptr;
+            unsigned* td = nullptr;
+            c->cost_ws.carve([&](auto& cv) {
+                tmp = cv.template take<float>(c->cells);
+                tv = cv.template take<float>(c->cells);
+                tp = cv.template take<double>(c->cells);
+                td = cv.template take<unsigned>(c->tracks);
+            });
             hipLaunchKernelGGL(refresh_tracks_kernel, dim3(c->tracks), dim3(kRefreshThreads),
                                size_t(c->maxlen) * sizeof(double), c->stream, c->g, c->capacity, c->demand, tv, tp,
                                tmp, td, 1, c->cp, (unsigned long long*)nullptr);
             hip_check(hipGetLastError(), "refresh for wcost");
-            std::vector<float> h(c->cells);
-            download(h.data(), tmp, sizeof(float) * c->cells, c->stream);
-            from_track_major(c->g, h, wcost);
         }
-        if (vcost) {
-            std::vector<float> h(c->cells);
-            download(h.data(), c->vcost, sizeof(float) * c->cells, c->stream);
-            from_track_major(c->g, h, vcost);
-        }
-        if (presum) {
-            std::vector<double> h(c->cells);
-            download(h.data(), c->presum, sizeof(double) * c->cells, c->stream);
-            from_track_major(c->g, h, presum);
-        }
+        if (wcost || vcost) download_grids<float>(c, tmp, wcost, c->vcost, vcost);
+        if (presum) download_grids<double>(c, c->presum, presum);
     });
 }
 
 int gr_demand_upload(gr_ctx* c, const float* demand) {
     return guarded([&] {
         if (!c || !demand) throw GrError(GR_E_ARG, "null argument");
-        std::vector<float> h;
-        to_track_major(c->g, demand, h);
-        upload(c->demand, h.data(), sizeof(float) * c->cells, c->stream);
-        std::vector<unsigned> ones(c->tracks, 1u);
-        upload(c->track_dirty, ones.data(), sizeof(unsigned) * c->tracks, c->stream);
+        mark_tracks(c);
+        upload_grids<float>(c, c->demand, demand);
         hip_check(hipStreamSynchronize(c->stream), "demand upload");
     });
 }
@@ -1375,18 +1426,14 @@ int gr_demand_upload(gr_ctx* c, const float* demand) {
 int gr_demand_download(gr_ctx* c, float* demand) {
     return guarded([&] {
         if (!c || !demand) throw GrError(GR_E_ARG, "null argument");
-        std::vector<float> h(c->cells);
-        download(h.data(), c->demand, sizeof(float) * c->cells, c->stream);
-        from_track_major(c->g, h, demand);
+        download_grids<float>(c, c->demand, demand);
     });
 }
 
 int gr_timestamp_download(gr_ctx* c, int* ts) {
     return guarded([&] {
         if (!c || !ts) throw GrError(GR_E_ARG, "null argument");
-        std::vector<int> h(c->cells);
-        download(h.data(), c->timestamp, sizeof(int) * c->cells, c->stream);
-        from_track_major(c->g, h, ts);
+        download_grids<int>(c, c->timestamp, ts);
     });
 }
 
@@ -1844,8 +1891,7 @@ int gr_ctx_reset(gr_ctx* c) {
             hip_check(hipMemsetAsync(c->routes, 0, sizeof(int) * size_t(c->route_words), c->stream), "clear routes");
         // a fresh context has no phase-two storage (it belongs to an FLT stage)
         c->release_phase2();
-        std::vector<unsigned> ones(c->tracks, 1u);
-        upload(c->track_dirty, ones.data(), sizeof(unsigned) * c->tracks, c->stream);
+        mark_tracks(c);
         hip_check(hipStreamSynchronize(c->stream), "gr_ctx_reset");
     });
 }
@@ -2691,12 +2737,7 @@ int gr_soft_edge_grads(gr_ctx* c, double* grad_wcost, double* grad_vcost) {
     return guarded([&] {
         if (!c) throw GrError(GR_E_ARG, "null context");
         if (!c->soft_ready) throw GrError(GR_E_STATE, "no soft pass");
-        for (auto [dst, src] : {std::pair<double*, double*>{grad_wcost, c->soft.gw}, {grad_vcost, c->soft.gv}}) {
-            if (!dst) continue;
-            std::vector<double> h(c->cells);
-            download(h.data(), src, sizeof(double) * c->cells, c->stream);
-            from_track_major(c->g, h, dst);
-        }
+        download_grids<double>(c, c->soft.gw, grad_wcost, c->soft.gv, grad_vcost);
     });
 }
 
