@@ -50,6 +50,35 @@ struct DeviceArena {
     }
 };
 
+// Device blocks kept from one call for the next: the k-th alloc of a call
+// takes the k-th block, replaced when it is too small.
+struct ReuseArena {
+    std::vector<std::pair<void*, size_t>> blocks;
+    size_t at = 0;
+    ReuseArena() = default;
+    ReuseArena(const ReuseArena&) = delete;
+    ReuseArena& operator=(const ReuseArena&) = delete;
+    void begin() { at = 0; }
+    template <class T>
+    T* alloc(size_t count) {
+        const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+        if (at == blocks.size()) blocks.push_back({nullptr, 0});
+        auto& [p, cap] = blocks[at++];
+        if (bytes > cap) {
+            if (p) (void)hipFree(p);
+            p = nullptr;
+            cap = 0;
+            hip_check(hipMalloc(&p, bytes), "hipMalloc");
+            cap = bytes;
+        }
+        return static_cast<T*>(p);
+    }
+    ~ReuseArena() {
+        for (auto& [p, cap] : blocks)
+            if (p) (void)hipFree(p);
+    }
+};
+
 // Sequential aligned sub-buffers of a base pointer (sizes only when base is null).
 struct Carver {
     char* base;
@@ -166,6 +195,7 @@ struct gr_ctx {
     size_t gscratch_bytes = 0;
     double* noalloc_scratch = nullptr;    // this device's `scratch` (gr_lshape_batch_noalloc)
     std::vector<int> noalloc_slots;       // sized at gr_lshape_upload
+    ReuseArena score_mem;  // gr_score: lines, per-cell counters, partial sums
     // grid arrays on their way between IDX and track-major order, and the
     // recomputed costs of gr_cost_download
     Workspace layout_ws, cost_ws;
@@ -995,7 +1025,8 @@ void bind_flt_storage(gr_ctx* c) {
 // The per-net line inputs of the evaluator score and connectivity check,
 // checked and uploaded into `ar`: every index the kernels derive from them
 // is validated here.
-ScoreArgs net_lines(gr_ctx* c, DeviceArena& ar, int nets, const int* pin_off, const int* pins, const int* extra_off,
+template <class Arena>
+ScoreArgs net_lines(gr_ctx* c, Arena& ar, int nets, const int* pin_off, const int* pins, const int* extra_off,
                     const int* extra, const int* sub_off, const int* subs, const int* layer_dir) {
     if (nets < 0 || !pin_off || !extra_off || !sub_off || !layer_dir) throw GrError(GR_E_ARG, "null argument");
     if (!c->routes) throw GrError(GR_E_STATE, "routes not allocated (gr_ctx_set_routes)");
@@ -1022,13 +1053,13 @@ ScoreArgs net_lines(gr_ctx* c, DeviceArena& ar, int nets, const int* pin_off, co
         if (layer_dir[z] != 0 && layer_dir[z] != 1) throw GrError(GR_E_ARG, "layer direction must be 0 or 1");
     ScoreArgs a{};
     a.nets = nets, a.X = X, a.Y = Y, a.M = M;
-    int* d_pin_off = ar.alloc<int>(nets + 1);
-    int* d_pins = ar.alloc<int>(np);
-    int* d_extra_off = ar.alloc<int>(nets + 1);
-    int* d_extra = ar.alloc<int>(ne);
-    int* d_sub_off = ar.alloc<int>(nets + 1);
-    int* d_subs = ar.alloc<int>(ns);
-    int* d_dir = ar.alloc<int>(M);
+    int* d_pin_off = ar.template alloc<int>(nets + 1);
+    int* d_pins = ar.template alloc<int>(np);
+    int* d_extra_off = ar.template alloc<int>(nets + 1);
+    int* d_extra = ar.template alloc<int>(ne);
+    int* d_sub_off = ar.template alloc<int>(nets + 1);
+    int* d_subs = ar.template alloc<int>(ns);
+    int* d_dir = ar.template alloc<int>(M);
     hipStream_t st = c->stream;
     upload(d_pin_off, pin_off, sizeof(int) * (nets + 1), st);
     if (np) upload(d_pins, pins, sizeof(int) * np, st);
@@ -1733,9 +1764,7 @@ int gr_lshape_tune(gr_ctx* c, int nbatch, const int* batch_off, int* per_wave, d
         launch_refresh(c, 0);
         const bool profiling = c->profiling;
         c->profiling = false;
-        hipEvent_t e0, e1;
-        hip_check(hipEventCreate(&e0), "hipEventCreate");
-        hip_check(hipEventCreate(&e1), "hipEventCreate");
+        hipEvent_t e0 = take_event(c), e1 = take_event(c);
         const int candidates[4] = {1, 2, 4, 8};
         for (int k = 0; k < kTreeClasses; ++k) {
             int nmax = 1;
@@ -1768,8 +1797,7 @@ int gr_lshape_tune(gr_ctx* c, int nbatch, const int* batch_off, int* per_wave, d
             c->per_wave[k] = choice;
             if (per_wave) per_wave[k] = choice;
         }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        c->next_event -= 2;
         c->profiling = profiling;
         c->drop_graph();
         check_device_error(c, "gr_lshape_tune");
@@ -2615,9 +2643,7 @@ int gr_flt_tune(gr_ctx* c, int* per_wave, double* ms) {
         launch_refresh(c, 0);
         const bool profiling = c->profiling;
         c->profiling = false;
-        hipEvent_t e0, e1;
-        hip_check(hipEventCreate(&e0), "hipEventCreate");
-        hip_check(hipEventCreate(&e1), "hipEventCreate");
+        hipEvent_t e0 = take_event(c), e1 = take_event(c);
         const int candidates[4] = {1, 2, 4, 8};
         double t[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
         bool seen[2] = {false, false};
@@ -2648,8 +2674,7 @@ int gr_flt_tune(gr_ctx* c, int* per_wave, double* ms) {
                   "restore phase-two routes");
         hip_check(hipStreamSynchronize(c->stream), "FLT tuning");
         c->mem.release(saved);
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        c->next_event -= 2;
         c->profiling = profiling;
         for (int cls = 0; cls < 2; ++cls) {
             int best = 0;
@@ -3028,7 +3053,8 @@ int gr_score(gr_ctx* c, int nets, const int* pin_off, const int* pins, const int
              const double* overflow_cost, double* out, unsigned short* demand) {
     return guarded([&] {
         if (!c || !capacity || !overflow_cost || !out) throw GrError(GR_E_ARG, "null argument");
-        DeviceArena ar;
+        ReuseArena& ar = c->score_mem;
+        ar.begin();
         ScoreArgs a = net_lines(c, ar, nets, pin_off, pins, extra_off, extra, sub_off, subs, layer_dir);
         const int X = c->g.X, Y = c->g.Y, M = c->g.L + 1;
         const long long XY = (long long)X * Y, cells = XY * M;
@@ -3036,25 +3062,28 @@ int gr_score(gr_ctx* c, int nets, const int* pin_off, const int* pins, const int
         double* d_cap = ar.alloc<double>(cells);
         int* d_wire = ar.alloc<int>(cells);
         int* d_stacked = ar.alloc<int>(cells);
-        const int ncount = kStatStripes * kScoreLayers + 1;  // striped via counters, rejected nets
+        const int ncount = kStatStripes * kScoreLayers + 2;  // striped via counters, rejected nets, big nets
         unsigned long long* d_counts = ar.alloc<unsigned long long>(ncount);
+        a.big = ar.alloc<int>(nets);
         double* d_ploss = ar.alloc<double>(size_t(M) * blocks_per_layer);
         unsigned long long* d_pwl = ar.alloc<unsigned long long>(size_t(M) * blocks_per_layer);
         unsigned short* d_demand = demand ? ar.alloc<unsigned short>(cells) : nullptr;
         hipStream_t st = c->stream;
         upload(d_cap, capacity, sizeof(double) * cells, st);
-        a.wire = d_wire, a.stacked = d_stacked, a.vias = d_counts, a.bad_nets = d_counts + ncount - 1;
-        hipEvent_t e0, e1;
-        hip_check(hipEventCreate(&e0), "hipEventCreate");
-        hip_check(hipEventCreate(&e1), "hipEventCreate");
+        a.wire = d_wire, a.stacked = d_stacked, a.vias = d_counts, a.bad_nets = d_counts + ncount - 2;
+        a.big_count = reinterpret_cast<int*>(d_counts + ncount - 1);
+        hipEvent_t e0 = take_event(c), e1 = take_event(c);
         hip_check(hipEventRecord(e0, st), "hipEventRecord");
         hipLaunchKernelGGL(fill_int_kernel, dim3(int(std::min<long long>(4096, (cells + 255) / 256))), dim3(256), 0, st,
                            d_wire, 0, cells);
         hipLaunchKernelGGL(fill_int_kernel, dim3(int(std::min<long long>(4096, (cells + 255) / 256))), dim3(256), 0, st,
                            d_stacked, 0, cells);
         hipLaunchKernelGGL(fill_int_kernel, dim3(16), dim3(256), 0, st, (int*)d_counts, 0, 2LL * ncount);
-        if (nets)
-            hipLaunchKernelGGL(score_nets_kernel, dim3(std::min(nets, std::max(1, c->cus) * 16)), dim3(kWave), 0, st, a);
+        if (nets) {
+            const int cus = std::max(1, c->cus);
+            hipLaunchKernelGGL(score_nets_kernel, dim3(std::min((nets + 3) / 4, cus * 8)), dim3(256), 0, st, a);
+            hipLaunchKernelGGL(score_big_kernel, dim3(std::min(nets, cus * 7)), dim3(kWave), 0, st, a);
+        }
         hipLaunchKernelGGL(score_cells_kernel, dim3(blocks_per_layer, M), dim3(256), 0, st, a, d_cap, c->g.x_edge_len,
                            c->g.y_edge_len, d_ploss, d_pwl, d_demand);
         hip_check(hipEventRecord(e1, st), "hipEventRecord");
@@ -3067,8 +3096,7 @@ int gr_score(gr_ctx* c, int nets, const int* pin_off, const int* pins, const int
         if (demand) download(demand, d_demand, sizeof(unsigned short) * cells, st);
         float ms = 0.f;
         hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        c->next_event -= 2;
         // resources/evaluator.cpp:575-623, every layer routable (CAP
         // directions are 0 or 1)
         double wl_cost = 0, via_cost = 0, overflow = 0;
@@ -3089,7 +3117,7 @@ int gr_score(gr_ctx* c, int nets, const int* pin_off, const int* pins, const int
         out[1] = via_cost;
         out[2] = overflow;
         out[3] = overflow + via_cost + wl_cost;
-        out[4] = double(counts[ncount - 1]);
+        out[4] = double(counts[ncount - 2]);
         out[5] = double(ms);
     });
 }

@@ -352,11 +352,14 @@ struct ScoreArgs {
     int* stacked;                   // [M * X * Y] stacked-via demand per cell
     unsigned long long* vias;       // [kStatStripes * kScoreLayers] via layer-steps per stripe and layer
     unsigned long long* bad_nets;   // nets with a line the evaluator rejects
+    int *big, *big_count;           // score: nets of more than kScoreSmall lines, and how many
 };
 constexpr int kScoreCells = 8192;  // cells per score_cells_kernel block
-constexpr int kScoreLines = 1024;  // lines of a net staged in LDS by score_nets_kernel
+constexpr int kScoreSmall = 128;   // lines of a net staged in LDS by score_nets_kernel
+constexpr int kScoreLines = 1024;  // lines of a net staged in LDS by score_big_kernel and connectivity_kernel
 constexpr int kScoreLayers = 32;   // metal layers the score supports (via counters per stripe)
 __global__ void score_nets_kernel(ScoreArgs a);
+__global__ void score_big_kernel(ScoreArgs a);
 
 // The evaluator's completion test per net (resources/evaluator.cpp:527-538,
 // check_connectivity :677-749) over the same lines as the score.

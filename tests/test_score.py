@@ -498,3 +498,42 @@ def test_gpu_connectivity_matches_oracle(ga, ora, tmp_path):
                             routes2=ctx.routes2(), pin_off2=fs["pin_off2"])
     assert np.array_equal(st, want) and counts["incomplete"] == 0
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [(1, 2, 127), (128, 129, 300), (1023, 1024, 1025)])
+def test_gpu_score_line_counts_match_oracle(ga, ora, counts):
+    """Nets of line counts around the 128 lines staged per wavefront and the
+    1,024 staged per workgroup, on a few tracks so that many wires, vias and
+    places share a chain: demand, costs and rejected nets against the oracle."""
+    d, t = topology(6, 0)
+    mg = d.metal_grid()
+    M, X, Y = mg["layers"], int(t["X"]), int(t["Y"])
+    rng = np.random.default_rng(counts[0])
+    print(f"score line counts {counts}", flush=True)
+    off, extra = [0], []
+    for n in counts:
+        for _ in range(n):
+            x, y, z = int(rng.integers(0, 6)), int(rng.integers(0, 6)), int(rng.integers(0, M))
+            if rng.random() < 0.5:  # a via column, now and then one that moves
+                x2, y2, z2 = x + int(rng.random() < 0.01), y, int(rng.integers(0, M))
+            else:  # a wire, some against their layer's direction, some empty
+                step, along_y = int(rng.integers(0, 5)), bool(mg["dir"][z]) != (rng.random() < 0.01)
+                x2, y2, z2 = x + (0 if along_y else step), y + (step if along_y else 0), z
+            extra += [(z * X + x) * Y + y, (z2 * X + x2) * Y + y2]
+        off.append(len(extra))
+    zero = np.zeros(len(counts) + 1, np.int32)
+    lines = dict(pin_off=zero, pins=np.zeros(0, np.int32), extra_off=np.array(off, np.int32),
+                 extra=np.array(extra, np.int32), sub_off=zero, subs=np.zeros(0, np.int32))
+    cap = np.asarray(mg["capacity"], np.float64)
+    ctx = ga.Context(t)
+    ctx.set_routes(t["pin_acc_num"])
+    for _ in range(2):  # the second call runs in the first one's buffers
+        got = ctx.score(lines, mg["dir"], cap, mg["overflow_cost"], demand=True)
+        want = ora.score(X, Y, M, lines, ctx.routes(), t["pin_acc_num"], 12, mg["dir"], cap, mg["overflow_cost"],
+                         t["x_edge_len"], t["y_edge_len"], t["unit_length_wire_cost"], t["unit_via_cost"])
+        assert np.array_equal(got["demand"], want["demand"])
+        assert got["rejected"] == want["rejected"]
+        assert got["wirelength"] == want["wirelength"] and got["via"] == want["via"]
+        assert got["overflow"] == pytest.approx(want["overflow"], rel=1e-10)
+    ctx.close()
