@@ -149,6 +149,20 @@ double* noalloc_scratch_address() {
 
 }  // namespace
 
+namespace {
+// One batch's L-shape DP launches: its slots by tree size class
+struct BatchLaunch {
+    int begin;
+    int count[kTreeClasses];
+    int nmax[kTreeClasses];
+    // plan_batch: the last `tiny` slots of class 0 are its trees of at most
+    // tiny_bound nodes (the persistent form drains them from a queue of their
+    // own, with tables sized for them)
+    int tiny = 0;
+    int tiny_nmax = 1;
+};
+}  // namespace
+
 struct gr_ctx {
     DeviceArena mem;
     hipStream_t stream = nullptr;
@@ -191,6 +205,11 @@ struct gr_ctx {
     std::vector<int> slots_h;      // stage slot per execution position
     int4* desc = nullptr;          // per execution position: node begin, nodes, route word, route capacity
     std::vector<int4> desc_h;
+    // the last gr_lshape_run's launches, slots_h and descriptors, kept while
+    // what they are made of stays the same (contents, not addresses)
+    std::vector<BatchLaunch> run_plan;
+    std::vector<int> run_plan_key;
+    int routes_gen = 0;  // counts the route stores
     double* gscratch = nullptr;
     size_t gscratch_bytes = 0;
     double* noalloc_scratch = nullptr;    // this device's `scratch` (gr_lshape_batch_noalloc)
@@ -569,50 +588,38 @@ void launch_commit(gr_ctx* c, int begin, int count, int stamp, int K, const int*
 // more in launch and tail time than the smaller tables save.)
 constexpr int kClassNodes[kTreeClasses - 1] = {kSmallTree};
 
-struct BatchLaunch {
-    int begin;
-    int count[kTreeClasses];
-    int nmax[kTreeClasses];
-    // plan_batch: the last `tiny` slots of class 0 are its trees of at most
-    // tiny_bound nodes (the persistent form drains them from a queue of their
-    // own, with tables sized for them)
-    int tiny = 0;
-    int tiny_nmax = 1;
-};
-
 int tree_class(int n) {
     int k = 0;
     while (k < kTreeClasses - 1 && n > kClassNodes[k]) ++k;
     return k;
 }
 
+// The launches of one batch, its slots in slots[begin, begin + count): the
+// small class's trees above tiny_bound nodes, its tiny trees, the large class,
+// each with the tallest trees first (the nets with the longest level chains
+// start first and the launch's tail is short) and in stage order among equal
+// heights.  One counting pass and one placing pass over (group, height).
 BatchLaunch plan_batch(gr_ctx* c, int begin, int count, std::vector<int>& slots) {
     BatchLaunch b{begin, {0, 0}, {1, 1}};
+    int H = 0;
+    for (int s = begin; s < begin + count; ++s) H = std::max(H, c->height_h[s]);
+    auto bucket = [&](int s, int n) {
+        const int g = tree_class(n) ? 2 : n <= c->tiny_bound ? 1 : 0;
+        return size_t(g) * (H + 1) + (H - c->height_h[s]);
+    };
+    std::vector<int> at(3 * size_t(H + 1) + 1, 0);
     for (int s = begin; s < begin + count; ++s) {
         const int n = c->node_off_h[s + 1] - c->node_off_h[s], k = tree_class(n);
         ++b.count[k];
         b.nmax[k] = std::max(b.nmax[k], n);
-    }
-    int at[kTreeClasses];
-    at[0] = begin;
-    for (int k = 1; k < kTreeClasses; ++k) at[k] = at[k - 1] + b.count[k - 1];
-    for (int s = begin; s < begin + count; ++s) slots[at[tree_class(c->node_off_h[s + 1] - c->node_off_h[s])]++] = s;
-    // tallest trees first inside a class: the nets with the longest level
-    // chains start first and the launch's tail is short; class 0's trees of
-    // at most c->tiny_bound nodes after its others
-    // (slots enter in ascending order, so ordering ties by slot is the
-    // stable order, without the temporary buffer of a stable sort)
-    auto tiny = [&](int u) { return c->node_off_h[u + 1] - c->node_off_h[u] <= c->tiny_bound; };
-    for (int k = 0, lo = begin; k < kTreeClasses; lo += b.count[k++])
-        std::sort(slots.begin() + lo, slots.begin() + lo + b.count[k], [&](int u, int v) {
-            if (k == 0 && tiny(u) != tiny(v)) return tiny(v);
-            return c->height_h[u] != c->height_h[v] ? c->height_h[u] > c->height_h[v] : u < v;
-        });
-    for (int j = begin; j < begin + b.count[0]; ++j)
-        if (tiny(slots[j])) {
+        if (!k && n <= c->tiny_bound) {
             ++b.tiny;
-            b.tiny_nmax = std::max(b.tiny_nmax, c->node_off_h[slots[j] + 1] - c->node_off_h[slots[j]]);
+            b.tiny_nmax = std::max(b.tiny_nmax, n);
         }
+        ++at[bucket(s, n) + 1];
+    }
+    for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
+    for (int s = begin; s < begin + count; ++s) slots[begin + at[bucket(s, c->node_off_h[s + 1] - c->node_off_h[s])]++] = s;
     return b;
 }
 
@@ -923,21 +930,31 @@ void reserve_dp_scratch(gr_ctx* c, const std::vector<BatchLaunch>& plan) {
     ensure_gscratch(c, need);
 }
 
+// Stages of at least this many nets plan on several host threads (starting
+// them costs about what 60k nets take on one).
+constexpr int kParallelPlan = 1 << 16;
+
 // Execution-order descriptors of the stage slots in slots[first, last):
 // each DP workgroup reads one int4 instead of chasing slot -> net -> offsets.
 void upload_desc(gr_ctx* c, const std::vector<int>& slots, int first, int last) {
     if (c->desc_h.size() != size_t(c->stage_count)) c->desc_h.assign(c->stage_count, int4{-1, -1, -1, -1});
-    bool changed = false;
-    for (int j = first; j < last; ++j) {
+    c->run_plan_key.clear();  // gr_lshape_run sets it again where these are its own
+    std::atomic<bool> changed{false};
+    auto make = [&](int j) {
         const int s = slots[j], id = c->net_ids_h[s];
         // nodes (at most kMaxTreeNodes) | the root's height << 16
         const int4 d{c->node_off_h[s], (c->node_off_h[s + 1] - c->node_off_h[s]) | c->height_h[s] << 16,
                      c->route_per_pin * c->pin_acc_num_h[id],
                      c->route_per_pin * (c->pin_acc_num_h[id + 1] - c->pin_acc_num_h[id])};
         int4& h = c->desc_h[j];
-        if (h.x != d.x || h.y != d.y || h.z != d.z || h.w != d.w) changed = true;
-        h = d;
-    }
+        if (h.x != d.x || h.y != d.y || h.z != d.z || h.w != d.w) {
+            h = d;
+            if (!changed.load(std::memory_order_relaxed)) changed = true;
+        }
+    };
+    if (last - first >= kParallelPlan) parallel_items(last - first, [&](int k) { make(first + k); });
+    else
+        for (int j = first; j < last; ++j) make(j);
     if (changed) upload(c->desc + first, c->desc_h.data() + first, sizeof(int4) * size_t(last - first), c->stream);
 }
 
@@ -1366,6 +1383,7 @@ int gr_ctx_set_routes(gr_ctx* c, int net_count, const int* pin_acc_num) {
     return guarded([&] {
         if (!c || net_count < 0 || !pin_acc_num) throw GrError(GR_E_ARG, "invalid route storage arguments");
         c->drop_graph();  // a captured batch loop holds the old route storage addresses
+        ++c->routes_gen;
         c->route_per_pin = c->next_route_per_pin;
         c->release_phase2();  // phase-two offsets index the old subnets
         c->mem.release(c->routes);
@@ -1643,15 +1661,29 @@ int gr_lshape_run(gr_ctx* c, int nbatch, const int* batch_off, int first_stamp, 
             throw GrError(GR_E_ARG, "execution mode not available (0 = plain, 1 = launches, 2 = persistent + graph)");
         require_stage(c, 0, batch_off[nbatch]);
         if (batch_off[0] != 0) throw GrError(GR_E_ARG, "batch offsets must start at 0");
-        std::vector<int> slots(c->stage_count);
-        std::vector<BatchLaunch> plan(nbatch);
-        size_t plain_need = 0;
-        for (int b = 0; b < nbatch; ++b) {
+        for (int b = 0; b < nbatch; ++b)
             if (batch_off[b + 1] < batch_off[b]) throw GrError(GR_E_ARG, "batch offsets must be non-decreasing");
-            const int begin = batch_off[b], count = batch_off[b + 1] - batch_off[b];
-            plan[b] = mode == 0 ? plan_batch_plain(c, begin, count, slots) : plan_batch(c, begin, count, slots);
-            if (mode == 0) plain_need = std::max(plain_need, plain_tables_needed(c, plan[b]));
+        std::vector<int> plan_key{c->stage_gen, c->routes_gen, mode == 0, c->tiny_bound};
+        plan_key.insert(plan_key.end(), batch_off, batch_off + nbatch + 1);
+        std::vector<BatchLaunch>& plan = c->run_plan;
+        if (plan_key != c->run_plan_key) {
+            c->run_plan_key.clear();
+            std::vector<int> slots(c->stage_count);
+            plan.assign(nbatch, BatchLaunch{});
+            auto make = [&](int b) {
+                const int begin = batch_off[b], count = batch_off[b + 1] - batch_off[b];
+                plan[b] = mode == 0 ? plan_batch_plain(c, begin, count, slots) : plan_batch(c, begin, count, slots);
+            };
+            if (batch_off[nbatch] >= kParallelPlan) parallel_tasks(nbatch, make);
+            else
+                for (int b = 0; b < nbatch; ++b) make(b);
+            c->slots_h.swap(slots);
+            upload_desc(c, c->slots_h, 0, c->stage_count);
+            c->run_plan_key = plan_key;
         }
+        size_t plain_need = 0;
+        if (mode == 0)
+            for (const BatchLaunch& b : plan) plain_need = std::max(plain_need, plain_tables_needed(c, b));
         if (mode == 0) ensure_gscratch(c, plain_need);
         else reserve_dp_scratch(c, plan);
         const long long qwords = (long long)kPersistentGroups * kDpQueues * kDpQueueStride;  // per batch
@@ -1680,9 +1712,6 @@ int gr_lshape_run(gr_ctx* c, int nbatch, const int* batch_off, int first_stamp, 
             std::vector<int> key{c->stage_gen, first_stamp, nbatch, c->per_wave[0], c->per_wave[1], mode, c->tiny_bound,
                                  c->tiny_per_wave};
             key.insert(key.end(), batch_off, batch_off + nbatch + 1);
-            // the graph reads the descriptors when it runs
-            c->slots_h = slots;
-            upload_desc(c, slots, 0, c->stage_count);
             if (!c->graph_exec || key != c->graph_key) {
                 c->drop_graph();
                 hip_check(hipStreamSynchronize(c->stream), "before graph capture");
@@ -1703,9 +1732,6 @@ int gr_lshape_run(gr_ctx* c, int nbatch, const int* batch_off, int first_stamp, 
                 hip_check(hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0), "hipGraphInstantiate");
                 c->graph_key = key;
             }
-        } else {
-            c->slots_h = slots;
-            upload_desc(c, slots, 0, c->stage_count);
         }
         hip_check(hipStreamSynchronize(c->stream), "stage plan");
         hip_check(hipDeviceSynchronize(), "before DAG interval");
