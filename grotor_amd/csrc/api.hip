@@ -215,6 +215,10 @@ struct gr_ctx {
     double* noalloc_scratch = nullptr;    // this device's `scratch` (gr_lshape_batch_noalloc)
     std::vector<int> noalloc_slots;       // sized at gr_lshape_upload
     ReuseArena score_mem;  // gr_score: lines, per-cell counters, partial sums
+    // exclusive prefix sums of the edge lengths, and the wire commit of the DP
+    // launches being enqueued (demand null: none)
+    long long *x_len_sum = nullptr, *y_len_sum = nullptr;
+    WireCommit dp_wires{};
     // grid arrays on their way between IDX and track-major order, and the
     // recomputed costs of gr_cost_download
     Workspace layout_ws, cost_ws;
@@ -556,8 +560,9 @@ constexpr int kCommitPackedNets = 4096;  // batches of at least this many nets c
 // Commit (K = 1) or removal (K = -1) of stage slots [begin, begin + count):
 // routes from `rs` (phase-one storage when null), or, with `current`, each
 // net's current route (phase-two words for nets marked live).
+// `wires` false: the DP launches have committed the wires (WireCommit).
 void launch_commit(gr_ctx* c, int begin, int count, int stamp, int K, const int* net_ids = nullptr,
-                   const RouteStore* rs = nullptr, bool current = false) {
+                   const RouteStore* rs = nullptr, bool current = false, bool wires = true) {
     if (!count) return;
     CommitArgs a = commit_args(c, begin, count, stamp, K);
     if (net_ids) a.net_ids = net_ids;
@@ -567,13 +572,13 @@ void launch_commit(gr_ctx* c, int begin, int count, int stamp, int K, const int*
     // resident at once; otherwise a wavefront per net
     if (count >= kCommitPackedNets) {
         const int blocks = std::min((count + 15) / 16, 4096);
-        timed(c, GR_K_COMMIT_WIRES, 0.0,
+        if (wires) timed(c, GR_K_COMMIT_WIRES, 0.0,
               [&] { hipLaunchKernelGGL(commit_wires_kernel<16>, dim3(blocks), dim3(256), 0, c->stream, a); });
         timed(c, GR_K_COMMIT_VIAS, 0.0,
               [&] { hipLaunchKernelGGL(commit_vias_kernel<16>, dim3(blocks), dim3(256), 0, c->stream, a); });
     } else {
         const int blocks = std::min((count + 3) / 4, 4096);
-        timed(c, GR_K_COMMIT_WIRES, 0.0,
+        if (wires) timed(c, GR_K_COMMIT_WIRES, 0.0,
               [&] { hipLaunchKernelGGL(commit_wires_kernel<64>, dim3(blocks), dim3(256), 0, c->stream, a); });
         timed(c, GR_K_COMMIT_VIAS, 0.0,
               [&] { hipLaunchKernelGGL(commit_vias_kernel<64>, dim3(blocks), dim3(256), 0, c->stream, a); });
@@ -731,6 +736,7 @@ void launch_lshape_class(gr_ctx* c, const BatchLaunch& b, int k, int per_wave_ov
     a.error = c->error;
     a.queue = nullptr;
     a.cus = c->cus;
+    a.wires = c->dp_wires;
     a.begin = b.begin;
     for (int j = 0; j < k; ++j) a.begin += b.count[j];
     a.count = b.count[k];
@@ -813,6 +819,7 @@ void launch_lshape_plain(gr_ctx* c, const BatchLaunch& b) {
     a.error = c->error;
     a.queue = nullptr;
     a.cus = c->cus;
+    a.wires = c->dp_wires;
     a.begin = b.begin;
     a.count = b.count[0];
     a.nmax = b.nmax[0];
@@ -855,6 +862,7 @@ void launch_lshape_queue_range(gr_ctx* c, int begin, int count, int nmax, int k,
     a.error = c->error;
     a.queue = queue;
     a.cus = c->cus;
+    a.wires = c->dp_wires;
     a.begin = begin;
     a.count = count;
     a.nmax = nmax;
@@ -1350,6 +1358,12 @@ int gr_ctx_create(const gr_grid_desc* grid, gr_ctx** out) {
         upload(xl, grid->x_edge_len, sizeof(int) * (g.X - 1), c->stream);
         upload(yl, grid->y_edge_len, sizeof(int) * (g.Y - 1), c->stream);
         g.x_edge_len = xl, g.y_edge_len = yl;
+        std::vector<long long> sums(size_t(g.X) + g.Y, 0);
+        for (int i = 1; i < g.X; ++i) sums[i] = sums[i - 1] + grid->x_edge_len[i - 1];
+        for (int i = 1; i < g.Y; ++i) sums[g.X + i] = sums[g.X + i - 1] + grid->y_edge_len[i - 1];
+        c->x_len_sum = c->mem.alloc<long long>(sums.size());
+        c->y_len_sum = c->x_len_sum + g.X;
+        upload(c->x_len_sum, sums.data(), sizeof(long long) * sums.size(), c->stream);
         c->capacity = c->mem.alloc<float>(c->cells);
         c->demand = c->mem.alloc<float>(c->cells);
         c->vcost = c->mem.alloc<float>(c->cells);
@@ -1697,12 +1711,29 @@ int gr_lshape_run(gr_ctx* c, int nbatch, const int* batch_off, int first_stamp, 
             if (mode == 2 && nbatch)  // a kernel, not a memset: the loop may be captured
                 hipLaunchKernelGGL(fill_int_kernel, dim3(unsigned((nbatch * qwords + 255) / 256)), dim3(256), 0,
                                    c->stream, c->dp_queue, 0, nbatch * qwords);
+            // The DP launches of a batch below kCommitPackedNets nets commit its
+            // wires: there the commit's own launch costs more than its work (64x64x5,
+            // 92 nets a batch: loop 0.91 -> 0.81 ms; 131x131x5, 510 a batch,
+            // plain form 1.84 -> 1.70).  Larger batches keep the launch of four nets
+            // per wavefront, whose lanes share a net's cells (590k nets, 9.7k a batch:
+            // 8.30 ms with it everywhere, 8.44 without it).  Profiled runs keep
+            // it too, so that each launch is timed alone.
+            struct Wires {
+                gr_ctx* c;
+                ~Wires() { c->dp_wires = WireCommit{}; }
+            } wires{c};
             for (int b = 0; b < nbatch; ++b) {
+                const int count = batch_off[b + 1] - batch_off[b];
+                const bool fused = !c->profiling && count < kCommitPackedNets;
                 launch_refresh(c, 0);
+                c->dp_wires = WireCommit{};
+                if (fused)
+                    c->dp_wires = WireCommit{c->demand, c->timestamp, c->track_dirty, c->stats,
+                                             c->x_len_sum, c->y_len_sum, first_stamp + b};
                 if (mode == 2) launch_lshape_persistent(c, plan[b], c->dp_queue + size_t(b) * qwords);
                 else if (mode == 1) launch_lshape(c, plan[b]);
                 else launch_lshape_plain(c, plan[b]);
-                launch_commit(c, batch_off[b], batch_off[b + 1] - batch_off[b], first_stamp + b, 1);
+                launch_commit(c, batch_off[b], count, first_stamp + b, 1, nullptr, nullptr, false, !fused);
             }
         };
         // a captured graph cannot carry profiling events: profiled runs of

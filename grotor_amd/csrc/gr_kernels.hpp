@@ -77,6 +77,16 @@ __global__ void commit_wires_kernel(CommitArgs a);
 template <int W>
 __global__ void commit_vias_kernel(CommitArgs a);
 
+// Wire commit of the nets a DP launch routes (demand nullptr: none): what
+// commit_wires_kernel adds for them at K = 1.
+struct WireCommit {
+    float* demand;
+    int* timestamp;
+    unsigned* track_dirty;
+    Stats* stats;
+    const long long *x_len_sum, *y_len_sum;  // exclusive prefix sums of the edge lengths
+    int stamp;
+};
 struct LshapeArgs {
     DeviceGrid g;
     const float* vcost;
@@ -94,6 +104,7 @@ struct LshapeArgs {
     int* error;
     int* queue;        // persistent form: the batch's kDpQueues work-queue counters (nullptr: one workgroup per P nets)
     int cus;           // compute units, for the persistent grid
+    WireCommit wires;
 };
 // Bytes of one net's DP tables for trees of up to nmax nodes (0 if L is not
 // supported), and the launch of `blocks` workgroups of a.per_wave nets each

@@ -336,13 +336,66 @@ __device__ __forceinline__ void root_merge(double& m, int& ch) {
     ch = take ? oc : ch;
 }
 
+// The net's wires committed where they were found: nets of a batch read the
+// costs, which only the next refresh changes, so their demand can go up while
+// others are still being solved, and the vias' launch, which needs every
+// wire timestamp of the batch, follows as before.  One lane per wire (a node's
+// edge has one or two); its unit edges are additions and stores nothing waits
+// for.  The lengths come as a difference of prefix sums, one load at each
+// end.  Used for the batches whose commit is all launch (gr_lshape_run has the
+// rule and both sides' times).
+template <int L>
+__device__ __forceinline__ void commit_net_wires(const LshapeArgs& a, const Tables<L>& s, int n, int lane, int W) {
+    const DeviceGrid& g = a.g;
+    const WireCommit& c = a.wires;
+    long long length = 0;
+    int edges = 0;
+    for (int t = lane + 2; t < 2 * n; t += W) {  // the root has no edge
+        const int i = t >> 1, second = t & 1;
+        const int v = s.xy[i], q = s.xy[s.par[i]];
+        const int x = v >> 16, y = v & 0xFFFF, px = q >> 16, py = q & 0xFFFF;
+        const int cl = s.path[i] / L % L, pl = s.path[i] % L;
+        const bool straight = x == px || y == py;
+        if (straight && second) continue;
+        const int l = second ? pl : cl;
+        const bool along_y = straight ? x == px : (layer_dir(g, cl) != 0) != (second != 0);
+        const int fixed = along_y ? (second ? px : x) : (second ? py : y);
+        const int lo = along_y ? min(y, py) : min(x, px), hi = along_y ? max(y, py) : max(x, px);
+        const int c0 = along_y ? cell_of(g, l, fixed, lo) : cell_of(g, l, lo, fixed);
+        const bool one_track = along_y == (layer_dir(g, l) != 0);
+        const int step = one_track ? 1 : (along_y ? g.X : g.Y);
+        c.timestamp[c0] = c.stamp;
+        c.timestamp[along_y ? cell_of(g, l, fixed, hi) : cell_of(g, l, hi, fixed)] = c.stamp;
+        if (lo == hi) continue;
+        if (one_track) c.track_dirty[track_of_cell(g, c0)] = 1u;
+        for (int d = 0; d < hi - lo; ++d) {
+            const int cell = c0 + d * step;
+            atomicAdd(c.demand + cell, 1.0f);
+            c.timestamp[cell] = c.stamp;
+            if (!one_track) c.track_dirty[track_of_cell(g, cell)] = 1u;
+        }
+        const long long* sum = along_y ? c.y_len_sum : c.x_len_sum;
+        length += sum[hi] - sum[lo];
+        edges += hi - lo;
+    }
+    for (int o = W / 2; o; o >>= 1) {
+        length += __shfl_xor(length, o, kWave);
+        edges += __shfl_xor(edges, o, kWave);
+    }
+    Stats* st = c.stats + blockIdx.x % kStatStripes;
+    if (lane == 0 && length) atomicAdd(&st->total_wirelength, double(length));
+    if (lane == 0 && edges) atomicAdd(&st->wire_edges, (unsigned long long)edges);
+}
+
 // rows (node, layer) per lane and pass of the cost gathers
 constexpr int kGatherRows = 2;
 
 // With a queue counter, lane 0 dequeues the workgroup's next chunk before
 // the traceback and parks it in *stash once the route words are placed, so
 // the atomic's round trip overlaps the last phases of this net's solve.
-template <int L>
+// WIRES: the net's wires are committed at the end (a variant of its own: the
+// code in the common kernel cost it 3 % where it is not used).
+template <int L, bool WIRES>
 __device__ void solve_net(const LshapeArgs& a, double* base, size_t words, int first_slot, int* counter = nullptr,
                           int* stash = nullptr) {
     constexpr int LL = L * L, T = kTri<L>;
@@ -660,18 +713,19 @@ __device__ void solve_net(const LshapeArgs& a, double* base, size_t words, int f
         }
     }
     if (lane == 0) routes[0] = s.woff[n];
+    if (WIRES) commit_net_wires<L>(a, s, n, lane, W);
 }
 
-template <int L>
+template <int L, bool WIRES>
 __global__ __launch_bounds__(kWave) void lshape_dp_lds_kernel(LshapeArgs a) {
     extern __shared__ double smem[];
-    solve_net<L>(a, smem, (table_bytes<L>(a.nmax, net_lanes<L>(a.per_wave)) + 7) / 8, blockIdx.x * a.per_wave);
+    solve_net<L, WIRES>(a, smem, (table_bytes<L>(a.nmax, net_lanes<L>(a.per_wave)) + 7) / 8, blockIdx.x * a.per_wave);
 }
 
-template <int L>
+template <int L, bool WIRES>
 __global__ __launch_bounds__(kWave) void lshape_dp_global_kernel(LshapeArgs a) {
     const size_t words = (table_bytes<L>(a.nmax, net_lanes<L>(a.per_wave)) + 7) / 8;
-    solve_net<L>(a, a.gscratch + words * a.per_wave * blockIdx.x, words, blockIdx.x * a.per_wave);
+    solve_net<L, WIRES>(a, a.gscratch + words * a.per_wave * blockIdx.x, words, blockIdx.x * a.per_wave);
 }
 
 // Persistent form: a grid no larger than what stays resident drains the
@@ -680,7 +734,7 @@ __global__ __launch_bounds__(kWave) void lshape_dp_global_kernel(LshapeArgs a) {
 // 128-byte line apart and zero at launch: workgroup w dequeues from counter
 // w % kDpQueues, which hands out chunks q, q + kDpQueues, ... in order (one
 // counter for all workgroups serializes the dequeues).
-template <int L>
+template <int L, bool WIRES>
 __global__ __launch_bounds__(kWave) void lshape_dp_queue_kernel(LshapeArgs a) {
     extern __shared__ double smem[];
     __shared__ int s_next;
@@ -694,28 +748,28 @@ __global__ __launch_bounds__(kWave) void lshape_dp_queue_kernel(LshapeArgs a) {
     if (threadIdx.x == 0) got = atomicAdd(counter, 1);
     int first = (__builtin_amdgcn_readfirstlane(got) * kDpQueues + q) * a.per_wave;
     while (first < a.count) {
-        solve_net<L>(a, smem, words, first, counter, &s_next);
+        solve_net<L, WIRES>(a, smem, words, first, counter, &s_next);
         __syncthreads();  // the tables and s_next are reused by the next nets
         first = (__builtin_amdgcn_readfirstlane(s_next) * kDpQueues + q) * a.per_wave;
         __syncthreads();  // every lane has read s_next before the next solve writes it
     }
 }
 
-template <int L>
+template <int L, bool WIRES>
 void launch_for(const LshapeArgs& a, int blocks, bool lds, hipStream_t st) {
     const size_t lds_bytes = ((table_bytes<L>(a.nmax, net_lanes<L>(a.per_wave)) + 7) / 8) * 8 * a.per_wave;
     if (a.queue) {
         int resident = 0;  // workgroups per compute unit; any value keeps the queue correct
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, lshape_dp_queue_kernel<L>, kWave, lds_bytes) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, (lshape_dp_queue_kernel<L, WIRES>), kWave, lds_bytes) !=
                 hipSuccess ||
             resident < 1)
             resident = 1;
         const int grid = std::max(1, std::min(blocks, resident * a.cus));
-        hipLaunchKernelGGL(lshape_dp_queue_kernel<L>, dim3(grid), dim3(kWave), lds_bytes, st, a);
+        hipLaunchKernelGGL((lshape_dp_queue_kernel<L, WIRES>), dim3(grid), dim3(kWave), lds_bytes, st, a);
     } else if (lds)
-        hipLaunchKernelGGL(lshape_dp_lds_kernel<L>, dim3(blocks), dim3(kWave), lds_bytes, st, a);
+        hipLaunchKernelGGL((lshape_dp_lds_kernel<L, WIRES>), dim3(blocks), dim3(kWave), lds_bytes, st, a);
     else
-        hipLaunchKernelGGL(lshape_dp_global_kernel<L>, dim3(blocks), dim3(kWave), 0, st, a);
+        hipLaunchKernelGGL((lshape_dp_global_kernel<L, WIRES>), dim3(blocks), dim3(kWave), 0, st, a);
 }
 
 }  // namespace
@@ -733,9 +787,10 @@ size_t lshape_scratch_bytes(int L, int nmax) {
 
 bool launch_lshape_dp(const LshapeArgs& a, int blocks, bool lds, hipStream_t st) {
     switch (a.g.L) {
-#define GR_L_CASE(n)                     \
-    case n:                              \
-        launch_for<n>(a, blocks, lds, st); \
+#define GR_L_CASE(n)                                                         \
+    case n:                                                                  \
+        if (a.wires.demand) launch_for<n, true>(a, blocks, lds, st);         \
+        else launch_for<n, false>(a, blocks, lds, st);                       \
         return true;
         GR_L_CASE(1) GR_L_CASE(2) GR_L_CASE(3) GR_L_CASE(4) GR_L_CASE(5) GR_L_CASE(6) GR_L_CASE(7) GR_L_CASE(8)
         GR_L_CASE(9) GR_L_CASE(10) GR_L_CASE(11) GR_L_CASE(12) GR_L_CASE(13) GR_L_CASE(14) GR_L_CASE(15)
