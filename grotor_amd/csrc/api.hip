@@ -2055,7 +2055,8 @@ int gr_ripup(gr_ctx* c, int threshold, unsigned char* is_of_net) {
         RipupArgs a{c->g, c->capacity, c->demand, c->of_sum, threshold};
         hipLaunchKernelGGL(overflow_prefix_kernel, dim3(c->tracks), dim3(256), 0, c->stream, a);
         if (c->net_count)
-            hipLaunchKernelGGL(overflow_nets_kernel, dim3((c->net_count + 255) / 256), dim3(256), 0, c->stream, c->g,
+            hipLaunchKernelGGL(overflow_nets_kernel, dim3(unsigned((size_t(c->net_count) * kOverflowLanes + 255) / 256)),
+                               dim3(256), 0, c->stream, c->g,
                                c->of_sum, RouteStore{c->routes, c->pin_acc_num, c->route_per_pin},
                                RouteStore{c->routes2, c->pin_off2, c->route2_per_pin}, c->live2, c->net_count,
                                c->of_flags);

@@ -210,25 +210,29 @@ __global__ __launch_bounds__(256) void overflow_prefix_kernel(RipupArgs a) {
     }
 }
 
+// Eight lanes per net, lanes over its segments: a thread per net walked its
+// words one dependent gather after the other (166k nets: 47.7 us; 16 lanes
+// 40.3, 8 lanes 31.8, 4 lanes 32.3: a net has about 8 segments).  Every
+// segment's count is non-negative, so the reference's early exit above 10 is
+// the same test on the whole sum.
 __global__ __launch_bounds__(256) void overflow_nets_kernel(DeviceGrid g, const int* of_sum, RouteStore rs,
                                                             RouteStore rs2, const unsigned char* live2, int net_count,
                                                             unsigned char* is_of_net) {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= net_count) return;
+    const int id = blockIdx.x * (256 / kOverflowLanes) + threadIdx.x / kOverflowLanes;
+    const int lane = threadIdx.x % kOverflowLanes;
+    if (id >= net_count) return;  // uniform over the net's lanes
     const int* r = current_route(rs, rs2, live2, id);
+    const int end = r[0];
     int of = 0;
-    unsigned char flag = 0;
-    for (int i = 1; i < r[0]; i += 2) {
-        const int l = r[i] / g.XY, x0 = r[i] / g.Y % g.X, y0 = r[i] % g.Y;
-        const int x1 = r[i + 1] / g.Y % g.X, y1 = r[i + 1] % g.Y;
+    for (int i = 1 + 2 * lane; i < end; i += 2 * kOverflowLanes) {
+        const int ra = r[i], rb = r[i + 1];
+        const int l = ra / g.XY, x0 = ra / g.Y % g.X, y0 = ra % g.Y;
+        const int x1 = rb / g.Y % g.X, y1 = rb % g.Y;
         if (x0 != x1) of += of_sum[cell_of(g, l, max(x0, x1), y0)] - of_sum[cell_of(g, l, min(x0, x1), y0)];
         if (y0 != y1) of += of_sum[cell_of(g, l, x0, max(y0, y1))] - of_sum[cell_of(g, l, x0, min(y0, y1))];
-        if (of > 10) {
-            flag = 1;
-            break;
-        }
     }
-    is_of_net[id] = flag;
+    for (int o = kOverflowLanes / 2; o; o >>= 1) of += __shfl_xor(of, o, kOverflowLanes);
+    if (lane == 0) is_of_net[id] = of > 10;
 }
 
 // Phase-two storage re-laid at a wider stride: one workgroup copies one

@@ -125,6 +125,7 @@ struct RipupArgs {
     int threshold;
 };
 __global__ void overflow_prefix_kernel(RipupArgs a);
+constexpr int kOverflowLanes = 8;  // lanes per net
 __global__ void overflow_nets_kernel(DeviceGrid g, const int* of_sum, RouteStore rs, RouteStore rs2,
                                      const unsigned char* live2, int net_count, unsigned char* is_of_net);
 
