@@ -2171,14 +2171,20 @@ int gr_zshape_run(gr_ctx* c, int first_stamp, double* elapsed_ms) {
             launch_refresh(c, 0);
             if (!count) continue;
             const gr_ctx::ZBatch& zb = c->z_split[b];
+            // the per-net kernel commits the wires where it routes the whole
+            // batch; profiled runs time the commit as a launch of its own
+            const bool fused = !zb.slow && !c->profiling;
             a.points = c->z_records + c->z_rec_off[b];
             a.list = c->z_list + zb.slow_off;
             a.count = zb.slow;
             a.raw_cap = c->z_raw_cap + begin;
             timed(c, GR_K_ZSHAPE, 0.0, [&] {
                 if (zb.fast) {
-                    const ZnetArgs f{g, c->presum, c->vcost, c->z_desc + zb.fast_off, c->z_fast_ids + zb.fast_off,
-                                     c->z_recs, rs, c->error};
+                    ZnetArgs f{g, c->presum, c->vcost, c->z_desc + zb.fast_off, c->z_fast_ids + zb.fast_off,
+                               c->z_recs, rs, c->error, {}};
+                    if (fused)
+                        f.wires = WireCommit{c->demand, c->timestamp, c->track_dirty, c->stats,
+                                             c->x_len_sum, c->y_len_sum, first_stamp + b};
                     launch_zshape_nets(f, zb.fast, zb.fast_nmax, c->stream);
                 }
                 if (!zb.slow) return;
@@ -2187,7 +2193,7 @@ int gr_zshape_run(gr_ctx* c, int first_stamp, double* elapsed_ms) {
                 hipLaunchKernelGGL(zshape_convert_kernel, dim3((zb.slow + 255) / 256), dim3(256), 0, c->stream, a,
                                    (const int*)(c->z_net_ids + begin), rs);
             });
-            launch_commit(c, begin, count, first_stamp + b, 1, c->z_net_ids);
+            launch_commit(c, begin, count, first_stamp + b, 1, c->z_net_ids, nullptr, false, !fused);
             hip_check(hipGetLastError(), "Z-shape kernels");
         }
         hip_check(hipStreamSynchronize(c->stream), "DAG interval");

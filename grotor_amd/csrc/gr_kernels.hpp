@@ -27,6 +27,17 @@ struct alignas(128) Stats {
 constexpr int kStatStripes = 64;
 constexpr int kCounterStride = 16;  // 64-bit counters per 128-byte stripe
 
+// Wire commit of the nets a DP launch routes (demand nullptr: none): what
+// commit_wires_kernel adds for them at K = 1.
+struct WireCommit {
+    float* demand;
+    int* timestamp;
+    unsigned* track_dirty;
+    Stats* stats;
+    const long long *x_len_sum, *y_len_sum;  // exclusive prefix sums of the edge lengths
+    int stamp;
+};
+
 // Error codes written by kernels into the context's device error word.
 enum DeviceError : int {
     kDevOk = 0,
@@ -77,16 +88,6 @@ __global__ void commit_wires_kernel(CommitArgs a);
 template <int W>
 __global__ void commit_vias_kernel(CommitArgs a);
 
-// Wire commit of the nets a DP launch routes (demand nullptr: none): what
-// commit_wires_kernel adds for them at K = 1.
-struct WireCommit {
-    float* demand;
-    int* timestamp;
-    unsigned* track_dirty;
-    Stats* stats;
-    const long long *x_len_sum, *y_len_sum;  // exclusive prefix sums of the edge lengths
-    int stamp;
-};
 struct LshapeArgs {
     DeviceGrid g;
     const float* vcost;
@@ -224,6 +225,7 @@ struct ZnetArgs {
     const int* recs;
     RouteStore rs;
     int* error;
+    WireCommit wires;
 };
 size_t znet_lds_bytes(int L, int n);
 // nmax: the most nodes of a net in the list
