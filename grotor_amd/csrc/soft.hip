@@ -34,8 +34,8 @@
 //
 // Both passes run level by level over the nodes of a chunk of nets (see
 // "chunks of nets" below), L lanes per node, and for kind 1 over the edges of
-// a level, 16 lanes each, lane = bend position.  R, the type of the tables and of exp /
-// log, is float or double; costs and gradients stay FP64.
+// a level, 16 lanes each, lane = bend position.  R, the type of the tables and
+// of exp / log, is float or double; costs and gradients stay FP64.
 #include "gr_kernels.hpp"
 
 namespace grotor {
