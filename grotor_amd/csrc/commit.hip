@@ -210,11 +210,24 @@ __global__ __launch_bounds__(256) void overflow_prefix_kernel(RipupArgs a) {
     }
 }
 
+// Overflowed edges of a route segment.  One across its layer's tracks (a net
+// that found no finite solution holds such words) counts a difference of two
+// tracks' prefixes, which may be negative.
+__device__ __forceinline__ int segment_overflow(const DeviceGrid& g, const int* of_sum, int ra, int rb) {
+    const int l = ra / g.XY, x0 = ra / g.Y % g.X, y0 = ra % g.Y;
+    const int x1 = rb / g.Y % g.X, y1 = rb % g.Y;
+    int of = 0;
+    if (x0 != x1) of += of_sum[cell_of(g, l, max(x0, x1), y0)] - of_sum[cell_of(g, l, min(x0, x1), y0)];
+    if (y0 != y1) of += of_sum[cell_of(g, l, x0, max(y0, y1))] - of_sum[cell_of(g, l, x0, min(y0, y1))];
+    return of;
+}
+
 // Eight lanes per net, lanes over its segments: a thread per net walked its
 // words one dependent gather after the other (166k nets: 47.7 us; 16 lanes
-// 40.3, 8 lanes 31.8, 4 lanes 32.3: a net has about 8 segments).  Every
-// segment's count is non-negative, so the reference's early exit above 10 is
-// the same test on the whole sum.
+// 40.3, 8 lanes 31.8, 4 lanes 32.3: a net has about 8 segments).  The
+// reference leaves its walk where the running count exceeds 10, which is the
+// test on the whole sum while no segment counts below zero; a net with one
+// that does is walked in order.
 __global__ __launch_bounds__(256) void overflow_nets_kernel(DeviceGrid g, const int* of_sum, RouteStore rs,
                                                             RouteStore rs2, const unsigned char* live2, int net_count,
                                                             unsigned char* is_of_net) {
@@ -223,15 +236,20 @@ __global__ __launch_bounds__(256) void overflow_nets_kernel(DeviceGrid g, const 
     if (id >= net_count) return;  // uniform over the net's lanes
     const int* r = current_route(rs, rs2, live2, id);
     const int end = r[0];
-    int of = 0;
+    int of = 0, low = 0;
     for (int i = 1 + 2 * lane; i < end; i += 2 * kOverflowLanes) {
-        const int ra = r[i], rb = r[i + 1];
-        const int l = ra / g.XY, x0 = ra / g.Y % g.X, y0 = ra % g.Y;
-        const int x1 = rb / g.Y % g.X, y1 = rb % g.Y;
-        if (x0 != x1) of += of_sum[cell_of(g, l, max(x0, x1), y0)] - of_sum[cell_of(g, l, min(x0, x1), y0)];
-        if (y0 != y1) of += of_sum[cell_of(g, l, x0, max(y0, y1))] - of_sum[cell_of(g, l, x0, min(y0, y1))];
+        const int d = segment_overflow(g, of_sum, r[i], r[i + 1]);
+        of += d;
+        low = min(low, d);
     }
     for (int o = kOverflowLanes / 2; o; o >>= 1) of += __shfl_xor(of, o, kOverflowLanes);
+    if (__any(low < 0)) {
+        for (int o = kOverflowLanes / 2; o; o >>= 1) low = min(low, __shfl_xor(low, o, kOverflowLanes));
+        if (low < 0) {
+            of = 0;
+            for (int i = 1; i < end && of <= 10; i += 2) of += segment_overflow(g, of_sum, r[i], r[i + 1]);
+        }
+    }
     if (lane == 0) is_of_net[id] = of > 10;
 }
 

@@ -414,3 +414,39 @@ def test_graph_replay_after_storage_changes(ga, ora):
     ctx.lshape_run(sched["batch_off"], first_stamp=1, mode=2)
     check(ctx, "stride pending")
     ctx.close()
+
+
+def test_ripup_counts_wires_across_tracks_in_order(ga, ora):
+    """Words a net without a finite solution leaves behind may run across its
+    layer's tracks, where a difference of prefixes can be negative: the rip-up
+    test is on the running count, 10 exceeded anywhere along the words."""
+    X, Y = 41, 7
+    cap = np.full((1, X, Y), 100, np.float32)
+    cap[0, :, 1] = 0  # the only overflowed track
+    t = dict(L=1, X=X, Y=Y, DIR=0, unit_length_wire_cost=0.01, unit_via_cost=4.0,
+             unit_length_short_costs=np.ones(1), x_edge_len=np.full(X - 1, 300, np.int32),
+             y_edge_len=np.full(Y - 1, 300, np.int32), capacity=cap.ravel())
+    nets = []
+    for last in range(0, 40, 3):
+        # the root, a neighbour on track 1 (some edges, all overflowed), and
+        # one on track 5 reached across the tracks (the same count, negative)
+        nets.append([(20, 1), (last, 1), (20, 5)])
+        nets.append([(last, 1), (20, 1), (20, 5), (12, 5), (12, 1), (last // 2, 1), (last // 2, 4)])
+    off = np.concatenate([[0], np.cumsum([len(n) for n in nets])]).astype(np.int32)
+    nodes = np.array([x * Y + y for n in nets for x, y in n], np.int32)
+    parents = np.array([p for k, n in enumerate(nets) for p in ([-1, 0, 0] if len(n) == 3 else range(-1, len(n) - 1))],
+                       np.int32)
+    print("rip-up across tracks", flush=True)
+    ctx = ga.Context(t)
+    ctx.set_routes(off)
+    ctx.lshape_upload(np.arange(len(nets)), off, nodes, parents)
+    ctx.upload_demand(np.ones(X * Y, np.float32))
+    ctx.refresh()
+    with pytest.raises(ga.GrError, match="no finite layer"):
+        ctx.lshape_batch(0, len(nets), 1)
+    routes = ctx.routes()
+    flags = ctx.ripup(len(nets), 0)
+    want = ora.Grid(t).ripup(ctx.demand(), routes, off, 0)
+    assert 0 < want.sum() < len(nets)
+    assert np.array_equal(flags, want)
+    ctx.close()
