@@ -1425,6 +1425,7 @@ int gr_ctx_set_route_stride(gr_ctx* c, int words_per_pin) {
 int gr_ctx_set_cost_params(gr_ctx* c, double slope, double zero_slope, double via_weight, int integer_wire) {
     return guarded([&] {
         if (!c) throw GrError(GR_E_ARG, "null context");
+        c->drop_graph();  // the captured loops hold the old parameters
         c->cp.slope = slope;
         c->cp.zero_slope = zero_slope;
         c->cp.via_weight = via_weight;

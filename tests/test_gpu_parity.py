@@ -450,3 +450,35 @@ def test_ripup_counts_wires_across_tracks_in_order(ga, ora):
     assert 0 < want.sum() < len(nets)
     assert np.array_equal(flags, want)
     ctx.close()
+
+
+def test_captured_loop_follows_the_cost_parameters(ga, ora):
+    """A replay after gr_ctx_set_cost_params runs with the new parameters:
+    equal to a context that had them from its start."""
+    _, t = topology(6, 4)
+    color, nb = ora.batches(t["X"], t["Y"], t["pt_off"], t["pts"], t["hs_off"], t["hsegs"], t["vs_off"], t["vsegs"])
+    sched = ga.execution_schedule(t, color, nb)
+    print("captured L-shape loop and cost parameters", flush=True)
+
+    def prepared():
+        ctx = ga.Context(t)
+        ctx.set_routes(t["pin_acc_num"])
+        ctx.lshape_upload(sched["net_ids"], sched["node_off"], sched["nodes"], sched["parents"])
+        return ctx
+
+    def run(ctx):
+        ctx.reset()
+        ctx.upload_demand(random_demand(t, 5))
+        ctx.lshape_run(sched["batch_off"], 1, 2)
+        return ctx.routes()
+
+    new = (3.0, 0.1, 0.05)
+    ctx, fresh = prepared(), prepared()
+    fresh.set_cost_params(*new)
+    old, want = run(ctx), run(fresh)
+    assert not np.array_equal(old, want)  # the parameters matter on this instance
+    ctx.set_cost_params(*new)
+    for _ in range(2):
+        assert np.array_equal(run(ctx), want)
+    ctx.close()
+    fresh.close()
