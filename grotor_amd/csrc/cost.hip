@@ -123,9 +123,10 @@ __global__ __launch_bounds__(256) void layout_kernel(DeviceGrid g, LayoutArrays<
     const int l = blockIdx.z % unsigned(g.L), tx = threadIdx.x % kLayoutTile, ty = threadIdx.x / kLayoutTile;
     const size_t base = size_t(l) * g.XY;
     // rows of the source: x (IDX) or the track y of a horizontal layer
-    const bool copy = layer_dir(g, l);
-    const int rows = to_track || copy ? g.X : g.Y, cols = to_track || copy ? g.Y : g.X;
-    const int r0 = blockIdx.y * kLayoutTile, c0 = blockIdx.x * kLayoutTile;
+    const bool copy = layer_dir(g, l), by_x = to_track || copy;
+    const int rows = by_x ? g.X : g.Y, cols = by_x ? g.Y : g.X;
+    // block y over the tiles of x, block x over those of y, for either order
+    const int r0 = (by_x ? blockIdx.y : blockIdx.x) * kLayoutTile, c0 = (by_x ? blockIdx.x : blockIdx.y) * kLayoutTile;
     for (int r = ty; r < kLayoutTile; r += 256 / kLayoutTile)
         if (r0 + r < rows && c0 + tx < cols) {
             const T v = src[base + size_t(r0 + r) * cols + c0 + tx];
@@ -140,9 +141,10 @@ __global__ __launch_bounds__(256) void layout_kernel(DeviceGrid g, LayoutArrays<
 
 template <class T>
 void launch_layout(const DeviceGrid& g, const LayoutArrays<T>& a, bool to_track, hipStream_t st) {
-    const unsigned side = unsigned((std::max(g.X, g.Y) + kLayoutTile - 1) / kLayoutTile);
     if (!a.count) return;
-    hipLaunchKernelGGL(layout_kernel<T>, dim3(side, side, unsigned(g.L * a.count)), dim3(256), 0, st, g, a, to_track ? 1 : 0);
+    const dim3 grid(unsigned((g.Y + kLayoutTile - 1) / kLayoutTile), unsigned((g.X + kLayoutTile - 1) / kLayoutTile),
+                    unsigned(g.L * a.count));
+    hipLaunchKernelGGL(layout_kernel<T>, grid, dim3(256), 0, st, g, a, to_track ? 1 : 0);
 }
 template void launch_layout<float>(const DeviceGrid&, const LayoutArrays<float>&, bool, hipStream_t);
 template void launch_layout<int>(const DeviceGrid&, const LayoutArrays<int>&, bool, hipStream_t);
