@@ -50,6 +50,13 @@ struct DeviceArena {
     }
 };
 
+// Scratch of one call that its context keeps for the next: at most this much
+// for each purpose (a 1024 x 1024 x 10 grid stays below it).  More is given back
+// when the call ends: next to the transfers of such a grid its allocation
+// does not count, and a call that used to fit must not fail over what an
+// earlier one left.
+constexpr size_t kKeptScratch = size_t(256) << 20;
+
 // Device blocks kept from one call for the next: the k-th alloc of a call
 // takes the k-th block, replaced when it is too small.
 struct ReuseArena {
@@ -59,6 +66,16 @@ struct ReuseArena {
     ReuseArena(const ReuseArena&) = delete;
     ReuseArena& operator=(const ReuseArena&) = delete;
     void begin() { at = 0; }
+    // Frees the blocks if they hold more than kKeptScratch (hipFree waits for
+    // the device).
+    void trim() {
+        size_t held = 0;
+        for (auto& [p, cap] : blocks) held += cap;
+        if (held <= kKeptScratch) return;
+        for (auto& [p, cap] : blocks)
+            if (p) (void)hipFree(p);
+        blocks.clear();
+    }
     template <class T>
     T* alloc(size_t count) {
         const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
@@ -118,6 +135,21 @@ struct Workspace {
         Carver real{base};
         layout(real);
     }
+    // Frees the buffer if it holds more than kKeptScratch (hipFree waits for
+    // the device).
+    void trim() {
+        if (cap <= kKeptScratch) return;
+        (void)hipFree(base);
+        base = nullptr;
+        cap = 0;
+    }
+};
+
+// At the end of a call, also one that throws: w.trim().
+template <class W>
+struct Trim {
+    W& w;
+    ~Trim() { w.trim(); }
 };
 
 // Scratch of the allocation-free DP entry point (gr_lshape_batch_noalloc):
@@ -431,9 +463,25 @@ void host_from_track_major(const DeviceGrid& g, const T* src, T* dst) {
 }
 
 // Up to two grid arrays of the ABI (IDX order, host) into track-major device
-// arrays and back, through the context's layout buffer, in one layout launch;
-// a null host pointer skips its array.  An upload may still be enqueued on
-// return: the caller waits for the stream before the host arrays may go.
+// arrays and back, through the context's layout buffer, in one layout launch,
+// or in several over slabs of layers where the arrays are larger than
+// kKeptScratch (a layer's cells lie together in both orders); a null host
+// pointer skips its array.  An upload may still be enqueued on return: the
+// caller waits for the stream before the host arrays may go.
+template <class T, class F>
+void for_layer_slabs(gr_ctx* c, int arrays, F&& f) {
+    if (!arrays) return;
+    const size_t layer = sizeof(T) * size_t(c->g.XY) * arrays;
+    const int slab = int(std::max<size_t>(1, std::min<size_t>(c->g.L, kKeptScratch * 4 / 5 / layer)));
+    T* tmp = nullptr;
+    c->layout_ws.carve([&](auto& cv) { tmp = cv.template take<T>(size_t(c->g.XY) * slab * arrays); });
+    Trim<Workspace> trim{c->layout_ws};
+    for (int l = 0; l < c->g.L; l += slab) {
+        LayoutArrays<T> a{};
+        a.first = l, a.layers = std::min(slab, c->g.L - l);
+        f(a, tmp, size_t(l) * c->g.XY, size_t(a.layers) * c->g.XY);
+    }
+}
 template <class T>
 void upload_grids(gr_ctx* c, T* dst0, const T* src0, T* dst1 = nullptr, const T* src1 = nullptr) {
     if (c->cells < kHostLayoutCells) {
@@ -446,17 +494,16 @@ void upload_grids(gr_ctx* c, T* dst0, const T* src0, T* dst1 = nullptr, const T*
         }
         return;
     }
-    T* tmp = nullptr;
-    c->layout_ws.carve([&](auto& cv) { tmp = cv.template take<T>(c->cells * (src1 ? 2 : 1)); });
-    LayoutArrays<T> a{};
-    for (auto [dst, src] : {std::pair<T*, const T*>{dst0, src0}, {dst1, src1}}) {
-        if (!src) continue;
-        upload(tmp, src, sizeof(T) * c->cells, c->stream);
-        a.src[a.count] = tmp, a.dst[a.count++] = dst;
-        tmp += c->cells;
-    }
-    launch_layout(c->g, a, true, c->stream);
-    hip_check(hipGetLastError(), "layout kernel");
+    for_layer_slabs<T>(c, (src0 != nullptr) + (src1 != nullptr), [&](LayoutArrays<T>& a, T* tmp, size_t at, size_t n) {
+        for (auto [dst, src] : {std::pair<T*, const T*>{dst0, src0}, {dst1, src1}}) {
+            if (!src) continue;
+            upload(tmp, src + at, sizeof(T) * n, c->stream);
+            a.src[a.count] = tmp, a.dst[a.count++] = dst + at;
+            tmp += n;
+        }
+        launch_layout(c->g, a, true, c->stream);
+        hip_check(hipGetLastError(), "layout kernel");
+    });
 }
 template <class T>
 void download_grids(gr_ctx* c, const T* src0, T* dst0, const T* src1 = nullptr, T* dst1 = nullptr) {
@@ -469,19 +516,18 @@ void download_grids(gr_ctx* c, const T* src0, T* dst0, const T* src1 = nullptr, 
         }
         return;
     }
-    T* tmp = nullptr;
-    c->layout_ws.carve([&](auto& cv) { tmp = cv.template take<T>(c->cells * (dst1 ? 2 : 1)); });
-    LayoutArrays<T> a{};
-    T* host[2];
-    for (auto [src, dst] : {std::pair<const T*, T*>{src0, dst0}, {src1, dst1}}) {
-        if (!dst) continue;
-        host[a.count] = dst;
-        a.src[a.count] = src, a.dst[a.count++] = tmp;
-        tmp += c->cells;
-    }
-    launch_layout(c->g, a, false, c->stream);
-    hip_check(hipGetLastError(), "layout kernel");
-    for (int k = 0; k < a.count; ++k) download(host[k], a.dst[k], sizeof(T) * c->cells, c->stream);
+    for_layer_slabs<T>(c, (dst0 != nullptr) + (dst1 != nullptr), [&](LayoutArrays<T>& a, T* tmp, size_t at, size_t n) {
+        T* host[2];
+        for (auto [src, dst] : {std::pair<const T*, T*>{src0, dst0}, {src1, dst1}}) {
+            if (!dst) continue;
+            host[a.count] = dst + at;
+            a.src[a.count] = src + at, a.dst[a.count++] = tmp;
+            tmp += n;
+        }
+        launch_layout(c->g, a, false, c->stream);
+        hip_check(hipGetLastError(), "layout kernel");
+        for (int k = 0; k < a.count; ++k) download(host[k], a.dst[k], sizeof(T) * n, c->stream);
+    });
 }
 
 // Every track marked for the next refresh.
@@ -1454,6 +1500,7 @@ int gr_cost_refresh_full(gr_ctx* c) {
 int gr_cost_download(gr_ctx* c, float* wcost, float* vcost, double* presum) {
     return guarded([&] {
         if (!c) throw GrError(GR_E_ARG, "null context");
+        Trim<Workspace> trim{c->cost_ws};
         float* tmp = nullptr;
         if (wcost) {
             // wcost is not kept resident: recompute it from the current demand
@@ -3120,6 +3167,7 @@ int gr_score(gr_ctx* c, int nets, const int* pin_off, const int* pins, const int
         if (!c || !capacity || !overflow_cost || !out) throw GrError(GR_E_ARG, "null argument");
         ReuseArena& ar = c->score_mem;
         ar.begin();
+        Trim<ReuseArena> trim{ar};
         ScoreArgs a = net_lines(c, ar, nets, pin_off, pins, extra_off, extra, sub_off, subs, layer_dir);
         const int X = c->g.X, Y = c->g.Y, M = c->g.L + 1;
         const long long XY = (long long)X * Y, cells = XY * M;

@@ -118,12 +118,13 @@ constexpr int kLayoutTile = 32;
 template <class T>
 __global__ __launch_bounds__(256) void layout_kernel(DeviceGrid g, LayoutArrays<T> arrays, int to_track) {
     __shared__ T tile[kLayoutTile][kLayoutTile + 1];
-    const T* __restrict__ src = blockIdx.z < unsigned(g.L) ? arrays.src[0] : arrays.src[1];
-    T* __restrict__ dst = blockIdx.z < unsigned(g.L) ? arrays.dst[0] : arrays.dst[1];
-    const int l = blockIdx.z % unsigned(g.L), tx = threadIdx.x % kLayoutTile, ty = threadIdx.x / kLayoutTile;
+    const unsigned layers = unsigned(arrays.layers);
+    const T* __restrict__ src = blockIdx.z < layers ? arrays.src[0] : arrays.src[1];
+    T* __restrict__ dst = blockIdx.z < layers ? arrays.dst[0] : arrays.dst[1];
+    const int l = blockIdx.z % layers, tx = threadIdx.x % kLayoutTile, ty = threadIdx.x / kLayoutTile;
     const size_t base = size_t(l) * g.XY;
     // rows of the source: x (IDX) or the track y of a horizontal layer
-    const bool copy = layer_dir(g, l), by_x = to_track || copy;
+    const bool copy = layer_dir(g, arrays.first + l), by_x = to_track || copy;
     const int rows = by_x ? g.X : g.Y, cols = by_x ? g.Y : g.X;
     // block y over the tiles of x, block x over those of y, for either order
     const int r0 = (by_x ? blockIdx.y : blockIdx.x) * kLayoutTile, c0 = (by_x ? blockIdx.x : blockIdx.y) * kLayoutTile;
@@ -143,7 +144,7 @@ template <class T>
 void launch_layout(const DeviceGrid& g, const LayoutArrays<T>& a, bool to_track, hipStream_t st) {
     if (!a.count) return;
     const dim3 grid(unsigned((g.Y + kLayoutTile - 1) / kLayoutTile), unsigned((g.X + kLayoutTile - 1) / kLayoutTile),
-                    unsigned(g.L * a.count));
+                    unsigned(a.layers * a.count));
     hipLaunchKernelGGL(layout_kernel<T>, grid, dim3(256), 0, st, g, a, to_track ? 1 : 0);
 }
 template void launch_layout<float>(const DeviceGrid&, const LayoutArrays<float>&, bool, hipStream_t);

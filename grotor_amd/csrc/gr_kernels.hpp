@@ -52,13 +52,15 @@ __global__ void refresh_tracks_kernel(DeviceGrid g, const float* capacity, const
                                       double* presum, float* wcost_out, unsigned* track_dirty, int force,
                                       CostParams cp, unsigned long long* refreshed);
 
-// dst = src for up to two device arrays over the whole grid, between IDX
-// order and track-major order; no array is its own copy
+// dst = src for up to two device arrays over `layers` layers from `first` on
+// (where the pointers point), between IDX order and track-major order; no
+// array is its own copy
 template <class T>
 struct LayoutArrays {
     const T* src[2];
     T* dst[2];
     int count;
+    int first, layers;
 };
 template <class T>
 void launch_layout(const DeviceGrid& g, const LayoutArrays<T>& a, bool to_track, hipStream_t stream);

@@ -3,6 +3,7 @@ device): uploads, downloads and the costs computed in between equal the
 oracle's on grids whose sides are no multiple of the transpose's 32 x 32
 tile, in both orientations of the first layer, on either side of the 32768
 cells above which the order changes on the device."""
+import ctypes
 import time
 
 import numpy as np
@@ -36,11 +37,10 @@ def test_grid_arrays_keep_their_cells(ga, ora, L, X, Y, DIR):
     ctx.close()
 
 
-def _context(ga, L, X, Y):
-    t = dict(L=L, X=X, Y=Y, DIR=0, unit_length_wire_cost=0.01, unit_via_cost=4.0,
-             unit_length_short_costs=np.ones(L), x_edge_len=np.full(X - 1, 30, np.int32),
-             y_edge_len=np.full(Y - 1, 30, np.int32), capacity=np.full(L * X * Y, 8, np.float32))
-    return ga.Context(t)
+def _grid(L, X, Y):
+    return dict(L=L, X=X, Y=Y, DIR=0, unit_length_wire_cost=0.01, unit_via_cost=4.0,
+                unit_length_short_costs=np.ones(L), x_edge_len=np.full(X - 1, 30, np.int32),
+                y_edge_len=np.full(Y - 1, 30, np.int32), capacity=np.full(L * X * Y, 8, np.float32))
 
 
 @pytest.mark.parametrize("X,Y", [(8192, 2), (2, 8192)])
@@ -51,7 +51,7 @@ def test_narrow_grids_cost_what_their_cells_do(ga, X, Y):
     print(f"narrow grid {X}x{Y}", flush=True)
     best = []
     for x, y in ((X, Y), (128, 128)):
-        ctx = _context(ga, 15, x, y)
+        ctx = ga.Context(_grid(15, x, y))
         demand = np.arange(15 * x * y, dtype=np.float32) % 31
         runs = []
         for _ in range(15):
@@ -63,3 +63,34 @@ def test_narrow_grids_cost_what_their_cells_do(ga, X, Y):
         best.append(min(runs))
         ctx.close()
     assert best[0] < 3 * best[1], best
+
+
+def test_scratch_of_a_large_grid_is_given_back(ga, ora):
+    """What the grid exchanges, the cost download and the score need on the
+    way does not stay allocated beyond a fixed amount, and arrays that change
+    their order a few layers at a time keep their cells."""
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert ga.lib().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    L, X, Y = 2, 4096, 4096
+    t = _grid(L, X, Y)
+    ctx = ga.Context(t)
+    ctx.set_routes(np.array([0, 1], np.int32))
+    demand = (np.arange(L * X * Y) % 17).astype(np.float32)
+    before = free()
+    print("scratch of a large grid", flush=True)
+    ctx.upload_demand(demand)
+    assert np.array_equal(ctx.demand(), demand)
+    ctx.refresh()
+    for got, want in zip(ctx.costs(), ora.Grid(t).refresh(demand)):
+        assert np.array_equal(_bits(got), _bits(want.ravel()))
+    none = np.zeros(2, np.int32)
+    lines = dict(pin_off=none, pins=none[:0], extra_off=none, extra=none[:0], sub_off=none, subs=none[:0])
+    M = L + 1
+    r = ctx.score(lines, np.arange(M) & 1, np.ones(M * X * Y), np.ones(M), demand=True)
+    assert r["wirelength"] == 0
+    held = before - free()
+    assert held <= 600 << 20, held
+    ctx.close()
