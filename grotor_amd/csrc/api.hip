@@ -1152,96 +1152,72 @@ void require_stage(gr_ctx* c, int begin, int count) {
     if (begin < 0 || count < 0 || begin + count > c->stage_count) throw GrError(GR_E_ARG, "slot range outside the stage");
 }
 
-// The Z-shape nets of a plan that zshape_net_kernel can route, in its record
-// layout (ZnetArgs), and the batch positions of the others (a tree too large
-// for LDS, two nodes at one place, a node without exactly one parent, a gap
-// in the child slots: the shared map of the general kernels gives those
-// cases their meaning).  n: side of the map the records' positions index.
-struct ZnetPlan {
-    std::vector<int4> desc;
-    std::vector<int> ids, recs, list;
-    std::vector<gr_ctx::ZBatch> split;
-};
+// One net's record (a Z-shape plan's, validated) as zshape_net_kernel takes
+// it: what its own record layout (ZnetArgs) is made of.  kZnetLds keeps the
+// node count below kZnetMaxNodes.
+struct ZnetTree {
+    int m, height_of_root;
+    int parent[kZnetMaxNodes];  // parent | slot << 16, -1: the root
+    int height[kZnetMaxNodes];
 
-ZnetPlan plan_znets(const DeviceGrid& g, int n, int nbatch, const int* batch_off, const int* net_ids,
-                    const long long* rec_off, const int* records, const int* raw_cap) {
-    ZnetPlan zp;
-    zp.split.resize(nbatch);
-    std::vector<int> parent, height, at, level, pos, order;
-    for (int b = 0; b < nbatch; ++b) {
-        gr_ctx::ZBatch& zb = zp.split[b];
-        zb = {int(zp.desc.size()), 0, 1, int(zp.list.size()), 0};
-        const int begin = batch_off[b], count = batch_off[b + 1] - begin;
-        for (int k = 0; k < count; ++k) {
-            const int* rec = records + rec_off[b] + records[rec_off[b] + k];
-            const int m = rec[1];
-            rec += 2;
-            bool fast = m <= kZnetMaxNodes && znet_lds_bytes(g.L, m) <= kZnetLds && zp.recs.size() < size_t(INT32_MAX / 2);
-            int H = 0;
-            if (fast) {
-                parent.assign(m, -1);
-                height.assign(m, 0);
-                pos.resize(m);
-                for (int i = 0; i < m; ++i) pos[i] = rec[6 * i];
-                std::sort(pos.begin(), pos.end());
-                fast = std::adjacent_find(pos.begin(), pos.end()) == pos.end();
-                for (int i = m - 1; i >= 0 && fast; --i)
-                    for (int j = 0; j < 3; ++j) {
-                        const int ch = rec[6 * i + 3 + j];
-                        if (ch == -1) continue;
-                        if ((j && rec[6 * i + 2 + j] == -1) || parent[ch / 6] >= 0) fast = false;
-                        parent[ch / 6] = i | j << 16;
-                        height[i] = std::max(height[i], height[ch / 6] + 1);
-                    }
-                for (int i = 1; i < m && fast; ++i) fast = parent[i] >= 0;
+    // False where the general kernels route the net: a tree too large for LDS,
+    // two nodes at one place, a node without exactly one parent, a gap in the
+    // child slots (the shared map gives those cases their meaning).
+    bool read(int L, const int* rec) {
+        m = rec[1];
+        rec += 2;
+        if (m >= kZnetMaxNodes || znet_lds_bytes(L, m) > kZnetLds) return false;
+        int pos[kZnetMaxNodes];
+        for (int i = 0; i < m; ++i) parent[i] = -1, height[i] = 0, pos[i] = rec[6 * i];
+        std::sort(pos, pos + m);
+        if (std::adjacent_find(pos, pos + m) != pos + m) return false;
+        for (int i = m - 1; i >= 0; --i)
+            for (int j = 0; j < 3; ++j) {
+                const int ch = rec[6 * i + 3 + j];
+                if (ch == -1) continue;
+                if ((j && rec[6 * i + 2 + j] == -1) || parent[ch / 6] >= 0) return false;
+                parent[ch / 6] = i | j << 16;
+                height[i] = std::max(height[i], height[ch / 6] + 1);
             }
-            if (!fast) {
-                zp.list.push_back(k);
-                ++zb.slow;
-                continue;
-            }
-            H = height[0];
-            level.assign(H + 2, 0);
-            for (int i = 0; i < m; ++i) ++level[height[i] + 1];
-            for (int h = 0; h <= H; ++h) level[h + 1] += level[h];
-            at.resize(m);
-            order.resize(m);
-            {
-                std::vector<int>& next = pos;  // level starts, consumed
-                next.assign(level.begin(), level.end());
-                for (int i = 0; i < m; ++i) at[i] = next[height[i]]++, order[at[i]] = i;
-            }
-            const size_t base = zp.recs.size();
-            zp.recs.resize(base + 4 * size_t(m) + (m + 1) + (H + 2) + m);
-            int* out = zp.recs.data() + base;
-            int items = 0;
-            for (int q = 0; q < m; ++q) {
-                const int i = order[q];
-                const int* r = rec + 6 * i;
-                const int x = r[0] / n, y = r[0] % n;
-                int nchild = 0, children = 0;
-                for (int j = 0; j < 3 && r[3 + j] != -1; ++j, ++nchild) children |= (at[r[3 + j] / 6] + 1) << (10 * j);
-                out[4 * q] = x | y << 16;
-                out[4 * q + 1] = (r[1] + 1) | (r[2] + 1) << 8 | nchild << 16;
-                out[4 * q + 2] = i ? at[parent[i] & 0xFFFF] | (parent[i] >> 16) << 16 : 0;
-                out[4 * q + 3] = children;
-                out[4 * m + q] = items;
-                if (i) {
-                    const int pp = rec[6 * (parent[i] & 0xFFFF)], px = pp / n, py = pp % n;
-                    items += px == x || py == y ? 1 : std::abs(px - x) + std::abs(py - y);
-                }
-            }
-            out[5 * m] = items;
-            std::copy(level.begin(), level.end(), out + 5 * m + 1);
-            for (int i = 0; i < m; ++i) out[5 * m + 1 + H + 2 + i] = at[i];
-            zp.desc.push_back(make_int4(int(base), m, H, raw_cap[begin + k]));
-            zp.ids.push_back(net_ids[begin + k]);
-            ++zb.fast;
-            zb.fast_nmax = std::max(zb.fast_nmax, m);
-        }
+        for (int i = 1; i < m; ++i)
+            if (parent[i] < 0) return false;
+        height_of_root = height[0];
+        return true;
     }
-    return zp;
-}
+    static size_t words(int m, int H) { return 4 * size_t(m) + (m + 1) + (H + 2) + m; }
+    // Into out[0 .. words(m, height_of_root)); n: side of the map the record's
+    // positions index.
+    void write(int n, const int* rec, int* out) const {
+        rec += 2;
+        const int H = height_of_root;
+        int level[kZnetMaxNodes + 1], next[kZnetMaxNodes + 1], at[kZnetMaxNodes], order[kZnetMaxNodes];
+        std::fill(level, level + H + 2, 0);
+        for (int i = 0; i < m; ++i) ++level[height[i] + 1];
+        for (int h = 0; h <= H; ++h) level[h + 1] += level[h];
+        std::copy(level, level + H + 2, next);
+        for (int i = 0; i < m; ++i) at[i] = next[height[i]]++, order[at[i]] = i;
+        int items = 0;
+        for (int q = 0; q < m; ++q) {
+            const int i = order[q];
+            const int* r = rec + 6 * i;
+            const int x = r[0] / n, y = r[0] % n;
+            int nchild = 0, children = 0;
+            for (int j = 0; j < 3 && r[3 + j] != -1; ++j, ++nchild) children |= (at[r[3 + j] / 6] + 1) << (10 * j);
+            out[4 * q] = x | y << 16;
+            out[4 * q + 1] = (r[1] + 1) | (r[2] + 1) << 8 | nchild << 16;
+            out[4 * q + 2] = i ? at[parent[i] & 0xFFFF] | (parent[i] >> 16) << 16 : 0;
+            out[4 * q + 3] = children;
+            out[4 * m + q] = items;
+            if (i) {
+                const int pp = rec[6 * (parent[i] & 0xFFFF)], px = pp / n, py = pp % n;
+                items += px == x || py == y ? 1 : std::abs(px - x) + std::abs(py - y);
+            }
+        }
+        out[5 * m] = items;
+        std::copy(level, level + H + 2, out + 5 * m + 1);
+        std::copy(at, at + m, out + 5 * m + 1 + H + 2);
+    }
+};
 
 // The level order of slots [begin, begin + count) for the soft passes.
 void ensure_soft_levels(gr_ctx* c, int begin, int count, int nodes) {
@@ -2124,15 +2100,29 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
         const int nets = batch_off[nbatch];
         const long long words = rec_off[nbatch];
         if ((nets && (!net_ids || !raw_cap)) || (words && !records)) throw GrError(GR_E_ARG, "null argument");
-        long long max_raw = 1;
-        // every index the kernels derive from the plan is checked here
-        for (int b = 0; b < nbatch; ++b) {
+        for (int b = 0; b < nbatch; ++b)
+            if (batch_off[b + 1] < batch_off[b] || rec_off[b + 1] < rec_off[b] + (batch_off[b + 1] - batch_off[b]))
+                throw GrError(GR_E_ARG, "batch offsets out of order");
+        // Batch by batch on the host's threads where there are nets enough to
+        // pay for starting them: every index the kernels derive from the plan is
+        // checked, and each net's form chosen ({nodes, root height}, nodes 0:
+        // general).  On one thread, into growing arrays, the nets' own records
+        // took 65 of 75 ms of an upload of 383k nets.
+        const bool threads = nets >= 4096;
+        auto each_batch = [&](auto&& f) {
+            if (threads) parallel_tasks(nbatch, f);
+            else
+                for (int b = 0; b < nbatch; ++b) f(b);
+        };
+        std::vector<int2> form(nets);
+        std::vector<long long> raw_words(nbatch, 0);
+        each_batch([&](int b) {
             const int begin = batch_off[b], count = batch_off[b + 1] - begin;
             const long long r0 = rec_off[b], r1 = rec_off[b + 1];
-            if (count < 0 || r1 < r0 + count) throw GrError(GR_E_ARG, "batch offsets out of order");
             long long raw = 0;
             for (int k = 0; k < count; ++k) raw += raw_cap[begin + k];
-            max_raw = std::max(max_raw, raw);
+            raw_words[b] = raw;
+            ZnetTree tree;
             for (int k = 0; k < count; ++k) {
                 const int id = net_ids[begin + k];
                 if (id < 0 || id >= c->net_count) throw GrError(GR_E_ARG, "net id outside route storage");
@@ -2153,31 +2143,80 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
                         if (r[j] != -1 && (r[j] < 6 * (i + 1) || r[j] >= 6 * nodes || r[j] % 6))
                             throw GrError(GR_E_ARG, "child record must follow its parent in preorder");
                 }
+                form[begin + k] = tree.read(L, rec) ? make_int2(nodes, tree.height_of_root) : make_int2(0, 0);
             }
+        });
+        // The nets' places: per batch its nets with the DP in LDS (descriptor,
+        // subnet, record) and the positions of the others, whose batches' plan
+        // records cross too.
+        std::vector<gr_ctx::ZBatch> split(nbatch);
+        std::vector<long long> dev_rec_off(nbatch + 1, 0);
+        std::vector<int4> desc;
+        std::vector<int> ids, list;
+        desc.reserve(nets), ids.reserve(nets);
+        size_t own_words = 0;
+        long long max_raw = 1;
+        for (int b = 0; b < nbatch; ++b) {
+            gr_ctx::ZBatch& zb = split[b];
+            zb = {int(desc.size()), 0, 1, int(list.size()), 0};
+            const int begin = batch_off[b];
+            for (int j = begin; j < batch_off[b + 1]; ++j) {
+                const int m = form[j].x, H = form[j].y;
+                if (m && own_words < size_t(INT32_MAX / 2)) {
+                    desc.push_back(make_int4(int(own_words), m, H, raw_cap[j]));
+                    ids.push_back(net_ids[j]);
+                    own_words += ZnetTree::words(m, H);
+                    ++zb.fast;
+                    zb.fast_nmax = std::max(zb.fast_nmax, m);
+                } else {
+                    form[j].x = 0;
+                    list.push_back(j - begin);
+                    ++zb.slow;
+                }
+            }
+            dev_rec_off[b + 1] = dev_rec_off[b] + (zb.slow ? rec_off[b + 1] - rec_off[b] : 0);
+            if (zb.slow) max_raw = std::max(max_raw, raw_words[b]);
         }
-        ZnetPlan zp = plan_znets(g, n, nbatch, batch_off, net_ids, rec_off, records, raw_cap);
+        const std::unique_ptr<int[]> own(new int[std::max<size_t>(own_words, 1)]);
+        each_batch([&](int b) {
+            ZnetTree tree;
+            const int4* d = desc.data() + split[b].fast_off;
+            for (int j = batch_off[b]; j < batch_off[b + 1]; ++j) {
+                if (!form[j].x) continue;
+                const int* rec = records + rec_off[b] + records[rec_off[b] + (j - batch_off[b])];
+                tree.read(L, rec);
+                tree.write(n, rec, own.get() + (d++)->x);
+            }
+        });
+        c->z_batches = 0;  // nothing to run until every array is in place
         c->z_ws.carve([&](auto& cv) {
             c->z_net_ids = cv.template take<int>(nets);
-            c->z_records = cv.template take<int>(words);
+            c->z_records = cv.template take<int>(size_t(dev_rec_off[nbatch]));
             c->z_raw_cap = cv.template take<int>(nets);
             c->z_raw = cv.template take<int>(max_raw);
-            c->z_desc = cv.template take<int4>(zp.desc.size());
-            c->z_fast_ids = cv.template take<int>(zp.ids.size());
-            c->z_recs = cv.template take<int>(zp.recs.size());
-            c->z_list = cv.template take<int>(zp.list.size());
+            c->z_desc = cv.template take<int4>(desc.size());
+            c->z_fast_ids = cv.template take<int>(ids.size());
+            c->z_recs = cv.template take<int>(own_words);
+            c->z_list = cv.template take<int>(list.size());
         });
-        if (!zp.desc.empty()) {
-            upload(c->z_desc, zp.desc.data(), sizeof(int4) * zp.desc.size(), c->stream);
-            upload(c->z_fast_ids, zp.ids.data(), sizeof(int) * zp.ids.size(), c->stream);
-            upload(c->z_recs, zp.recs.data(), sizeof(int) * zp.recs.size(), c->stream);
+        if (!desc.empty()) {
+            upload(c->z_desc, desc.data(), sizeof(int4) * desc.size(), c->stream);
+            upload(c->z_fast_ids, ids.data(), sizeof(int) * ids.size(), c->stream);
+            upload(c->z_recs, own.get(), sizeof(int) * own_words, c->stream);
         }
-        if (!zp.list.empty()) upload(c->z_list, zp.list.data(), sizeof(int) * zp.list.size(), c->stream);
-        c->z_split = std::move(zp.split);
+        if (!list.empty()) upload(c->z_list, list.data(), sizeof(int) * list.size(), c->stream);
         if (nets) {
             upload(c->z_net_ids, net_ids, sizeof(int) * nets, c->stream);
             upload(c->z_raw_cap, raw_cap, sizeof(int) * nets, c->stream);
         }
-        if (words) upload(c->z_records, records, sizeof(int) * words, c->stream);
+        for (int b = 0; b < nbatch;) {  // runs of batches with general nets lie together on both sides
+            int e = b + 1;
+            if (split[b].slow) {
+                while (e < nbatch && split[e].slow) ++e;
+                upload(c->z_records + dev_rec_off[b], records + rec_off[b], sizeof(int) * (rec_off[e] - rec_off[b]), c->stream);
+            }
+            b = e;
+        }
         const long long plane = (long long)(L + 1) * nn;
         if (plane != c->z_plane) {
             c->mem.release(c->z_map);
@@ -2188,10 +2227,11 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
             hip_check(hipMemsetAsync(c->z_prev, 0, sizeof(int) * 16 * plane, c->stream), "clear Z-shape map");
             c->z_plane = plane;
         }
-        c->z_batches = nbatch;
+        c->z_split = std::move(split);
         c->z_batch_off.assign(batch_off, batch_off + nbatch + 1);
-        c->z_rec_off.assign(rec_off, rec_off + nbatch + 1);
+        c->z_rec_off = std::move(dev_rec_off);
         hip_check(hipStreamSynchronize(c->stream), "Z-shape upload");
+        c->z_batches = nbatch;
     });
 }
 

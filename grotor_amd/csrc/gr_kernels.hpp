@@ -208,12 +208,14 @@ __global__ void zshape_reset_kernel(ZshapeArgs a);
 __global__ void zshape_solve_kernel(ZshapeArgs a);
 __global__ void zshape_convert_kernel(ZshapeArgs a, const int* net_ids, RouteStore rs);
 
-// Nets routed with their DP in LDS (zshape_net_kernel): trees of at most
-// kZnetMaxNodes nodes whose tables take at most kZnetLds bytes, every node at
-// a place of its own, child slots filled from the first.
+// Nets routed with their DP in LDS (zshape_net_kernel): trees whose tables take
+// at most kZnetLds bytes (at least 116 a node), every node at a place of its
+// own, child slots filled from the first.  kZnetMaxNodes bounds the trees the
+// bytes admit; node numbers plus one take 10 bits in the records.
 constexpr int kZnetThreads = 256;
 constexpr int kZnetMaxNodes = 512;
 constexpr size_t kZnetLds = 48 * 1024;
+static_assert(kZnetLds / 116 < kZnetMaxNodes && kZnetMaxNodes < 1023);
 struct ZnetArgs {
     DeviceGrid g;
     const double* presum;
