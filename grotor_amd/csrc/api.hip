@@ -601,6 +601,7 @@ CommitArgs commit_args(gr_ctx* c, int begin, int count, int stamp, int K) {
     return a;
 }
 
+constexpr int kFusedCommitNets = 2048;   // batches of fewer nets commit their wires in the DP (gr_lshape_run)
 constexpr int kCommitPackedNets = 4096;  // batches of at least this many nets commit four nets per wavefront
 
 // Commit (K = 1) or removal (K = -1) of stage slots [begin, begin + count):
@@ -1735,20 +1736,21 @@ int gr_lshape_run(gr_ctx* c, int nbatch, const int* batch_off, int first_stamp, 
             if (mode == 2 && nbatch)  // a kernel, not a memset: the loop may be captured
                 hipLaunchKernelGGL(fill_int_kernel, dim3(unsigned((nbatch * qwords + 255) / 256)), dim3(256), 0,
                                    c->stream, c->dp_queue, 0, nbatch * qwords);
-            // The DP launches of a batch below kCommitPackedNets nets commit its
-            // wires: there the commit's own launch costs more than its work (64x64x5,
-            // 92 nets a batch: loop 0.91 -> 0.81 ms; 131x131x5, 510 a batch,
-            // plain form 1.84 -> 1.70).  Larger batches keep the launch of four nets
-            // per wavefront, whose lanes share a net's cells (590k nets, 9.7k a batch:
-            // 8.30 ms with it everywhere, 8.44 without it).  Profiled runs keep
-            // it too, so that each launch is timed alone.
+            // The DP launches of a batch below kFusedCommitNets nets commit its
+            // wires: there the commit's own launch costs more than it gains (64x64x5,
+            // 92 nets a batch: loop 0.91 -> 0.81 ms; 131x131x5, 510 a batch, plain
+            // form 1.84 -> 1.70).  Over two-pin nets with legs of 2 to 1000 cells
+            // a batch of 1 to 2000 takes 2 to 40 us less, one of 4000 as much or
+            // up to 2.5 % more (legs of 10 cells: 129.6 -> 126.9 us at 2000, 150.8
+            // -> 154.5 at 4000), one of 9.7k more (590k nets: 8.30 -> 8.44 ms).
+            // Profiled runs keep the launch, so that it is timed alone.
             struct Wires {
                 gr_ctx* c;
                 ~Wires() { c->dp_wires = WireCommit{}; }
             } wires{c};
             for (int b = 0; b < nbatch; ++b) {
                 const int count = batch_off[b + 1] - batch_off[b];
-                const bool fused = !c->profiling && count < kCommitPackedNets;
+                const bool fused = !c->profiling && count < kFusedCommitNets;
                 launch_refresh(c, 0);
                 c->dp_wires = WireCommit{};
                 if (fused)

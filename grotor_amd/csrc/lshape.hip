@@ -340,43 +340,43 @@ __device__ __forceinline__ void root_merge(double& m, int& ch) {
 // costs, which only the next refresh changes, so their demand can go up while
 // others are still being solved, and the vias' launch, which needs every
 // wire timestamp of the batch, follows as before.  One lane per wire (a node's
-// edge has one or two); its unit edges are additions and stores nothing waits
-// for.  The lengths come as a difference of prefix sums, one load at each
-// end.  Used for the batches whose commit is all launch (gr_lshape_run has the
-// rule and both sides' times).
+// edge has one or two), long wires shared by the net's lanes (commit_cells).
+// The lengths come as a difference of prefix sums, one load at each end.
+// gr_lshape_run has the rule for its use and both sides' times.
 template <int L>
 __device__ __forceinline__ void commit_net_wires(const LshapeArgs& a, const Tables<L>& s, int n, int lane, int W) {
     const DeviceGrid& g = a.g;
     const WireCommit& c = a.wires;
     long long length = 0;
     int edges = 0;
-    for (int t = lane + 2; t < 2 * n; t += W) {  // the root has no edge
-        const int i = t >> 1, second = t & 1;
-        const int v = s.xy[i], q = s.xy[s.par[i]];
-        const int x = v >> 16, y = v & 0xFFFF, px = q >> 16, py = q & 0xFFFF;
-        const int cl = s.path[i] / L % L, pl = s.path[i] % L;
-        const bool straight = x == px || y == py;
-        if (straight && second) continue;
-        const int l = second ? pl : cl;
-        const bool along_y = straight ? x == px : (layer_dir(g, cl) != 0) != (second != 0);
-        const int fixed = along_y ? (second ? px : x) : (second ? py : y);
-        const int lo = along_y ? min(y, py) : min(x, px), hi = along_y ? max(y, py) : max(x, px);
-        const int c0 = along_y ? cell_of(g, l, fixed, lo) : cell_of(g, l, lo, fixed);
-        const bool one_track = along_y == (layer_dir(g, l) != 0);
-        const int step = one_track ? 1 : (along_y ? g.X : g.Y);
-        c.timestamp[c0] = c.stamp;
-        c.timestamp[along_y ? cell_of(g, l, fixed, hi) : cell_of(g, l, hi, fixed)] = c.stamp;
-        if (lo == hi) continue;
-        if (one_track) c.track_dirty[track_of_cell(g, c0)] = 1u;
-        for (int d = 0; d < hi - lo; ++d) {
-            const int cell = c0 + d * step;
-            atomicAdd(c.demand + cell, 1.0f);
-            c.timestamp[cell] = c.stamp;
-            if (!one_track) c.track_dirty[track_of_cell(g, cell)] = 1u;
+    for (int t0 = 2; t0 < 2 * n; t0 += W) {  // the root has no edge
+        const int t = t0 + lane;
+        int c0 = 0, step = 0, len = 0;
+        bool one_track = false;
+        if (t < 2 * n) {
+            const int i = t >> 1, second = t & 1;
+            const int v = s.xy[i], q = s.xy[s.par[i]];
+            const int x = v >> 16, y = v & 0xFFFF, px = q >> 16, py = q & 0xFFFF;
+            const int cl = s.path[i] / L % L, pl = s.path[i] % L;
+            const bool straight = x == px || y == py;
+            if (!straight || !second) {
+                const int l = second ? pl : cl;
+                const bool along_y = straight ? x == px : (layer_dir(g, cl) != 0) != (second != 0);
+                const int fixed = along_y ? (second ? px : x) : (second ? py : y);
+                const int lo = along_y ? min(y, py) : min(x, px), hi = along_y ? max(y, py) : max(x, px);
+                c0 = along_y ? cell_of(g, l, fixed, lo) : cell_of(g, l, lo, fixed);
+                one_track = along_y == (layer_dir(g, l) != 0);
+                step = one_track ? 1 : (along_y ? g.X : g.Y);
+                len = hi - lo;
+                c.timestamp[c0] = c.stamp;
+                c.timestamp[along_y ? cell_of(g, l, fixed, hi) : cell_of(g, l, hi, fixed)] = c.stamp;
+                if (len && one_track) c.track_dirty[track_of_cell(g, c0)] = 1u;
+                const long long* sum = along_y ? c.y_len_sum : c.x_len_sum;
+                length += sum[hi] - sum[lo];
+                edges += len;
+            }
         }
-        const long long* sum = along_y ? c.y_len_sum : c.x_len_sum;
-        length += sum[hi] - sum[lo];
-        edges += hi - lo;
+        commit_cells(g, c, c0, step, one_track, len, lane, W);
     }
     for (int o = W / 2; o; o >>= 1) {
         length += __shfl_xor(length, o, kWave);

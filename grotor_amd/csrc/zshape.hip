@@ -785,7 +785,7 @@ namespace {
 // The wires among a net's `pairs` route pairs committed by its workgroup (what
 // commit_wires_kernel adds at K = 1): a batch's nets have their costs from the
 // refresh before it, so their demand can go up while others are being solved.
-// One lane per pair; its unit edges are additions and stores nothing waits for.
+// One lane per pair, long wires shared by the wavefront (commit_cells).
 // It saves the commit's launch, 6 us of a batch whose DP takes 23 (136
 // batches: loop 5.33 -> 4.84 ms).
 __device__ __forceinline__ void commit_words(const ZnetArgs& a, const int* out, int pairs) {
@@ -793,36 +793,37 @@ __device__ __forceinline__ void commit_words(const ZnetArgs& a, const int* out, 
     const WireCommit& c = a.wires;
     long long length = 0;
     int edges = 0;
-    for (int t = threadIdx.x; t < pairs; t += kZnetThreads) {
-        const int ra = out[1 + 2 * t], rb = out[2 + 2 * t];
+    const int lane = threadIdx.x % kWave;
+    for (int t0 = threadIdx.x - lane; t0 < pairs; t0 += kZnetThreads) {
+        const int t = t0 + lane;
+        int c0 = 0, step = 0, len = 0;
+        bool one_track = false;
+        const int ra = t < pairs ? out[1 + 2 * t] : 0, rb = t < pairs ? out[2 + 2 * t] : 0;
         const int l = ra / g.XY;
-        if (l != rb / g.XY) continue;
-        const int x0 = ra / g.Y % g.X, y0 = ra % g.Y, x1 = rb / g.Y % g.X, y1 = rb % g.Y;
-        const bool along_y = x0 == x1;
-        const int lo = along_y ? min(y0, y1) : min(x0, x1), hi = along_y ? max(y0, y1) : max(x0, x1);
-        const int c0 = along_y ? cell_of(g, l, x0, lo) : cell_of(g, l, lo, y0);
-        const bool one_track = along_y == (layer_dir(g, l) != 0);
-        const int step = one_track ? 1 : (along_y ? g.X : g.Y);
-        c.timestamp[cell_of(g, l, x0, y0)] = c.stamp;
-        c.timestamp[cell_of(g, l, x1, y1)] = c.stamp;
-        if (one_track && lo < hi) c.track_dirty[track_of_cell(g, c0)] = 1u;
-        for (int d = 0; d < hi - lo; ++d) {
-            const int cell = c0 + d * step;
-            atomicAdd(c.demand + cell, 1.0f);
-            c.timestamp[cell] = c.stamp;
-            if (!one_track) c.track_dirty[track_of_cell(g, cell)] = 1u;
+        if (t < pairs && l == rb / g.XY) {
+            const int x0 = ra / g.Y % g.X, y0 = ra % g.Y, x1 = rb / g.Y % g.X, y1 = rb % g.Y;
+            const bool along_y = x0 == x1;
+            const int lo = along_y ? min(y0, y1) : min(x0, x1), hi = along_y ? max(y0, y1) : max(x0, x1);
+            c0 = along_y ? cell_of(g, l, x0, lo) : cell_of(g, l, lo, y0);
+            one_track = along_y == (layer_dir(g, l) != 0);
+            step = one_track ? 1 : (along_y ? g.X : g.Y);
+            len = hi - lo;
+            c.timestamp[cell_of(g, l, x0, y0)] = c.stamp;
+            c.timestamp[cell_of(g, l, x1, y1)] = c.stamp;
+            if (one_track && len) c.track_dirty[track_of_cell(g, c0)] = 1u;
+            const long long* sum = along_y ? c.y_len_sum : c.x_len_sum;
+            length += sum[hi] - sum[lo];
+            edges += len;
         }
-        const long long* sum = along_y ? c.y_len_sum : c.x_len_sum;
-        length += sum[hi] - sum[lo];
-        edges += hi - lo;
+        commit_cells(g, c, c0, step, one_track, len, lane, kWave);
     }
     for (int o = kWave / 2; o; o >>= 1) {
         length += __shfl_xor(length, o, kWave);
         edges += __shfl_xor(edges, o, kWave);
     }
     Stats* st = c.stats + blockIdx.x % kStatStripes;
-    if (threadIdx.x % kWave == 0 && length) atomicAdd(&st->total_wirelength, double(length));
-    if (threadIdx.x % kWave == 0 && edges) atomicAdd(&st->wire_edges, (unsigned long long)edges);
+    if (lane == 0 && length) atomicAdd(&st->total_wirelength, double(length));
+    if (lane == 0 && edges) atomicAdd(&st->wire_edges, (unsigned long long)edges);
 }
 
 }  // namespace

@@ -482,3 +482,31 @@ def test_captured_loop_follows_the_cost_parameters(ga, ora):
         assert np.array_equal(run(ctx), want)
     ctx.close()
     fresh.close()
+
+
+def test_long_wires_do_not_hold_a_small_batch(ga):
+    """A batch of one net commits a wire of 8,000 cells in little more time
+    than one of 80: no lane walks a wire alone (8,000 steps of one lane took five
+    times the whole batch)."""
+    L, X, Y, nb = 2, 8192, 16, 24
+    t = dict(L=L, X=X, Y=Y, DIR=0, unit_length_wire_cost=0.01, unit_via_cost=4.0,
+             unit_length_short_costs=np.ones(L), x_edge_len=np.full(X - 1, 30, np.int32),
+             y_edge_len=np.full(Y - 1, 30, np.int32), capacity=np.full(L * X * Y, 8, np.float32))
+    times = {}
+    for length in (80, 8000):
+        ctx = ga.Context(t)
+        off = (np.arange(nb + 1) * 2).astype(np.int32)
+        ctx.set_routes(off)
+        nodes = np.array([x * Y + k % Y for k in range(nb) for x in (5, 5 + length)], np.int32)
+        ctx.lshape_upload(np.arange(nb), off, nodes, np.tile([-1, 0], nb).astype(np.int32))
+        runs = []
+        for r in range(12):
+            print(f"wire of {length} cells, run {r}", flush=True)
+            ctx.reset()
+            ctx.refresh()
+            runs.append(ctx.lshape_run(np.arange(nb + 1, dtype=np.int32), 1, 2))
+        times[length] = min(runs)
+        assert ctx.demand().sum() == nb * length
+        assert ctx.stats() == (30.0 * nb * length, 0)
+        ctx.close()
+    assert times[8000] < 2 * times[80], times
