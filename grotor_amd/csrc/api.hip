@@ -10,7 +10,6 @@
 #include <atomic>
 #include <memory>
 #include <mutex>
-#include <thread>
 #include <cstring>
 #include <stdexcept>
 #include <string>
@@ -18,6 +17,7 @@
 
 #include "../../include/grotor_amd.h"
 #include "gr_kernels.hpp"
+#include "gr_parallel.hpp"
 #include "gr_status.hpp"
 
 using namespace grotor;
@@ -673,67 +673,6 @@ BatchLaunch plan_batch(gr_ctx* c, int begin, int count, std::vector<int>& slots)
     for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
     for (int s = begin; s < begin + count; ++s) slots[begin + at[bucket(s, c->node_off_h[s + 1] - c->node_off_h[s])]++] = s;
     return b;
-}
-
-// f(k) for k in [0, n) on up to 16 host threads (chunks of 256 items);
-// the first exception thrown by any item is rethrown once all have stopped.
-template <class F>
-void parallel_items(int n, F&& f) {
-    const int threads = std::max(1, std::min<int>(16, int(std::thread::hardware_concurrency())));
-    if (n < 4096 || threads == 1) {
-        for (int k = 0; k < n; ++k) f(k);
-        return;
-    }
-    std::atomic<int> next{0};
-    std::atomic<bool> failed{false};
-    std::exception_ptr error;
-    std::mutex m;
-    auto work = [&] {
-        try {
-            while (!failed.load(std::memory_order_relaxed)) {
-                const int k0 = next.fetch_add(256);
-                if (k0 >= n) return;
-                for (int k = k0; k < std::min(n, k0 + 256); ++k) f(k);
-            }
-        } catch (...) {
-            std::lock_guard<std::mutex> lock(m);
-            if (!error) error = std::current_exception();
-            failed = true;
-        }
-    };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < threads; ++t) pool.emplace_back(work);
-    work();
-    for (auto& t : pool) t.join();
-    if (error) std::rethrow_exception(error);
-}
-
-// f(0) .. f(n - 1) for a few heavy items, one at a time per thread.
-template <class F>
-void parallel_tasks(int n, F&& f) {
-    const int threads = std::max(1, std::min<int>({16, n, int(std::thread::hardware_concurrency())}));
-    if (threads <= 1) {
-        for (int k = 0; k < n; ++k) f(k);
-        return;
-    }
-    std::atomic<int> next{0};
-    std::atomic<bool> failed{false};
-    std::exception_ptr error;
-    std::mutex m;
-    auto work = [&] {
-        try {
-            for (int k = next++; k < n && !failed.load(std::memory_order_relaxed); k = next++) f(k);
-        } catch (...) {
-            std::lock_guard<std::mutex> lock(m);
-            if (!error) error = std::current_exception();
-            failed = true;
-        }
-    };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < threads; ++t) pool.emplace_back(work);
-    work();
-    for (auto& t : pool) t.join();
-    if (error) std::rethrow_exception(error);
 }
 
 constexpr size_t kLdsLimit = 64 * 1024;
