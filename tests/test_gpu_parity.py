@@ -510,3 +510,43 @@ def test_long_wires_do_not_hold_a_small_batch(ga):
         assert ctx.stats() == (30.0 * nb * length, 0)
         ctx.close()
     assert times[8000] < 2 * times[80], times
+
+
+def test_stage_runs_between_other_launches_of_its_slots(ga, ora):
+    """gr_lshape_run keeps its launch plan while what it is made of stays:
+    single batches (with and without allocation), other tiny-tree bounds, other
+    batch offsets, tuners and new route storage in between, every mode, give
+    the oracle's stage each time."""
+    _, t = topology(6, 3)
+    color, nb = ora.batches(t["X"], t["Y"], t["pt_off"], t["pts"], t["hs_off"], t["hsegs"], t["vs_off"], t["vsegs"])
+    sched = ga.execution_schedule(t, color, nb)
+    bo = sched["batch_off"]
+    coarse = np.array([bo[0], bo[len(bo) // 2], bo[-1]], np.int32)  # the nets in two batches
+    want = ora.Grid(t).lshape_stage(sched, t["pin_acc_num"], threads=8)
+    want_coarse = ora.Grid(t).lshape_stage(dict(sched, batch_off=coarse), t["pin_acc_num"], threads=8)
+    ctx = ga.Context(t)
+    ctx.set_routes(t["pin_acc_num"])
+    ctx.lshape_upload(sched["net_ids"], sched["node_off"], sched["nodes"], sched["parents"])
+
+    def check(mode, off=bo, expect=want):
+        ctx.reset()
+        ctx.lshape_run(off, 1, mode)
+        routes_o, demand_o, ts_o, wl_o, vias_o = expect
+        assert np.array_equal(ctx.routes(), routes_o)
+        assert np.array_equal(_bits(ctx.demand()), _bits(demand_o))
+        assert np.array_equal(ctx.timestamps(), ts_o)
+        assert ctx.stats() == (wl_o, vias_o)
+
+    begin, count = int(bo[2]), int(bo[7] - bo[2])
+    between = [lambda: ctx.lshape_batch(begin, count, 1), lambda: ctx.lshape_batch_noalloc(begin, count, 1),
+               lambda: ctx.set_tiny_tree(8), lambda: ctx.set_tiny_tree(1), lambda: ctx.lshape_tune(bo),
+               lambda: ctx.lshape_tune_groups(bo), lambda: check(1, coarse, want_coarse),
+               lambda: ctx.set_routes(t["pin_acc_num"]), lambda: None]
+    for k, step in enumerate(between):
+        for mode in (2, 1, 0):
+            print(f"step {k} mode {mode}", flush=True)
+            check(mode)
+            ctx.refresh()
+            step()
+            check(mode)
+    ctx.close()

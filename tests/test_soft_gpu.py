@@ -214,3 +214,84 @@ def test_soft_trees_of_every_form_match_oracle(ga, ora, L, X, Y, kind):
     total, _, _ = ctx.soft_forward_costs(0, n, w, v, 0.5, 64)
     assert abs(total - want) <= 1e-10 * max(1.0, abs(want))
     ctx.close()
+
+
+def _many_trees(rng, L, X, Y, nets, tall):
+    """`nets` small trees in boxes of at most 14 x 14 cells and, next to each
+    other in the middle, `tall` chains of 300 nodes: (node_off, nodes,
+    parents)."""
+    sizes = rng.choice([1, 2, 2, 3, 4, 7, 12], nets)
+    sizes[nets // 2:nets // 2 + tall] = 300
+    off, nodes, parents = [0], [], []
+    for n in sizes:
+        ox, oy = rng.integers(0, X - 14), rng.integers(0, Y - 14)
+        x, y = ox + rng.integers(0, 14, n), oy + rng.integers(0, 14, n)
+        par = [-1] + [int(rng.integers(0, i)) for i in range(1, n)]
+        if n == 300:
+            x, y, par = ox + np.arange(n) % 3, oy + np.arange(n) // 2 % 14, list(range(-1, n - 1))
+        straight = rng.random(n) < 0.2
+        x = np.where(straight, x[0], x)
+        layer = np.where(rng.random(n) < 0.5, L, rng.integers(0, L, n))
+        nodes += ((layer * X + x) * Y + y).tolist()
+        parents += par
+        off.append(len(nodes))
+    return np.array(off, np.int32), np.array(nodes, np.int32), np.array(parents, np.int32)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("L,X,Y", [(4, 101, 87), (9, 70, 61)])
+def test_soft_chunks_of_several_nets_match_oracle(ga, ora, L, X, Y, kind):
+    """More nets than four times the compute units, so that a workgroup takes
+    several (5 of 5,203 on 256 units, the last chunk fewer), three chains taller
+    than the level bins in one chunk, on a grid whose arrays change their order
+    on the device: values, per-cell gradients and given costs against the
+    oracle, binary64 closely and binary32 within its rounding: a weight is
+    a product over the levels of some eight factors exp(-(x - y) / tau), each
+    off by two half units in the last place of a table entry, which on a net's
+    routes of any weight is at most the net's value plus 30 tau."""
+    rng = np.random.default_rng(10 * L + kind)
+    n, tall, tau = 5203, 3, 1.0
+    off, nodes, parents = _many_trees(rng, L, X, Y, n, tall)
+    t = dict(L=L, X=X, Y=Y, DIR=L & 1, unit_length_wire_cost=0.01, unit_via_cost=0.5,
+             unit_length_short_costs=np.full(L, 0.3), x_edge_len=np.full(X - 1, 30, np.int32),
+             y_edge_len=np.full(Y - 1, 30, np.int32), capacity=rng.integers(1, 6, L * X * Y).astype(np.float32))
+    assert L * X * Y >= 32768
+    demand = random_demand(t, 3, high=4)
+    ctx = ga.Context(t)
+    ctx.set_routes(off)
+    ctx.lshape_upload(np.arange(n), off, nodes, parents)
+    ctx.upload_demand(demand)
+    ctx.set_soft_kind(kind)
+    grid = ora.Grid(t)
+    print(f"soft chunks L={L} kind={kind}", flush=True)
+    # every net in binary64; the nets before the chains in both
+    for begin, count, precisions in ((0, n, (64,)), (3, n // 2 - 5, (64, 32))):
+        end = begin + count
+        o = off[begin:end + 1] - off[begin]
+        part = slice(off[begin], off[end])
+        F_o, gw_o, gv_o, gp_o = grid.soft_stage(demand, o, nodes[part], parents[part], tau, *THETA, grads=True, kind=kind)
+        for precision in precisions:
+            total, per_net, _ = ctx.soft_forward(begin, count, *THETA, tau=tau, precision=precision, per_net=True)
+            gp, _ = ctx.soft_backward()
+            gw, gv = ctx.soft_edge_grads()
+            if precision == 64:
+                values = per_net
+                rel, rtol, atol = 1e-10, 1e-8, 1e-10
+            else:
+                levels = 12  # a tree of at most 12 nodes
+                rel = 8 * levels * 2.0 ** -24
+                rtol, atol = levels * 8 * 2 * 2.0 ** -24 * (np.abs(values).max() + 30 * tau) / tau, 1e-10
+                assert rtol < 0.01
+                assert np.allclose(per_net, values, rtol=rel, atol=rel)
+            assert abs(total - F_o) <= rel * abs(F_o)
+            assert np.allclose(gw, gw_o, rtol=rtol, atol=atol) and np.allclose(gv, gv_o, rtol=rtol, atol=atol)
+            assert np.allclose(gp, gp_o, rtol=rtol, atol=atol)
+            print(f"binary{precision} largest difference", np.abs(gw - gw_o).max(), np.abs(gv - gv_o).max(), flush=True)
+    w, v = rng.gamma(2.0, 0.3, L * X * Y), rng.gamma(2.0, 0.3, L * X * Y)
+    first = n // 2 - 20  # the chains among the nets before and after them
+    total, per_net, _ = ctx.soft_forward_costs(first, n - first, w, v, 0.5, 64, per_net=True)
+    for k in range(0, 60):
+        part = slice(off[first + k], off[first + k + 1])
+        want = grid.soft_net(w, v, nodes[part], parents[part], 0.5, kind=kind)
+        assert abs(per_net[k] - want) <= 1e-10 * max(1.0, abs(want))
+    ctx.close()
