@@ -237,8 +237,11 @@ struct gr_ctx {
     std::vector<int> slots_h;      // stage slot per execution position
     int4* desc = nullptr;          // per execution position: node begin, nodes, route word, route capacity
     std::vector<int4> desc_h;
-    // the last gr_lshape_run's launches, slots_h and descriptors, kept while
-    // what they are made of stays the same (contents, not addresses)
+    // the last gr_lshape_run's launches, slots_h and descriptors, kept while its
+    // key stays the same: the uploads of the stage and of the route storage
+    // (counted), plain form or not, the tiny-tree bound, the batch offsets.
+    // It serves repeated runs of one uploaded stage (a plan of 590k nets takes
+    // some 5 ms); every other writer of the descriptors clears it.
     std::vector<BatchLaunch> run_plan;
     std::vector<int> run_plan_key;
     int routes_gen = 0;  // counts the route stores
@@ -246,13 +249,13 @@ struct gr_ctx {
     size_t gscratch_bytes = 0;
     double* noalloc_scratch = nullptr;    // this device's `scratch` (gr_lshape_batch_noalloc)
     std::vector<int> noalloc_slots;       // sized at gr_lshape_upload
-    ReuseArena score_mem;  // gr_score: lines, per-cell counters, partial sums
+    ReuseArena score_mem;  // gr_score: lines, per-cell counters, partial sums (at most kKeptScratch)
     // exclusive prefix sums of the edge lengths, and the wire commit of the DP
     // launches being enqueued (demand null: none)
     long long *x_len_sum = nullptr, *y_len_sum = nullptr;
     WireCommit dp_wires{};
     // grid arrays on their way between IDX and track-major order, and the
-    // recomputed costs of gr_cost_download
+    // recomputed costs of gr_cost_download (at most kKeptScratch each)
     Workspace layout_ws, cost_ws;
     // rip-up
     int* of_sum = nullptr;

@@ -14,11 +14,12 @@
 // (:383-388): it is no routing layer, its wires are rejected and only its
 // vias are costed.
 //
-// score_nets_kernel, score_big_kernel: one wavefront per design net, its lines in the .out
-// order (metal-0 pin vias, extra routes, then every subnet's route pairs
-// shifted up one metal layer).  The stacking test of a via scans the net's
-// own lines (decoded once into LDS), so nets run in parallel with the
-// evaluator's sequential result.
+// score_nets_kernel, score_big_kernel: one wavefront per design net, its lines
+// in the .out order (metal-0 pin vias, extra routes, then every subnet's route
+// pairs shifted up one metal layer).  The stacking test of a via looks at the
+// net's own lines that share its track or place (decoded once into LDS and
+// chained by both; nets of more than kScoreLines lines scan theirs in global
+// memory), so nets run in parallel with the evaluator's sequential result.
 // score_cells_kernel: per cell the demand, loss and wirelength, summed per
 // layer in fixed-shape partial sums that the host adds in order.
 #include "gr_kernels.hpp"

@@ -211,10 +211,12 @@ int gr_commit_batch(gr_ctx *ctx, int begin, int count, int stamp, int K);
  *           workgroups drain the batch's nets from a device work queue,
  *           tallest trees first, tables in LDS; the whole loop captured once
  *           into a HIP graph and replayed (the capture is reused while the
- *           stage topology, batch offsets, first stamp and nets per wavefront
- *           stay the same; capture happens before the timed interval);
+ *           stage topology, batch offsets, first stamp, cost parameters and
+ *           nets per wavefront stay the same; capture happens before the timed
+ *           interval);
  *       other values are rejected with GR_E_ARG.  Results are identical in
- *       every mode.
+ *       every mode.  Batches of fewer than 2048 nets commit their wires inside
+ *       the DP launches (not while profiling, see gr_profile_begin).
  * *elapsed_ms receives the synchronized interval (RoutingDagTimer,
  * include/router_state.hpp:238-265). */
 int gr_lshape_run(gr_ctx *ctx, int nbatch, const int *batch_off, int first_stamp,
@@ -304,6 +306,10 @@ enum {
 /* Start timing every kernel launch of this context with HIP events on its
  * stream; gr_profile_end returns, per kernel class, the summed device time
  * (ms), the launch count and the algorithmic HBM bytes of those launches.
+ * While profiling, the L-shape and Z-shape stages commit every batch's wires
+ * in a launch of its own, so that the DP and the commit are timed apart; other
+ * runs commit the wires of L-shape batches of fewer than 2048 nets, and of
+ * Z-shape batches without large trees, inside the DP launch.
  * No reference counterpart (the reference prints stage wall times only). */
 int gr_profile_begin(gr_ctx *ctx);
 /* Restrict the events of gr_profile_begin to the kernel classes whose bit
