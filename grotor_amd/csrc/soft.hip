@@ -408,11 +408,12 @@ namespace {
 // ---- kind 1 edges on 16 lanes ----
 constexpr int kZGroup = 16;
 
-// Minimum / sum over a row of 16 lanes, the same in each of them.
+// Minimum / sum over a row of `lanes` lanes, the same in each of them.
 template <class R, class Op>
-__device__ __forceinline__ R row_reduce(R v, Op&& op) {
+__device__ __forceinline__ R row_reduce(R v, int lanes, Op&& op) {
 #pragma unroll
-    for (int o = 1; o < kZGroup; o <<= 1) v = op(v, __shfl_xor(v, o, kWave));
+    for (int o = 1; o < kWave; o <<= 1)
+        if (o < lanes) v = op(v, __shfl_xor(v, o, kWave));
     return v;
 }
 
@@ -494,11 +495,11 @@ __device__ __forceinline__ void bend_minima(const ZBend<L>& z, const R* best, R 
 }
 
 // The bends of one orientation (d1 = direction of the first leg) of an edge,
-// kZGroup at a time: the child's own row (column) and those strictly between.
+// `lanes` at a time: the child's own row (column) and those strictly between.
 template <int L, int P, class F>
-__device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, int d1, int lane, F&& f) {
+__device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, int d1, int lane, int lanes, F&& f) {
     const int from = d1 ? E.y : E.x, to = d1 ? E.py : E.px, n = abs(to - from);
-    for (int b0 = 0; b0 < n; b0 += kZGroup) {
+    for (int b0 = 0; b0 < n; b0 += lanes) {
         const int k = b0 + lane;
         const bool live = k < n;
         ZBend<L> z;
@@ -519,14 +520,18 @@ __device__ __forceinline__ void for_each_bend(const SoftArgs& a, const Edge& E, 
 // 8 and 4 lanes leave fewer idle on the usual box of 5 x 5 cells but make the
 // long edges the tail (forward over 188k nodes, 8 layers, binary32, tau =
 // 0.1: 0.66 ms at 16, 0.80 at 8, 0.97 at 4, one launch per level; 0.53 by
-// chunks; before, 1.33).
+// chunks; before, 1.33).  A level of no more edges than the workgroup has
+// wavefronts gives each a whole one: with 16 lanes a few long edges leave the
+// rest idle (8 chains of 8 nodes across 512 x 512 cells, binary64: 4.51 ms, 1.14
+// here, 3.66 with one wavefront per net).
 template <class R, int L>
-__device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* order, int count, int first, int groups) {
+__device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* order, int count) {
     const DeviceGrid& g = a.g;
     const R tau = R(a.tau);
-    const int lane = threadIdx.x % kZGroup;
+    const int lanes = count <= 256 / kWave ? kWave : kZGroup;
+    const int lane = threadIdx.x % lanes;
     const SoftTables<R> t = soft_tables<R>(a);
-    for (int k = first; k < count; k += groups) {
+    for (int k = threadIdx.x / lanes; k < count; k += 256 / lanes) {
         const int4 it = order[k];
         if (it.w < 0) continue;
         const SoftNode c = soft_node(g, a.nodes[it.x]), p = soft_node(g, a.nodes[it.y + it.w]);
@@ -549,7 +554,7 @@ __device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* or
         for (int l = 0; l < L; ++l) best[l] = bn[l], st[l] = lse_empty<R>();
         auto pass = [&](auto par, int d1) {
             constexpr int P = decltype(par)::value;
-            for_each_bend<L, P>(a, E, d1, lane, [&](const ZBend<L>& z, int, bool live, int) {
+            for_each_bend<L, P>(a, E, d1, lane, lanes, [&](const ZBend<L>& z, int, bool live, int) {
                 R f1[L], mv[L];
                 bend_minima<R, L, P>(z, best, tau, f1, mv);
 #pragma unroll
@@ -567,9 +572,9 @@ __device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* or
         }
 #pragma unroll
         for (int e = 0; e < L; ++e) {
-            const R mn = row_reduce(st[e].mn, [](R u, R v) { return v < u ? v : u; });
+            const R mn = row_reduce(st[e].mn, lanes, [](R u, R v) { return v < u ? v : u; });
             const R s = st[e].mn < R(kSoftBig) ? st[e].s * r_exp<R>(-(st[e].mn - mn) / tau) : R(0);
-            const Lse<R> m{mn, row_reduce(s, [](R u, R v) { return u + v; })};
+            const Lse<R> m{mn, row_reduce(s, lanes, [](R u, R v) { return u + v; })};
             if (lane == e) out[e] = lse_value(m, tau);
         }
     }
@@ -823,7 +828,7 @@ __device__ __forceinline__ void backward_zedges(const SoftArgs& a, const int4* o
             double before[L];  // last-leg weights of the bends nearer the child
 #pragma unroll
             for (int l = 0; l < L; ++l) before[l] = 0.0;
-            for_each_bend<L, P>(a, E, d1, lane, [&](const ZBend<L>& z, int b, bool live, int b0) {
+            for_each_bend<L, P>(a, E, d1, lane, kZGroup, [&](const ZBend<L>& z, int b, bool live, int b0) {
                 const int ax = d1 ? E.x : b, ay = d1 ? b : E.y, bx = d1 ? E.px : b, by = d1 ? b : E.py;
                 const int cell = up ? b : b - 1;  // this lane's cell of the first and last legs' tracks
                 R f1[L], mv[L];
@@ -906,7 +911,7 @@ __device__ __forceinline__ void backward_zedges(const SoftArgs& a, const int4* o
         }
 #pragma unroll
         for (int l = 0; l < L; ++l) {
-            const double s = row_reduce(gb[l], [](double u, double v) { return u + v; });
+            const double s = row_reduce(gb[l], kZGroup, [](double u, double v) { return u + v; });
             if (lane == l) t.gbest[base + l] = R(s);
         }
     }
@@ -984,7 +989,7 @@ template <class R, int L, int K>
 __global__ __launch_bounds__(256) void soft_forward_chunk_kernel(SoftArgs a, SoftLevels lv) {
     const int* start = lv.dstart + size_t(blockIdx.x) * (lv.bins + 1);
     const int4* order = lv.order + (a.node_off[a.begin + blockIdx.x * lv.chunk] - a.node0);
-    const int wave = threadIdx.x / kWave, group = threadIdx.x / kZGroup;
+    const int wave = threadIdx.x / kWave;
     const int bins = min(lv.bins, kLevelBins - 1), tall = lv.bins == kLevelBins ? start[bins + 1] - start[bins] : 0;
     for (int h = 0; h < bins + tall; ++h) {
         const int b = h < bins ? start[h] : start[bins] + h - bins, e = h < bins ? start[h + 1] : b + 1;
@@ -992,7 +997,7 @@ __global__ __launch_bounds__(256) void soft_forward_chunk_kernel(SoftArgs a, Sof
         forward_nodes<R, L, K>(a, order + b, e - b, wave, 256 / kWave);
         __syncthreads();
         if (K) {
-            forward_zedges<R, L>(a, order + b, e - b, group, 256 / kZGroup);
+            forward_zedges<R, L>(a, order + b, e - b);
             __syncthreads();
         }
     }

@@ -181,9 +181,9 @@ def _soft_trees(rng, L, X, Y):
 @pytest.mark.parametrize("L,X,Y", [(1, 5, 9), (2, 3, 40), (5, 37, 20), (9, 20, 70), (10, 18, 17)])
 def test_soft_trees_of_every_form_match_oracle(ga, ora, L, X, Y, kind):
     """Every lane count (L lanes per node: 64, 32, 12, 7 and 6 nodes per
-    wavefront), edges of more bends than the 16 lanes of an edge, a slot range
-    that does not start at 0, given costs of either sign: FP64 equal to the
-    oracle as on the generated instance above."""
+    wavefront), edges of more bends than they have lanes (16, or 64 on a level
+    of few edges), a slot range that does not start at 0, given costs of either
+    sign: FP64 equal to the oracle as on the generated instance above."""
     rng = np.random.default_rng(1000 * L + X)
     off, nodes, parents = _soft_trees(rng, L, X, Y)
     t = dict(L=L, X=X, Y=Y, DIR=L & 1, unit_length_wire_cost=0.01, unit_via_cost=0.5,
