@@ -550,3 +550,33 @@ def test_stage_runs_between_other_launches_of_its_slots(ga, ora):
             step()
             check(mode)
     ctx.close()
+
+
+def test_ripup_of_long_nets_counts_to_the_limit(ga, ora):
+    """Nets of up to 200 unit segments with 10 or 11 overflowed edges, first,
+    last and spread over the words: on either side of the reference's limit."""
+    X, Y = 201, 60
+    cap = np.full((1, X, Y), 100, np.float32)
+    nets = []
+    for y in range(Y):
+        length = [12, 31, 32, 33, 64, 65, 128, 200][y % 8]
+        over = 10 + (y // 8) % 2
+        where = [np.arange(over), length - 1 - np.arange(over), np.linspace(0, length - 1, over).astype(int)][y % 3]
+        cap[0, where, y] = 0
+        nets.append([(x, y) for x in range(length + 1)])
+    t = dict(L=1, X=X, Y=Y, DIR=0, unit_length_wire_cost=0.01, unit_via_cost=4.0,
+             unit_length_short_costs=np.ones(1), x_edge_len=np.full(X - 1, 300, np.int32),
+             y_edge_len=np.full(Y - 1, 300, np.int32), capacity=cap.ravel())
+    off = np.concatenate([[0], np.cumsum([len(n) for n in nets])]).astype(np.int32)
+    nodes = np.array([x * Y + y for n in nets for x, y in n], np.int32)
+    parents = np.concatenate([np.arange(-1, len(n) - 1) for n in nets]).astype(np.int32)
+    print("rip-up of long nets", flush=True)
+    ctx = ga.Context(t)
+    ctx.set_routes(off)
+    ctx.lshape_upload(np.arange(len(nets)), off, nodes, parents)
+    ctx.lshape_run(np.array([0, len(nets)], np.int32), 1, 0)
+    flags = ctx.ripup(len(nets), 0)
+    want = ora.Grid(t).ripup(ctx.demand(), ctx.routes(), off, 0)
+    assert 0 < want.sum() < len(nets)
+    assert np.array_equal(flags, want)
+    ctx.close()
