@@ -445,11 +445,12 @@ void download(void* dst, const void* src, size_t bytes, hipStream_t s) {
 }
 
 // Grids of fewer cells change their order on the host: the extra launch and
-// its wait for the copy cost more there (a demand upload and download of 16k
-// cells 41 us on the host, 62 on the device; 32k 48 and 66, but the two cost
-// arrays and gradients of the soft DP 175 and 186; 65k 137 and 75; 262k 577 and
-// 150).
-constexpr size_t kHostLayoutCells = 32768;
+// its wait for the copy cost more there.  Host and device, in us: a cost
+// download 89 and 86 at 33k cells; the soft DP's gradients 54 and 57 at 33k, 61
+// and 60 at 40k.  One binary32 array on its way up 29 and 36 at 33k, 37 and 38
+// at 66k, 41 and 38 at 73k; down 20 and 30 at 33k, 30 and 35 at 66k, 34 and 37
+// at 80k, 61 and 47 at 131k.
+constexpr size_t kHostLayoutCells = 32768, kHostUploadCells = 65536, kHostDownloadCells = 90112;
 
 // IDX order <-> track-major order on the host, one pass.
 template <class T>
@@ -485,9 +486,10 @@ void for_layer_slabs(gr_ctx* c, int arrays, F&& f) {
         f(a, tmp, size_t(l) * c->g.XY, size_t(a.layers) * c->g.XY);
     }
 }
+// host_cells: the size below which the order changes on the host.
 template <class T>
-void upload_grids(gr_ctx* c, T* dst0, const T* src0, T* dst1 = nullptr, const T* src1 = nullptr) {
-    if (c->cells < kHostLayoutCells) {
+void upload_grids(gr_ctx* c, size_t host_cells, T* dst0, const T* src0, T* dst1 = nullptr, const T* src1 = nullptr) {
+    if (c->cells < host_cells) {
         std::vector<T> h(c->cells);
         for (auto [dst, src] : {std::pair<T*, const T*>{dst0, src0}, {dst1, src1}}) {
             if (!src) continue;
@@ -509,8 +511,8 @@ void upload_grids(gr_ctx* c, T* dst0, const T* src0, T* dst1 = nullptr, const T*
     });
 }
 template <class T>
-void download_grids(gr_ctx* c, const T* src0, T* dst0, const T* src1 = nullptr, T* dst1 = nullptr) {
-    if (c->cells < kHostLayoutCells) {
+void download_grids(gr_ctx* c, size_t host_cells, const T* src0, T* dst0, const T* src1 = nullptr, T* dst1 = nullptr) {
+    if (c->cells < host_cells) {
         std::vector<T> h(c->cells);
         for (auto [src, dst] : {std::pair<const T*, T*>{src0, dst0}, {src1, dst1}}) {
             if (!dst) continue;
@@ -1223,7 +1225,7 @@ void soft_forward(gr_ctx* c, int begin, int count, double slope, double zero_slo
     sc.via_weight = via_weight;
     const bool given = wcost != nullptr;
     if (given) {
-        upload_grids<double>(c, sc.wcost, wcost, sc.vcost, vcost);
+        upload_grids<double>(c, kHostLayoutCells, sc.wcost, wcost, sc.vcost, vcost);
     }
     a.g = c->g;
     a.presum = sc.presum;
@@ -1340,7 +1342,7 @@ int gr_ctx_create(const gr_grid_desc* grid, gr_ctx** out) {
         c->refreshed = c->mem.alloc<unsigned long long>(kStatStripes * kCounterStride);
         hip_check(hipMemsetAsync(c->refreshed, 0, sizeof(unsigned long long) * kStatStripes * kCounterStride, c->stream),
                   "clear counter");
-        upload_grids<float>(c.get(), c->capacity, grid->capacity);
+        upload_grids<float>(c.get(), kHostUploadCells, c->capacity, grid->capacity);
         hip_check(hipMemsetAsync(c->demand, 0, sizeof(float) * c->cells, c->stream), "clear demand");
         hip_check(hipMemsetAsync(c->timestamp, 0, sizeof(int) * c->cells, c->stream), "clear timestamps");
         hip_check(hipMemsetAsync(c->stats, 0, sizeof(Stats) * kStatStripes, c->stream), "clear statistics");
@@ -1439,8 +1441,8 @@ int gr_cost_download(gr_ctx* c, float* wcost, float* vcost, double* presum) {
                                tmp, td, 1, c->cp, (unsigned long long*)nullptr);
             hip_check(hipGetLastError(), "refresh for wcost");
         }
-        if (wcost || vcost) download_grids<float>(c, tmp, wcost, c->vcost, vcost);
-        if (presum) download_grids<double>(c, c->presum, presum);
+        if (wcost || vcost) download_grids<float>(c, kHostLayoutCells, tmp, wcost, c->vcost, vcost);
+        if (presum) download_grids<double>(c, kHostLayoutCells, c->presum, presum);
     });
 }
 
@@ -1448,7 +1450,7 @@ int gr_demand_upload(gr_ctx* c, const float* demand) {
     return guarded([&] {
         if (!c || !demand) throw GrError(GR_E_ARG, "null argument");
         mark_tracks(c);
-        upload_grids<float>(c, c->demand, demand);
+        upload_grids<float>(c, kHostUploadCells, c->demand, demand);
         hip_check(hipStreamSynchronize(c->stream), "demand upload");
     });
 }
@@ -1456,14 +1458,14 @@ int gr_demand_upload(gr_ctx* c, const float* demand) {
 int gr_demand_download(gr_ctx* c, float* demand) {
     return guarded([&] {
         if (!c || !demand) throw GrError(GR_E_ARG, "null argument");
-        download_grids<float>(c, c->demand, demand);
+        download_grids<float>(c, kHostDownloadCells, c->demand, demand);
     });
 }
 
 int gr_timestamp_download(gr_ctx* c, int* ts) {
     return guarded([&] {
         if (!c || !ts) throw GrError(GR_E_ARG, "null argument");
-        download_grids<int>(c, c->timestamp, ts);
+        download_grids<int>(c, kHostLayoutCells, c->timestamp, ts);
     });
 }
 
@@ -2858,7 +2860,7 @@ int gr_soft_edge_grads(gr_ctx* c, double* grad_wcost, double* grad_vcost) {
     return guarded([&] {
         if (!c) throw GrError(GR_E_ARG, "null context");
         if (!c->soft_ready) throw GrError(GR_E_STATE, "no soft pass");
-        download_grids<double>(c, c->soft.gw, grad_wcost, c->soft.gv, grad_vcost);
+        download_grids<double>(c, kHostLayoutCells, c->soft.gw, grad_wcost, c->soft.gv, grad_vcost);
     });
 }
 
