@@ -1105,29 +1105,52 @@ struct ZnetTree {
     int parent[kZnetMaxNodes];  // parent | slot << 16, -1: the root
     int height[kZnetMaxNodes];
 
-    // False where the general kernels route the net: a tree too large for LDS,
-    // two nodes at one place, a node without exactly one parent, a gap in the
-    // child slots (the shared map gives those cases their meaning).
-    bool read(int L, const int* rec) {
+    // kPerNet: zshape_net_kernel.  kGeneral: the general kernels (a tree too
+    // large for LDS, a node with two parents).  kLeftover: the general kernels,
+    // and the net's words rest on what earlier nets of the plan left on the
+    // shared map (two nodes at one place; a node without a parent or past a gap
+    // in the child slots, which the traceback never gives a layer).
+    enum Form { kPerNet, kGeneral, kLeftover };
+    Form read(int L, const int* rec) {
         m = rec[1];
         rec += 2;
-        if (m >= kZnetMaxNodes || znet_lds_bytes(L, m) > kZnetLds) return false;
-        int pos[kZnetMaxNodes];
-        for (int i = 0; i < m; ++i) parent[i] = -1, height[i] = 0, pos[i] = rec[6 * i];
-        std::sort(pos, pos + m);
-        if (std::adjacent_find(pos, pos + m) != pos + m) return false;
+        const bool large = m >= kZnetMaxNodes || znet_lds_bytes(L, m) > kZnetLds;
+        if (large) {
+            std::vector<int> at(m), up(m, 0);
+            return odd(rec, at.data(), up.data()) ? kLeftover : kGeneral;
+        }
+        int at[kZnetMaxNodes], parents[kZnetMaxNodes];
+        std::fill(parents, parents + m, 0);
+        if (odd(rec, at, parents)) return kLeftover;
+        for (int i = 0; i < m; ++i) {
+            if (parents[i] > 1) return kGeneral;
+            parent[i] = -1, height[i] = 0;
+        }
         for (int i = m - 1; i >= 0; --i)
             for (int j = 0; j < 3; ++j) {
                 const int ch = rec[6 * i + 3 + j];
                 if (ch == -1) continue;
-                if ((j && rec[6 * i + 2 + j] == -1) || parent[ch / 6] >= 0) return false;
                 parent[ch / 6] = i | j << 16;
                 height[i] = std::max(height[i], height[ch / 6] + 1);
             }
-        for (int i = 1; i < m; ++i)
-            if (parent[i] < 0) return false;
         height_of_root = height[0];
-        return true;
+        return kPerNet;
+    }
+    // Counts every node's parents (into zeros); at: scratch.
+    bool odd(const int* rec, int* at, int* parents) const {
+        for (int i = 0; i < m; ++i) {
+            at[i] = rec[6 * i];
+            for (int j = 0; j < 3; ++j) {
+                const int ch = rec[6 * i + 3 + j];
+                if (ch == -1) continue;
+                if (j && rec[6 * i + 2 + j] == -1) return true;
+                ++parents[ch / 6];
+            }
+        }
+        for (int i = 1; i < m; ++i)
+            if (!parents[i]) return true;
+        std::sort(at, at + m);
+        return std::adjacent_find(at, at + m) != at + m;
     }
     static size_t words(int m, int H) { return 4 * size_t(m) + (m + 1) + (H + 2) + m; }
     // Into out[0 .. words(m, height_of_root)); n: side of the map the record's
@@ -2062,6 +2085,7 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
         };
         std::vector<int2> form(nets);
         std::vector<long long> raw_words(nbatch, 0);
+        std::atomic<bool> leftover{false};
         each_batch([&](int b) {
             const int begin = batch_off[b], count = batch_off[b + 1] - begin;
             const long long r0 = rec_off[b], r1 = rec_off[b + 1];
@@ -2089,12 +2113,15 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
                         if (r[j] != -1 && (r[j] < 6 * (i + 1) || r[j] >= 6 * nodes || r[j] % 6))
                             throw GrError(GR_E_ARG, "child record must follow its parent in preorder");
                 }
-                form[begin + k] = tree.read(L, rec) ? make_int2(nodes, tree.height_of_root) : make_int2(0, 0);
+                const ZnetTree::Form f = tree.read(L, rec);
+                if (f == ZnetTree::kLeftover) leftover = true;
+                form[begin + k] = f == ZnetTree::kPerNet ? make_int2(nodes, tree.height_of_root) : make_int2(0, 0);
             }
         });
         // The nets' places: per batch its nets with the DP in LDS (descriptor,
         // subnet, record) and the positions of the others, whose batches' plan
-        // records cross too.
+        // records cross too.  All nets are general beside one that reads what
+        // they leave on the map.
         std::vector<gr_ctx::ZBatch> split(nbatch);
         std::vector<long long> dev_rec_off(nbatch + 1, 0);
         std::vector<int4> desc;
@@ -2108,7 +2135,7 @@ int gr_zshape_upload(gr_ctx* c, int nbatch, const int* batch_off, const int* net
             const int begin = batch_off[b];
             for (int j = begin; j < batch_off[b + 1]; ++j) {
                 const int m = form[j].x, H = form[j].y;
-                if (m && own_words < size_t(INT32_MAX / 2)) {
+                if (m && !leftover && own_words < size_t(INT32_MAX / 2)) {
                     desc.push_back(make_int4(int(own_words), m, H, raw_cap[j]));
                     ids.push_back(net_ids[j]);
                     own_words += ZnetTree::words(m, H);

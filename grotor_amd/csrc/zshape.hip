@@ -6,7 +6,8 @@
 //
 // Two forms.  zshape_net_kernel (end of this file) routes a net with its DP
 // in LDS and takes every net that fits; the general kernels take the rest
-// (large trees, and records whose meaning rests on the shared map).  In the
+// (large trees, nodes with two parents, and whole plans with a record whose
+// words rest on what earlier nets left on the shared map).  In the
 // general form one 64-lane wavefront routes one tree (the reference uses a
 // 32-lane warp).  Nets of a batch have disjoint bounding boxes, so they share one
 // map of LAYER = L + 1 planes of n x n cells (n = max(X, Y)) without

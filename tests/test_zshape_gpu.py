@@ -137,15 +137,15 @@ def _with_second_parent(rec):
     return rec
 
 
-@pytest.mark.parametrize("L,DIR,batches,odd", [(3, 1, 6, False), (6, 0, 260, False), (4, 1, 2, True)])
+@pytest.mark.parametrize("L,DIR,batches,odd", [(3, 1, 6, False), (6, 0, 260, False), (4, 1, 6, True)])
 def test_zshape_batches_of_both_kernels(ga, ora, L, DIR, batches, odd):
     """Batches of nets in boxes of their own, most with trees for the per-net
     kernel and, in some batches and at any position, nets for the general one
     (a tree beyond the LDS bound, a node with two parents), beside batches of
     one kind only; nodes with a range of layers.  6 batches are planned on one
     thread, 260 on several.  `odd`: gaps in the child slots and two nodes at one
-    place, which take nodes' layers from what the map holds: with general nets
-    only, in a new context, the words and the error are the oracle's."""
+    place, which take nodes' layers from what earlier nets left on the map: the
+    words and the error are the oracle's in a new context."""
     rng = np.random.default_rng(L)
     X, Y, w = 53, 44, 10
     n = max(X, Y)
@@ -169,7 +169,7 @@ def test_zshape_batches_of_both_kernels(ga, ora, L, DIR, batches, odd):
             pick = (r[:, 1] != -1) & (rng.random(len(r)) < 0.5)
             r[pick, 2] = rng.integers(r[pick, 1], L + 1)
             # every sixth batch is all of one kind, the others mix them
-            general = odd or b % 6 != 0 and (b % 6 == 1 or rng.random() < 0.3)
+            general = b % 6 != 0 and (b % 6 == 1 or rng.random() < 0.3)
             if general and side != 20:
                 rec = change(rec)
             kinds.add((b % 6, general or side == 20))
@@ -186,7 +186,7 @@ def test_zshape_batches_of_both_kernels(ga, ora, L, DIR, batches, odd):
         raw_cap += cap
         batch_off.append(batch_off[-1] + len(recs))
         rec_off.append(len(records))
-    assert odd or ((0, True) not in kinds and (1, False) not in kinds)
+    assert (0, True) not in kinds and (1, False) not in kinds
     nets = batch_off[-1]
     plan = dict(batch_off=np.array(batch_off, np.int32), net_ids=rng.permutation(nets).astype(np.int32),
                 rec_off=np.array(rec_off, np.int64), records=np.array(records, np.int32),
