@@ -580,3 +580,55 @@ def test_ripup_of_long_nets_counts_to_the_limit(ga, ora):
     assert 0 < want.sum() < len(nets)
     assert np.array_equal(flags, want)
     ctx.close()
+
+
+@pytest.mark.parametrize("L,X,Y", [(1, 300, 40), (2, 90, 300), (5, 120, 120), (9, 64, 500)])
+def test_wires_committed_in_the_dp_equal_the_commit_launch(ga, L, X, Y):
+    """Demand, timestamps and statistics of small batches (wires committed by
+    the DP launches) equal those of the commit's own launch, which profiled
+    runs keep: wires of 0 to several hundred cells, zero-length edges, one to
+    eight nets per wavefront, and on one layer nets without a finite solution,
+    whose words run across the tracks."""
+    rng = np.random.default_rng(L)
+    n = 400
+    sizes = rng.choice([1, 2, 3, 5, 9, 20, 40], n)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    nodes, parents = [], []
+    for k in sizes:
+        x, y = rng.integers(0, X, k), rng.integers(0, Y, k)
+        x[rng.random(k) < 0.3] = x[0]
+        if k > 2:
+            x[2], y[2] = x[1], y[1]
+        par = [-1] + [int(rng.integers(0, i)) for i in range(1, k)]
+        if k > 2:
+            par[2] = 1
+        layer = np.where(rng.random(k) < 0.5, L, rng.integers(0, L, k))
+        nodes += ((layer * X + x) * Y + y).tolist()
+        parents += par
+    t = dict(L=L, X=X, Y=Y, DIR=L // 2 & 1, unit_length_wire_cost=0.01, unit_via_cost=4.0,
+             unit_length_short_costs=np.full(L, 0.1), x_edge_len=rng.integers(1, 400, X - 1).astype(np.int32),
+             y_edge_len=rng.integers(1, 400, Y - 1).astype(np.int32), capacity=np.full(L * X * Y, 50, np.float32))
+    bo = np.array([0, 1, 3, 60, 200, n], np.int32)
+    ctx = ga.Context(t)
+    ctx.set_routes(off)
+    ctx.lshape_upload(np.arange(n), off, np.array(nodes, np.int32), np.array(parents, np.int32))
+    for mode, per_wave in ((0, 1), (1, 1), (1, 4), (1, 8), (2, 1), (2, 8)):
+        print(f"fused wires L={L} mode={mode} per wave={per_wave}", flush=True)
+        ctx.set_nets_per_wave((per_wave, 1))
+        states = []
+        for profiled in (False, True):
+            ctx.reset()
+            if profiled:
+                ctx.profile_begin()
+            try:
+                ctx.lshape_run(bo, 1, mode)
+                assert L > 1
+            except ga.GrError as e:
+                assert L == 1 and "no finite layer" in str(e)
+            if profiled:
+                ctx.profile_end()
+            states.append((ctx.routes(), _bits(ctx.demand()), ctx.timestamps(), ctx.stats()))
+        for a, b in zip(*states):
+            assert np.array_equal(a, b)
+        assert states[0][1].any()
+    ctx.close()
