@@ -126,8 +126,9 @@ __global__ __launch_bounds__(256) void layout_kernel(DeviceGrid g, LayoutArrays<
     // rows of the source: x (IDX) or the track y of a horizontal layer
     const bool copy = layer_dir(g, arrays.first + l), by_x = to_track || copy;
     const int rows = by_x ? g.X : g.Y, cols = by_x ? g.Y : g.X;
-    // block y over the tiles of x, block x over those of y, for either order
-    const int r0 = (by_x ? blockIdx.y : blockIdx.x) * kLayoutTile, c0 = (by_x ? blockIdx.x : blockIdx.y) * kLayoutTile;
+    // tiles along the source's rows first
+    const int ctiles = (cols + kLayoutTile - 1) / kLayoutTile;
+    const int r0 = int(blockIdx.x) / ctiles * kLayoutTile, c0 = int(blockIdx.x) % ctiles * kLayoutTile;
     for (int r = ty; r < kLayoutTile; r += 256 / kLayoutTile)
         if (r0 + r < rows && c0 + tx < cols) {
             const T v = src[base + size_t(r0 + r) * cols + c0 + tx];
@@ -143,8 +144,8 @@ __global__ __launch_bounds__(256) void layout_kernel(DeviceGrid g, LayoutArrays<
 template <class T>
 void launch_layout(const DeviceGrid& g, const LayoutArrays<T>& a, bool to_track, hipStream_t st) {
     if (!a.count) return;
-    const dim3 grid(unsigned((g.Y + kLayoutTile - 1) / kLayoutTile), unsigned((g.X + kLayoutTile - 1) / kLayoutTile),
-                    unsigned(a.layers * a.count));
+    const int xtiles = (g.X + kLayoutTile - 1) / kLayoutTile, ytiles = (g.Y + kLayoutTile - 1) / kLayoutTile;
+    const dim3 grid(unsigned(xtiles * ytiles), 1, unsigned(a.layers * a.count));
     hipLaunchKernelGGL(layout_kernel<T>, grid, dim3(256), 0, st, g, a, to_track ? 1 : 0);
 }
 template void launch_layout<float>(const DeviceGrid&, const LayoutArrays<float>&, bool, hipStream_t);
