@@ -528,14 +528,16 @@ template <class R, int L>
 __device__ __forceinline__ void forward_zedges(const SoftArgs& a, const int4* order, int count) {
     const DeviceGrid& g = a.g;
     const R tau = R(a.tau);
-    const int lanes = count <= 256 / kWave ? kWave : kZGroup;
-    const int lane = threadIdx.x % lanes;
+    const int group = count <= 256 / kWave ? kWave : kZGroup;
     const SoftTables<R> t = soft_tables<R>(a);
-    for (int k = threadIdx.x / lanes; k < count; k += 256 / lanes) {
+    for (int k = threadIdx.x / group; k < count; k += 256 / group) {
         const int4 it = order[k];
         if (it.w < 0) continue;
         const SoftNode c = soft_node(g, a.nodes[it.x]), p = soft_node(g, a.nodes[it.y + it.w]);
         const Edge E{c.x, c.y, p.x, p.y};
+        // short edges keep rows of 16, all four of the wavefront the same
+        const int lanes = max(abs(E.x - E.px), abs(E.y - E.py)) <= kZGroup ? kZGroup : group;
+        const int lane = threadIdx.x % lanes;
         const R* bn = t.best + size_t(it.x - a.node0) * L;
         R* out = t.diag + size_t(it.x - a.node0) * L;
         if (E.x == E.px || E.y == E.py) {
